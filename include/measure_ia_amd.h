@@ -133,7 +133,8 @@ typedef struct mia_tuning {
     int32_t slabs_per_side;     /* line-of-sight slabs per box side                   */
     int32_t slabs_per_block;    /* shape-block height in slabs                        */
     int32_t block_shapes;       /* shapes per block, <= 64                            */
-    int32_t item_positions;     /* max positions per work item                        */
+    int32_t item_positions;     /* positions per work item, about (whole position
+                                   columns, 1 to 64 of them)                            */
     int32_t waves;              /* persistent waves of the pair kernel (at most 2^20)  */
     int32_t hist_copies;        /* ignored (one LDS histogram copy per wave)           */
     int32_t cell_shapes;        /* > 0: size cells to hold this many shapes on average

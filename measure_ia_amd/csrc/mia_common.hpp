@@ -56,6 +56,7 @@ __device__ __forceinline__ int xcd_run_block() {
 constexpr int kScheduleUnits = 32;
 constexpr double kTailMinCost = 4.0e5;   // item-cost units per wave (about 5 ms of pair work)
 constexpr double kTailFineCost = 8.0e5;  // (about 10 ms)
+constexpr int64_t kTailItems = 16;       // items per unit below which groups of several waves take no chunks
 constexpr int kMaxWaves = 1 << 20;       // persistent waves per launch (tail counter stays in int)
 
 struct WaveSchedule {
@@ -73,6 +74,10 @@ struct WaveSchedule {
         int k = 0;
         if (lane == 0) k = atomicAdd(counter, 1);
         k = __builtin_amdgcn_readfirstlane(k);
+        return chunk(k, i0, i1);
+    }
+    // tail chunk k; false past the last
+    __device__ __forceinline__ bool chunk(int k, int64_t &i0, int64_t &i1) const {
         if (k >= tail) return false;
         const int64_t u = (int64_t)W * S + (int64_t)k * G;
         i0 = bounds[u];
@@ -98,7 +103,7 @@ void schedule_bounds(const int64_t *cost_prefix, int64_t n, int waves, int64_t *
 // takes only its static range (no tail claims), so the item -> wave map is
 // fixed by the costs
 void schedule_bounds(const int64_t *cost_prefix, const int64_t *n_dev, int waves, int64_t *bounds,
-                     hipStream_t st, bool all_static = false);
+                     hipStream_t st, bool all_static = false, int waves_per_unit = 1);
 
 constexpr int kMaxBins2 = 256;      // max n_2 (pi or mu bins)
 constexpr int kMaxBinsR = 256;      // max n_r
@@ -169,8 +174,9 @@ struct Grid {
     double cw = 0, hz = 0; // nominal column width and slab height
     double margin = 0;     // geometric slack for rounding at cell edges
     int G = 0;             // slabs per shape block chosen with the grid (0: decide later)
-    int pmax = 0;          // positions per work item chosen with the grid (0: the default)
-    int keys() const { return nc * nc * (nz + 1); }
+    int m = 1;             // position columns per column and axis: positions are sorted by columns of width cw / m
+    int64_t keys() const { return (int64_t)nc * nc * (nz + 1); }
+    int64_t pkeys() const { return keys() * m * m; }  // cells of the positions
 };
 
 // Sorted sample in HBM (structure of arrays, sorted by cell key).
@@ -248,9 +254,10 @@ struct SortedSample {
     int weighted = 0;                 // a weight array was given
     const double *prec = nullptr;     // 4 doubles per position {a, b, l, w}, sorted order
     const double *srec = nullptr;     // 8 doubles per shape {a, b, l, ax, ay, e*w, w, 2*e*w}
-    const int32_t *pstart = nullptr, *sstart = nullptr;  // keys + 1 start offsets into the arrays above
-    const int32_t *pfine = nullptr;   // (keys << sbits) + 1 starts of the positions' fine keys
-    int sbits = 0;                    // fine key = (cell << sbits) + line-of-sight part of the slab
+    const int32_t *sstart = nullptr;  // shapes: keys + 1 start offsets
+    const int32_t *pfine = nullptr;   // positions: (pkeys << pbits) + 1 starts of the fine keys
+    int pbits = 0;                    // fine key = (cell << pbits) + line-of-sight part of the slab
+    const int32_t *flags = nullptr;   // bit 0: a coordinate out of the box; bit 1: positions in a column's tail
     const unsigned long long *rcnt = nullptr;  // [2K] per region: positions, shapes
     const double *rsum = nullptr;     // [2K] per region: sum w_s, sum w_s (1 - e^2/2)
 };
@@ -291,15 +298,9 @@ struct CountCall;
 // Host plan of a staged count over n sorted samples: worst-case sizes,
 // launch shapes and the pair-kernel configuration.
 struct CountPlan;
-// Work-item packing of the planner: one plan thread walks kGroupColumns
-// stencil columns of a shape block and packs their position ranges into items
-// of at most kItemRanges ranges (and the item's position limit).
-constexpr int kGroupColumns = 8;
-constexpr int kItemRanges = 8;
-// item_cap, range_cap: at least this many work-item slots and range records
-// (exactly this many with cap_exact)
+// item_cap: at least this many work-item slots (exactly this many with cap_exact)
 struct CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_bins &bins,
-                             const mia_tuning *tuning, int64_t item_cap, int64_t range_cap, bool cap_exact);
+                             const mia_tuning *tuning, int64_t item_cap, bool cap_exact);
 void free_plan(CountPlan *p);
 // workspace bytes of the count stages (after plan_count)
 size_t count_bytes(const CountPlan &p);
@@ -315,18 +316,16 @@ void *count_param_dev(const CountPlan &p);
 // pairs and at the end.
 void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev);
 // Device words read back after a count: [0] rechecks, [1] candidates of the
-// planned items, [2] item or range overflow, [3] items, [4] pair-kernel start
+// planned items, [2] item overflow, [3] items, [4] pair-kernel start
 // (~wall clock), [5] end, [6] wave-iterations of the pair kernel (one 64-lane
-// position batch against one shape), [7] range records of the multi-range
-// items, [8] position ranges of the planner.
+// position batch against one shape).
 const unsigned long long *count_readback(const CountPlan &p);
-constexpr int kCountReadback = 9;
+constexpr int kCountReadback = 7;
 int count_waves(const CountPlan &p);
 int count_bsz(const CountPlan &p);
 bool count_det(const CountPlan &p);
 int count_G(const CountPlan &p, int sample);
 int64_t count_item_cap(const CountPlan &p);
-int64_t count_range_cap(const CountPlan &p);
 // a key identifying the launch sequence (everything but caller pointers)
 std::string count_key(const CountPlan &p);
 
@@ -352,7 +351,6 @@ struct Ctx {
     hipGraphExec_t gexec = nullptr;
     std::string gkey;               // launch-sequence key of gexec
     int64_t item_cap = 0;           // grown after an item overflow
-    int64_t range_cap = 0;          // grown after a range-record overflow
     double wall_khz = 100000.0;     // device wall-clock rate
     void *scratch = nullptr;        // the device's static workspace (allocation-free entry point)
 };

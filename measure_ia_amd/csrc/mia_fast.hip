@@ -4,28 +4,29 @@
 // (src/measureia/measure_w_box_jk.py:386-461, measure_m_box_jk.py:403-487)
 // with three steps on the device:
 //   1. plan   : shapes of one column and a few line-of-sight slabs form a
-//               block (<= 64 shapes, one jackknife region R_s); every block
-//               is paired with the position cell ranges within reach, split
-//               at jackknife sub-box faces so that every range has one
-//               position region R_p and one periodic shift per axis.  The
-//               ranges of up to 8 neighbouring stencil columns with the same
-//               region and shift are packed into one work item.  Items are
-//               counting-sorted by (sample, R_s, R_p).
-//   2. pairs  : a persistent grid of wavefronts takes contiguous runs of the
-//               sorted list, balanced by estimated cost, then claims tail
-//               chunks from a counter.  Each wave reads its
-//               shape block through the scalar cache (one 64-byte record per
-//               shape, wave-uniform) and streams positions through registers,
-//               64 at a time.  Separations are the reference's own FP64
-//               differences, so r_p^2 (or r^2) and pi are compared exactly
-//               with the host-bisected thresholds (an FP32 log2 only guesses
-//               the bin); e+ and ex are FP64 (CDNA4 runs FP64 FMA at the rate
-//               of non-packed FP32) and go into the wave's private LDS
-//               histogram with LDS atomics.  mu = pi/r is screened in FP32 and recomputed in
+//               block (<= 64 shapes, one jackknife region R_s).  Positions are
+//               sorted by thinner columns.  A block's reach along each axis
+//               falls into segments of one jackknife sub-box and one periodic
+//               shift; a rectangle of two such segments and a line-of-sight
+//               run have one position region R_p, and up to 64 columns of it
+//               make a work item.  Items are counting-sorted by
+//               (sample, R_s, R_p).
+//   2. pairs  : a persistent grid takes contiguous runs of the sorted list,
+//               balanced by estimated cost, then claims tail chunks from a
+//               counter.  Each lane looks up the positions of one column of an
+//               item; the wave then reads its shape block through the scalar
+//               cache (one 64-byte record per shape, wave-uniform) and streams
+//               the positions through registers, 64 at a time.  Separations
+//               are the reference's own FP64 differences, so r_p^2 (or r^2)
+//               and pi are compared exactly with the host-bisected thresholds
+//               (an FP32 log2 only guesses the bin); e+ and ex are FP64 (CDNA4
+//               runs FP64 FMA at the rate of non-packed FP32) and go into an
+//               LDS histogram (a wave's own, or shared by a workgroup) with
+//               LDS atomics.  mu = pi/r is screened in FP32 and recomputed in
 //               FP64 when it lies within a guard band of a bin edge; the
 //               arccos NaN rule is likewise checked in FP64 for nearly
 //               parallel pairs.
-//   3. flush  : a wave adds its histogram to the workspace's FP64
+//   3. flush  : a histogram is added to the workspace's FP64
 //               accumulators of the total and of tally[R_s] / tally[R_p]
 //               only when the (R_s, R_p) key changes, i.e. a handful of times
 //               per wave; k_finalize then writes the caller's outputs.  In
@@ -48,6 +49,9 @@ namespace {
 constexpr int kMaxWavesPerBlock = 4;
 constexpr int kThreads = kWave * kMaxWavesPerBlock;
 constexpr size_t kLdsBytes = 160 * 1024;         // LDS per CU (gfx950)
+constexpr size_t kPairStaticLds = 64;            // the pair kernel's own LDS words, at most
+constexpr int kSharedBelow = 16;                 // private waves per CU below which histograms are shared
+constexpr int kPairWavesPerSimd = 6;             // waves per SIMD the pair kernel's registers allow
 constexpr int64_t kMaxKeysPerSample = 1 << 24;   // K^2 planner keys per sample (K regions)
 constexpr double kSinExact = 1e-5;  // FP64 arccos-domain check when |sin phi| < 1e-5 |cos phi|
 
@@ -57,32 +61,29 @@ struct Block {
     int32_t sample, rs;
 };
 
-// A work item pairs one shape block with up to kItemRanges position ranges of
-// one key and one shift class (the ranges of neighbouring stencil columns are
-// packed together, so short columns still fill the 64 lanes).  Item
-// coordinates k = 0 .. np-1 run over the ranges in order.
+// A work item pairs one shape block with the positions of up to kItemColumns
+// consecutive position columns of one rectangle (columns within reach of the
+// block, of one jackknife sub-box and one periodic shift class per axis), over
+// one line-of-sight run of slabs.  The pair kernel looks the columns' positions
+// up itself, one column per lane, so the plan holds no per-column record.
 struct Item {
     int32_t blk;
-    int32_t p0;         // nr == 1: first position; nr > 1: first of nr Range records
-    int32_t np;
-    int16_t rp;
-    uint8_t shifts;     // 2 bits per axis (a, b, l): 0 -> 0, 1 -> +L, 2 -> -L ; bit 6: per-pair wrap
-    uint8_t nr;         // position ranges
+    int32_t w;          // R_p | shift byte << 16: 2 bits per axis (a, b, l): 0 -> 0, 1 -> +L, 2 -> -L ;
+                        // bit 6: per-pair wrap | line-of-sight class (3: mixed) << 24
+    uint16_t ja, jb;    // first column of the rectangle
+    uint16_t wb, nc;    // columns of the rectangle along b; columns of the item
+    int32_t c0;         // the item's first column, counted row by row in the rectangle
+    uint16_t k0, k1;    // slabs [k0, k1); k0 == nz: the columns' tails
+    int32_t np;         // positions (k_item_cost)
+    int32_t key;        // planner key over all samples
 };
-static_assert(sizeof(Item) == 16, "Item layout");
-// One range of a multi-range item: item coordinates k in [end of the previous
-// range, end) are positions base + k.
-struct Range {
-    int32_t base, end;
-};
-static_assert(sizeof(Range) == 8, "Range layout");
+static_assert(sizeof(Item) == 32, "Item layout");
 static_assert(sizeof(Block) == 24, "Block layout");
 
 struct SampleDev {
     // sorted sample
     const double *prec;          // 4 doubles per position {a, b, l, w}, sorted order
     const double *srec;          // 8 doubles per shape, sorted order
-    const int32_t *pstart;
     double L, half;
     int los, K, nbins, pad;
     // accumulators (workspace)
@@ -92,27 +93,21 @@ struct SampleDev {
 };
 
 // Planner view of one sample (per-call parameter block).  Its (column, slab
-// group) cells occupy [cell0, cell0 + ncells) of the global cell arrays, its
-// range threads (one per block and stencil column) [t0r, t0r + ntr) and its
-// pack threads (one per block and group of stencil columns) [t0, t0 + nt),
-// both starting at multiples of kPlanThreads, so a workgroup never straddles
-// two samples.
+// group) cells occupy [cell0, cell0 + ncells) of the global cell arrays.
 struct PlanSample {
     Grid g;
     int mode, periodic;
     int ng, G;           // slab groups per column, slabs per group
-    int kx, nxw;         // stencil half width / width in columns
-    int pmax;            // positions per work item at most
-    int ngc;             // plan threads per block: groups of kGroupColumns stencil columns
+    int ncp, cpi;        // position columns per side (g.nc * g.m), columns per item
+    int pbits, pad;      // positions' fine key = (cell << pbits) + line-of-sight part of the slab
+    double fw, hq;       // position column width, height of a line-of-sight part
     double reach_r, reach_z;
-    const int32_t *sstart, *pstart;
-    const int32_t *pfine;  // starts of the positions' fine keys (cell << sbits) + line-of-sight part
-    int sbits, pad2;
-    double x_lo, x_hi;     // (r_p, pi): the pi domain, for cutting slab runs to a block's window
+    double x_lo, x_hi;   // line-of-sight domain, for cutting slab runs to a block's window
+    const int32_t *sstart;
+    const int32_t *pfine;  // starts of the positions' fine keys
+    const int32_t *flags;  // bit 1: some position lies in a column's tail
     const double *srec;  // shape records (block bounding boxes)
     int64_t cell0, ncells;
-    int64_t t0, nt;      // pack threads: worst-case blocks x ngc
-    int64_t t0r, ntr;    // range threads: worst-case blocks x nxw^2
 };
 
 // Finalisation view of one sample: accumulators to caller outputs.
@@ -187,520 +182,349 @@ __device__ __forceinline__ double shift_val(int cls, double L) {
     return cls == 1 ? L : (cls == 2 ? -L : 0.0);
 }
 
-// The slabs within line-of-sight reach of a block (its shapes' extent
-// [zlo, zhi]) for a column at squared transverse distance dxy2, merged into
-// runs [k0, k) of equal periodic shift class and jackknife slab:
-// close(k0, k, class) for each run in slab order.  For (r_p, pi) the runs do
-// not depend on the column; for (r, mu) a column's runs are those of
-// dxy2 = 0 with slabs out of its reach taken off their ends.
-// Whether slab k is within reach of a block's shapes (extent [zlo, zhi]) for
-// a column at squared transverse distance dxy2, and its shift class cz.
-__device__ __forceinline__ bool slab_in(const PlanSample &P, double zlo, double zhi, int k, double dxy2, double rr,
-                                        int &cz) {
+// Whether slab k is within line-of-sight reach of a block's shapes (extent
+// [zlo, zhi]), and its shift class cz.
+__device__ __forceinline__ bool slab_in(const PlanSample &P, double zlo, double zhi, int k, int &cz) {
     const Grid &g = P.g;
     const double m = g.margin;
     double dzmin;
     axis_class(zlo - (k + 1) * g.hz - 2 * m, zhi - k * g.hz + 2 * m, g.L, g.half, P.periodic, dzmin, cz);
-    bool inc = dzmin < P.reach_z + 4 * m;
-    if (inc && P.mode == MIA_RMU) inc = dxy2 + dzmin * dzmin < rr * rr;
-    return inc;
+    return dzmin < P.reach_z + 4 * m;
 }
 
-template <class F>
-__device__ __forceinline__ void slab_runs(const PlanSample &P, double zlo, double zhi, double dxy2, double rr,
-                                          F &&close) {
-    const Grid &g = P.g;
-    int run_k0 = -1, run_cls = 0, run_jz = 0;
-    for (int k = 0; k <= g.nz; ++k) {
-        bool inc = false;
-        int cz = 0;
-        if (k < g.nz) inc = slab_in(P, zlo, zhi, k, dxy2, rr, cz);
-        const int jz = k / g.nzj;
-        if (run_k0 >= 0 && (!inc || cz != run_cls || jz != run_jz)) {
-            close(run_k0, k, run_cls);
-            run_k0 = -1;
-        }
-        if (inc && run_k0 < 0) {
-            run_k0 = k;
-            run_cls = cz;
-            run_jz = jz;
-        }
-    }
+// The positions [pb, pb + n) of one position column (ja, jb) within reach of a
+// block (bounding box of its shapes bb): slabs [k0, k1) of shift class cz, cut
+// to the block's line-of-sight window, or (k0 == nz) the column's tail.
+struct ColumnView {
+    const int32_t *pfine;
+    double L, half, margin, fw, hq, reach_r, x_lo, x_hi;
+    int ncp, nz, pbits, mode, periodic;
+};
+
+template <class PS>
+__device__ __forceinline__ ColumnView column_view(const PS *p) {
+    ColumnView v;
+    v.pfine = p->pfine;
+    v.L = p->g.L;
+    v.half = p->g.half;
+    v.margin = p->g.margin;
+    v.fw = p->fw;
+    v.hq = p->hq;
+    v.reach_r = p->reach_r;
+    v.x_lo = p->x_lo;
+    v.x_hi = p->x_hi;
+    v.ncp = p->ncp;
+    v.nz = p->g.nz;
+    v.pbits = p->pbits;
+    v.mode = p->mode;
+    v.periodic = p->periodic;
+    return v;
 }
 
-// Enumerate the position ranges of one (block, stencil column) pair: slab
-// runs within reach of the block, merged while the periodic shift class and
-// the jackknife slab stay the same, plus the column's anomalous tail.  For
-// each range calls emit(local key, p_begin, p_end, rp, shift byte) with
-// local key = R_s * K1 + R_p.  Shift byte: 2 bits per axis (a, b, l) for the
-// constant shift class, bit 6 the per-pair wrap.  Reach is tested from the
-// bounding box bb of the block's shapes, not from its cells, so a column or
-// slab that no shape of the block can reach is left out.  runs: the block's
-// slab runs when they were stored (count >= 0), else they are walked here.
-template <class F>
-__device__ __forceinline__ void plan_ranges(const PlanSample &P, const Block &B, const double *bb, int so, int K1,
-                                            const int32_t *runs, F &&emit) {
-    const Grid &g = P.g;
-    int ox = so / P.nxw, oy = so % P.nxw;
-    int ia = B.col / g.nc, ib = B.col % g.nc;
-    bool full = P.nxw >= g.nc;
-    int jx = full ? ox : ia - P.kx + ox;
-    int jy = full ? oy : ib - P.kx + oy;
-    if (!full) {
-        if (P.periodic) {
-            jx = ((jx % g.nc) + g.nc) % g.nc;
-            jy = ((jy % g.nc) + g.nc) % g.nc;
-        } else if (jx < 0 || jx >= g.nc || jy < 0 || jy >= g.nc) {
-            return;
-        }
-    }
-    double m = g.margin;
-    double da_min, db_min;
+__device__ __forceinline__ void column_positions(const ColumnView &v, double b0, double b1, double b2, double b3,
+                                                 double zlo, double zhi, int ja, int jb, int k0, int k1, int cz,
+                                                 int &pb, int &n) {
+    const double m = v.margin;
+    double da, db;
     int ca, cb;
-    // separations between the block's shapes (their bounding box bb) and the
-    // target column's positions
-    axis_class(bb[0] - (jx + 1) * g.cw - 2 * m, bb[1] - jx * g.cw + 2 * m, g.L, g.half, P.periodic, da_min, ca);
-    axis_class(bb[2] - (jy + 1) * g.cw - 2 * m, bb[3] - jy * g.cw + 2 * m, g.L, g.half, P.periodic, db_min, cb);
-    double rr = P.reach_r + 4 * m;
-    double dxy2 = da_min * da_min + db_min * db_min;
+    axis_class(b0 - (ja + 1) * v.fw - 2 * m, b1 - ja * v.fw + 2 * m, v.L, v.half, v.periodic, da, ca);
+    axis_class(b2 - (jb + 1) * v.fw - 2 * m, b3 - jb * v.fw + 2 * m, v.L, v.half, v.periodic, db, cb);
+    const double rr = v.reach_r + 4 * m;
+    const double dxy2 = da * da + db * db;
+    pb = 0;
+    n = 0;
     if (dxy2 >= rr * rr) return;
-    // line-of-sight extent of the block's shapes (a tail block's shapes may lie anywhere)
-    const double zlo = bb[4], zhi = bb[5];
-    int col = jx * g.nc + jy;
-    int64_t base = (int64_t)col * (g.nz + 1);
-    const int kr = B.rs * K1;
-    auto range = [&](int p_begin, int p_end, int rp, int cz) {
-        if (p_end <= p_begin) return;
-        // mixed shift classes take the per-pair minimum-image wrap; a
-        // non-periodic box never wraps (classes are always 0 there, and the
-        // anomalous tail's "any LOS value" class means no shift)
-        bool wrap = P.periodic && ((ca == 3) || (cb == 3) || (cz == 3));
-        uint8_t sh = (uint8_t)((ca == 3 ? 0 : ca) | ((cb == 3 ? 0 : cb) << 2) |
-                               ((cz == 3 ? 0 : cz) << 4) | (wrap ? 64 : 0));
-        emit(kr + rp, p_begin, p_end, rp, sh);
-    };
-    // the positions of a run of slabs [k0, k) of one shift class
-    auto run = [&](int k0, int k, int cls) {
-        int pb = P.pstart[base + k0], pe = P.pstart[base + k];
-        if (cls != 3 && P.sbits > 0) {
-            // the run's positions are in line-of-sight order (to 2^-sbits
-            // of a slab): keep those a shape of the block can pair with,
-            // l in (zlo + sh - x_hi, zhi + sh - x_lo] for the run's shift
-            // sh, one fine bucket of slack on each side
-            const double sh = shift_val(cls, g.L);
-            double wlo, whi;
-            if (P.mode == MIA_RPPI) {
-                wlo = zlo + sh - P.x_hi - 4 * m;
-                whi = zhi + sh - P.x_lo + 4 * m;
-            } else {
-                const double rz2 = sqrt(fmax(rr * rr - dxy2, 0.0));
-                wlo = zlo + sh - rz2 - 4 * m;
-                whi = zhi + sh + rz2 + 4 * m;
-            }
-            const double hq = g.hz / (double)(1 << P.sbits);
-            const int64_t f0 = (int64_t)k0 << P.sbits, f1 = ((int64_t)k << P.sbits) - 1;
-            const double flo = floor(wlo / hq) - 1.0, fhi = floor(whi / hq) + 1.0;
-            const int64_t fa = flo < (double)f0 ? f0 : (flo > (double)f1 ? f1 + 1 : (int64_t)flo);
-            const int64_t fb = fhi > (double)f1 ? f1 : (fhi < (double)f0 ? f0 - 1 : (int64_t)fhi);
-            const int64_t fbase = base << P.sbits;
-            if (fb < fa) {
-                pe = pb;
-            } else {
-                pb = P.pfine[fbase + fa];
-                pe = P.pfine[fbase + fb + 1];
-            }
+    const int64_t base = ((int64_t)ja * v.ncp + jb) * (v.nz + 1);
+    int64_t f0 = (base + k0) << v.pbits, f1 = (base + k1) << v.pbits;
+    if (cz != 3) {
+        // a shape of the block pairs with l in (zlo + sh - x_hi, zhi + sh - x_lo]
+        // for the run's shift sh ((r, mu): within the sphere over the column)
+        const double sh = shift_val(cz, v.L);
+        double wlo, whi;
+        if (v.mode == MIA_RPPI) {
+            wlo = zlo + sh - v.x_hi - 4 * m;
+            whi = zhi + sh - v.x_lo + 4 * m;
+        } else {
+            const double rz = sqrt(rr * rr - dxy2);
+            wlo = zlo + sh - rz - 4 * m;
+            whi = zhi + sh + rz + 4 * m;
         }
-        range(pb, pe, region_of(g, jx, jy, k0), cls);
-    };
-    if (runs && runs[0] >= 0) {
-        // the block's slab runs: (r_p, pi) the same for every column; (r, mu)
-        // those of the block's own column, cut at both ends to this column's
-        // reach (the slabs a column reaches within one run are contiguous,
-        // the distance growing away from the block on either side)
-        for (int r = 0; r < runs[0]; ++r) {
-            const int v = runs[1 + r];
-            int k0 = v & 0x7ff, k1 = (v >> 11) & 0x7ff, cz;
-            if (P.mode == MIA_RMU) {
-                while (k0 < k1 && !slab_in(P, zlo, zhi, k0, dxy2, rr, cz)) ++k0;
-                while (k1 > k0 && !slab_in(P, zlo, zhi, k1 - 1, dxy2, rr, cz)) --k1;
-                if (k0 >= k1) continue;
-            }
-            run(k0, k1, (v >> 22) & 3);
-        }
-    } else {
-        slab_runs(P, zlo, zhi, dxy2, rr, run);
+        const double q0 = (double)(k0 << v.pbits), q1 = (double)(k1 << v.pbits);
+        const double lo = fmin(fmax(floor(wlo / v.hq), q0), q1), hi = fmin(fmax(floor(whi / v.hq) + 1.0, q0), q1);
+        f0 = (base << v.pbits) + (int64_t)lo;
+        f1 = (base << v.pbits) + (int64_t)hi;
+        if (f1 <= f0) return;
     }
-    // anomalous tail of the target column: region 0, any line-of-sight value
-    range(P.pstart[base + g.nz], P.pstart[base + g.nz + 1], 0, 3);
+    pb = v.pfine[f0];
+    n = v.pfine[f1] - pb;
 }
 
 constexpr int kPlanThreads = 256;
-constexpr int kBlockRuns = 15;          // slab runs of a block kept for its columns
-constexpr int kPlanGridPerCu = 16;      // workgroups per CU of the planner's persistent grid
+constexpr int kPlanWaves = kPlanThreads / kWave;
+constexpr int kPlanGridPerCu = 8;        // workgroups per CU of the planner's persistent grids
+constexpr int kItemPositions = 8192;    // positions of an item, about
 constexpr int64_t kItemOverhead = 256;  // per-item cost, in pair evaluations
-constexpr int kOpenItems = 4;           // items a plan thread fills at once (one per key and shift)
-
-// One position range of a (block, stencil column) pair as plan_ranges
-// enumerates it.
-struct RawRange {
-    int32_t pb, pe;   // positions [pb, pe)
-    int32_t key;      // local key R_s * K1 + R_p
-    int32_t w;        // R_p | shift byte << 16
-};
-static_assert(sizeof(RawRange) == 16, "RawRange layout");
-
-struct RangeLaunch {
-    const PlanSample *ps;
-    const int64_t *t0r;       // [S + 1] first range thread of each sample (t0r[S]: total)
-    int S, K1;
-    const int32_t *boff;
-    const Block *blocks;
-    const double *bbox;
-    const int32_t *bruns;     // slab runs of every block (k_blocks)
-    RawRange *raw;            // the ranges, one chunk per workgroup
-    unsigned long long *raw_cursor;  // ranges taken (may pass raw_cap)
-    int64_t raw_cap;
-    int32_t *roff, *rcnt;     // [range threads] first range and number of ranges of the thread
-    unsigned long long *overflow;
-};
-
-// The position ranges of every (block, stencil column) pair: one thread per
-// pair counts its ranges, the workgroup reserves one chunk of the range list,
-// and each thread stores its ranges there with their first index and count.
-__global__ __launch_bounds__(kPlanThreads) void k_plan_ranges(RangeLaunch A) {
-    __shared__ int cnt_l;
-    __shared__ int64_t base_l;
-    const int64_t nvwg = (A.t0r[A.S] + kPlanThreads - 1) / kPlanThreads;
-    for (int64_t vb = blockIdx.x; vb < nvwg; vb += gridDim.x) {
-        const int s = find_sample(A.t0r, A.S, vb * kPlanThreads);
-        const PlanSample &P = A.ps[s];
-        const int64_t tl0 = vb * kPlanThreads - P.t0r;
-        const int nx2 = P.nxw * P.nxw;
-        const int b0 = A.boff[P.cell0], b1 = A.boff[P.cell0 + P.ncells];
-        // the whole virtual workgroup lies past the sample's blocks
-        if (tl0 >= P.ntr || b0 + tl0 / nx2 >= b1) continue;
-        const int64_t tl = tl0 + threadIdx.x;
-        const int blk = b0 + (int)(tl / nx2);
-        const bool active = tl < P.ntr && blk < b1;
-        const int so = (int)(tl % nx2);
-        const double *bb = A.bbox + 6 * (int64_t)blk;
-        Block B{};
-        if (active) B = A.blocks[blk];
-        __syncthreads();  // the previous virtual workgroup is done with cnt_l, base_l
-        if (threadIdx.x == 0) cnt_l = 0;
-        __syncthreads();
-        int n = 0;
-        const int32_t *br = A.bruns + (kBlockRuns + 1) * (int64_t)blk;
-        if (active) plan_ranges(P, B, bb, so, A.K1, br, [&](int, int, int, int, uint8_t) { ++n; });
-        const int off = n ? atomicAdd(&cnt_l, n) : 0;
-        __syncthreads();
-        if (threadIdx.x == 0) base_l = cnt_l ? (int64_t)atomicAdd(A.raw_cursor, (unsigned long long)cnt_l) : 0;
-        __syncthreads();
-        int64_t o = base_l + off;
-        if (o + n > A.raw_cap) {
-            if (n) atomicOr(A.overflow, 1ull);
-            n = 0;
-            o = 0;
-        }
-        if (active) {
-            A.roff[P.t0r + tl] = (int32_t)o;
-            A.rcnt[P.t0r + tl] = n;
-        }
-        if (active && n)
-            plan_ranges(P, B, bb, so, A.K1, br, [&](int k, int pb, int pe, int rp, uint8_t sh) {
-                A.raw[o++] = RawRange{pb, pe, k, (rp & 0xffff) | ((int)sh << 16)};
-            });
-    }
-}
-
-// A finished item of a plan thread.
-struct OpenItem {
-    int key, rp, np, nr;
-    int sh;
-    int32_t p[kItemRanges];  // first position of every range
-    int32_t e[kItemRanges];  // end of every range in item coordinates
-};
-
-// Pack the ranges of the stencil columns [so0, so1) of one block (range
-// threads tr0 + so) into work items: ranges of one (key, shift) go into the
-// same item, in column order, until it holds pmax positions or kItemRanges
-// ranges (a range that does not fit is split).  Up to kOpenItems items are
-// filled at once; a range of a further (key, shift) finishes the fullest.
-// close(o) is called once per finished item, in an order fixed by the data
-// alone.  The open items live in registers: every array index is a
-// compile-time constant after unrolling.
-template <class F>
-__device__ __forceinline__ void pack_items(int pmax, const RawRange *raw, const int32_t *roff, const int32_t *rcnt,
-                                           int64_t tr0, int so0, int so1, F &&close) {
-    int okey[kOpenItems], osh[kOpenItems], orp[kOpenItems], onp[kOpenItems], onr[kOpenItems];
-    int32_t op[kOpenItems][kItemRanges], oe[kOpenItems][kItemRanges];
-#pragma unroll
-    for (int i = 0; i < kOpenItems; ++i) {
-        okey[i] = -1;
-        osh[i] = orp[i] = onp[i] = onr[i] = 0;
-#pragma unroll
-        for (int j = 0; j < kItemRanges; ++j) op[i][j] = oe[i][j] = 0;
-    }
-    auto finish = [&](int s) {
-        OpenItem o;
-#pragma unroll
-        for (int i = 0; i < kOpenItems; ++i)
-            if (i == s) {
-                o.key = okey[i];
-                o.rp = orp[i];
-                o.sh = osh[i];
-                o.np = onp[i];
-                o.nr = onr[i];
-#pragma unroll
-                for (int j = 0; j < kItemRanges; ++j) {
-                    o.p[j] = op[i][j];
-                    o.e[j] = oe[i][j];
-                }
-                onp[i] = 0;
-                onr[i] = 0;
-            }
-        close(o);
-    };
-    for (int so = so0; so < so1; ++so) {
-        const int n = rcnt[tr0 + so];
-        const int64_t o0 = roff[tr0 + so];
-        for (int q = 0; q < n; ++q) {
-            const RawRange r = raw[o0 + q];
-            const int k = r.key, sh = (r.w >> 16) & 0xff, rp = (int16_t)(r.w & 0xffff);
-            int pb = r.pb;
-            const int pe = r.pe;
-            int s = -1;
-#pragma unroll
-            for (int i = 0; i < kOpenItems; ++i)
-                if (okey[i] == k && osh[i] == sh) s = i;
-            int evict = -1;
-            if (s < 0) {
-                // a free slot, else the fullest item is finished early
-#pragma unroll
-                for (int i = kOpenItems - 1; i >= 0; --i)
-                    if (okey[i] < 0) s = i;
-                if (s < 0) {
-                    s = 0;
-                    int most = onp[0];
-#pragma unroll
-                    for (int i = 1; i < kOpenItems; ++i)
-                        if (onp[i] > most) {
-                            most = onp[i];
-                            s = i;
-                        }
-                    evict = s;
-                }
-            }
-            while (evict >= 0 || pb < pe) {
-                if (evict >= 0) {
-                    finish(evict);
-                    evict = -1;
-                }
-                bool full = false;
-                int take = 0;
-#pragma unroll
-                for (int i = 0; i < kOpenItems; ++i)
-                    if (i == s) {
-                        okey[i] = k;
-                        osh[i] = sh;
-                        orp[i] = rp;
-                        take = pe - pb < pmax - onp[i] ? pe - pb : pmax - onp[i];
-#pragma unroll
-                        for (int j = 0; j < kItemRanges; ++j)
-                            if (j == onr[i]) {
-                                op[i][j] = pb;
-                                oe[i][j] = onp[i] + take;
-                            }
-                        onp[i] += take;
-                        onr[i] += 1;
-                        full = onp[i] == pmax || onr[i] == kItemRanges;
-                    }
-                pb += take;
-                if (full) evict = s;
-                if (pb >= pe && evict >= 0) {
-                    finish(evict);
-                    evict = -1;
-                }
-            }
-        }
-    }
-    for (int i = 0; i < kOpenItems; ++i) {
-        bool open = false;
-#pragma unroll
-        for (int q = 0; q < kOpenItems; ++q)
-            if (q == i) open = okey[q] >= 0 && onr[q] > 0;
-        if (open) finish(i);
-    }
-}
+// Segments a block's reach falls into along one axis: the sub-boxes it meets
+// (at most one of them twice, where the periodic image closes on itself) plus
+// the changes of shift class (-L, mixed, none, mixed, +L).
+constexpr int kSegExtra = 6;
+constexpr int kMaxSegs = 16 + kSegExtra;  // fast_path_fits: at most 16 sub-boxes per side
 
 struct PlanLaunch {
     const PlanSample *ps;
-    const int64_t *t0;        // [S + 1] first pack thread of each sample (t0[S]: total)
-    int S;
+    int64_t ncells;           // cells of all samples
     int K1;                   // regions + 1 of the largest sample's key space (keys per sample K1^2)
+    int kseg;                 // segments stored per axis
     const int32_t *boff;      // block offset of every cell (exclusive scan of the block counts)
     const Block *blocks;
-    const RawRange *raw;      // the ranges of every (block, column) pair
-    const int32_t *roff, *rcnt;
-    unsigned long long *key_count;   // count pass
-    unsigned long long *key_cursor;  // emit pass
+    double *bbox;             // bounding box {a_lo, a_hi, b_lo, b_hi, l_lo, l_hi} of every block's shapes
+    uint32_t *geo;            // per block: 3 counts, then kseg segments per axis (a, b, l)
+    unsigned long long *key_count;   // k_block_geom
+    unsigned long long *key_cursor;  // k_emit_items
     const int64_t *key_off;
     Item *items;
-    int64_t *cost;            // emit pass: balancing cost of every item
     int64_t cap;              // item capacity
-    Range *ranges;            // emit pass: range records of the multi-range items
-    unsigned long long *range_cursor;  // emit pass: range records taken (may pass range_cap)
-    int64_t range_cap;
-    unsigned long long *overflow;  // set when the items or ranges exceed their capacity
-    unsigned long long *candidates;  // emit pass: sum of ns * np
-    int emit;
-    int local;                // 1: aggregate per workgroup in LDS (K1^2 keys fit)
-    // deterministic order: with it, the emit pass also writes every item's
-    // (key << 32 | pack thread); a stable sort by it fixes the order the
-    // cursor atomics gave the items of one key
+    unsigned long long *overflow;  // set when the items exceed their capacity
+    // deterministic order: with it, every item's (key, block, rectangle) word;
+    // a stable sort by it fixes the order the cursor atomics gave the items of one key
     unsigned long long *sort_key;
+    int sort_shift;
 };
 
-// Count (emit == 0) or emit the work items of every (block, group of
-// kGroupColumns stencil columns) pair of every sample, counting-sorted by key
-// (sample, R_s, R_p).  A persistent grid walks the virtual workgroups of the
-// samples' worst-case thread ranges and skips those past a sample's actual
-// block count (known only on the device).  With `local` the key counts are
-// aggregated per workgroup in LDS, so each key sees one global atomic per
-// workgroup instead of one per item.  The emit pass packs the items twice:
-// first to reserve the workgroup's slots (keys, range records), then to place
-// them.  Items or ranges beyond their capacity are not written and raise the
-// overflow flag (the host then grows the capacity and counts again).
-__global__ __launch_bounds__(kPlanThreads) void k_plan_items(PlanLaunch A) {
-    // local: reserved bases [nk] (64-bit), then counts [nk]
-    extern __shared__ int64_t lmem[];
-    const int nk = A.K1 * A.K1;
-    int64_t *lbase = lmem;
-    int32_t *lcnt = (int32_t *)(lmem + nk);
-    __shared__ unsigned long long cand_l;
-    __shared__ int rcount_l;
-    __shared__ int64_t rbase_l;
-    const int64_t nvwg = (A.t0[A.S] + kPlanThreads - 1) / kPlanThreads;
-    const bool local = A.local != 0;
-    unsigned long long cand = 0;
-    for (int64_t vb = blockIdx.x; vb < nvwg; vb += gridDim.x) {
-        const int s = find_sample(A.t0, A.S, vb * kPlanThreads);
-        const PlanSample &P = A.ps[s];
-        const int64_t tl0 = vb * kPlanThreads - P.t0;
-        const int nx2 = P.nxw * P.nxw;
-        const int ngc = P.ngc;
-        const int b0 = A.boff[P.cell0], b1 = A.boff[P.cell0 + P.ncells];
-        // the whole virtual workgroup lies past the sample's blocks
-        if (tl0 >= P.nt || b0 + tl0 / ngc >= b1) continue;
-        const int64_t tl = tl0 + threadIdx.x;
-        const int blk = b0 + (int)(tl / ngc);
-        const bool active = tl < P.nt && blk < b1;
-        const int so0 = (int)(tl % ngc) * kGroupColumns;
-        const int so1 = so0 + kGroupColumns < nx2 ? so0 + kGroupColumns : nx2;
-        const int64_t tr0 = P.t0r + (int64_t)(blk - b0) * nx2;  // the block's first range thread
-        const int kb = s * nk;
-        const int ns = active ? A.blocks[blk].ns : 0;
-        __syncthreads();  // the previous virtual workgroup is done with the LDS tables
-        if (local)
-            for (int j = threadIdx.x; j < nk; j += blockDim.x) {
-                lcnt[j] = 0;
-                lbase[j] = 0;
-            }
-        if (threadIdx.x == 0) rcount_l = 0;
-        __syncthreads();
-        // pass 1: key counts (count pass; emit pass with local) and the
-        // thread's range records (emit pass)
-        int nrng = 0;
-        if (active)
-            pack_items(P.pmax, A.raw, A.roff, A.rcnt, tr0, so0, so1, [&](const OpenItem &o) {
-                if (!A.emit || local) {
-                    if (local)
-                        atomicAdd(&lcnt[o.key], 1);
-                    else
-                        atomicAdd(&A.key_count[kb + o.key], 1ull);
-                }
-                if (o.nr > 1) nrng += o.nr;
-            });
-        if (!A.emit) {
-            if (local) {
-                __syncthreads();
-                for (int j = threadIdx.x; j < nk; j += blockDim.x)
-                    if (lcnt[j]) atomicAdd(&A.key_count[kb + j], (unsigned long long)lcnt[j]);
-            }
-            continue;
+// A segment: indices [j0, j1] of one shift class, 12 bits each and 2 bits of class.
+__device__ __forceinline__ int seg_j0(uint32_t s) { return s & 0xfff; }
+__device__ __forceinline__ int seg_j1(uint32_t s) { return (s >> 16) & 0xfff; }
+__device__ __forceinline__ int seg_cls(uint32_t s) { return (s >> 12) & 3; }
+
+// The rectangles of one block: every combination of an a segment, a b segment
+// and a line-of-sight run (plus, where the sample has tail positions, the
+// tails).  Calls f(index, key, items, seg a, seg b, run, R_p), the run ~0 for
+// the tail, for this lane's combinations.
+template <class F>
+__device__ __forceinline__ void for_rects(const PlanSample &P, int rs, int K1, int nA, int nB, int nR,
+                                          const uint32_t *segA, const uint32_t *segB, const uint32_t *segR, int lane,
+                                          F &&f) {
+    const Grid &g = P.g;
+    const int nL = nR + ((*P.flags & 2) ? 1 : 0);
+    const int T = nA * nB * nL;
+    const int pj = g.ncj * g.m;
+    for (int t = lane; t < T; t += kWave) {
+        const int ir = t % nL, ib = (t / nL) % nB, ia = t / (nL * nB);
+        const uint32_t a = segA[ia], b = segB[ib], r = ir < nR ? segR[ir] : ~0u;
+        const int cols = (seg_j1(a) - seg_j0(a) + 1) * (seg_j1(b) - seg_j0(b) + 1);
+        int rp = 0;
+        if (g.jk > 0 && ir < nR) {
+            int j[3];
+            j[g.ax_a] = seg_j0(a) / pj;
+            j[g.ax_b] = seg_j0(b) / pj;
+            j[g.los] = seg_j0(r) / g.nzj;
+            rp = j[0] * g.jk * g.jk + j[1] * g.jk + j[2];
         }
-        const int roff = nrng ? atomicAdd(&rcount_l, nrng) : 0;
-        __syncthreads();
-        if (local)
-            for (int j = threadIdx.x; j < nk; j += blockDim.x) {
-                const int c = lcnt[j];
-                lbase[j] = c ? (int64_t)atomicAdd(&A.key_cursor[kb + j], (unsigned long long)c) : 0;
-                lcnt[j] = 0;
-            }
-        if (threadIdx.x == 0)
-            rbase_l = rcount_l ? (int64_t)atomicAdd(A.range_cursor, (unsigned long long)rcount_l) : 0;
-        __syncthreads();
-        int64_t rnext = rbase_l + roff;
-        if (rnext + nrng > A.range_cap) {
-            atomicOr(A.overflow, 1ull);
-            continue;
-        }
-        // pass 2: place
-        if (active)
-            pack_items(P.pmax, A.raw, A.roff, A.rcnt, tr0, so0, so1, [&](const OpenItem &o) {
-                const int k = o.key;
-                const int64_t slot = A.key_off[kb + k] + (local ? lbase[k] + (int64_t)atomicAdd(&lcnt[k], 1)
-                                                                : (int64_t)atomicAdd(&A.key_cursor[kb + k], 1ull));
-                if (slot >= A.cap) {
-                    atomicOr(A.overflow, 1ull);
-                    return;
-                }
-                Item it;
-                it.blk = blk;
-                it.np = o.np;
-                it.rp = (int16_t)o.rp;
-                it.shifts = (uint8_t)o.sh;
-                it.nr = (uint8_t)o.nr;
-                if (o.nr == 1) {
-                    it.p0 = o.p[0];
-                } else {
-                    it.p0 = (int32_t)rnext;
-#pragma unroll
-                    for (int i = 0; i < kItemRanges; ++i)
-                        if (i < o.nr) {
-                            Range r;
-                            r.base = o.p[i] - (i ? o.e[i - 1] : 0);
-                            r.end = o.e[i];
-                            A.ranges[rnext + i] = r;
-                        }
-                    rnext += o.nr;
-                }
-                A.items[slot] = it;
-                if (A.sort_key)
-                    A.sort_key[slot] = ((unsigned long long)(kb + k) << 32) | (unsigned long long)(P.t0 + tl);
-                // a wave pays for whole 64-lane position batches plus a fixed
-                // per-item overhead, whatever the item's true pair count
-                A.cost[slot] = (int64_t)ns * (((it.np + kWave - 1) / kWave) * kWave) + kItemOverhead;
-                cand += (unsigned long long)ns * it.np;
-            });
+        f(t, rs * K1 + rp, (cols + P.cpi - 1) / P.cpi, a, b, r, rp);
     }
-    if (!A.emit) return;
-    __syncthreads();
+}
+
+// One wave per shape block: the bounding box of its shapes, its reach along
+// each axis as segments of one sub-box and one shift class, and the items per
+// key.  Reach is tested from the bounding box, not from the block's cells.
+__global__ __launch_bounds__(kPlanThreads) void k_block_geom(PlanLaunch A) {
+    __shared__ uint32_t seg[kPlanWaves][3][kMaxSegs + 2];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int nblk = A.boff[A.ncells];
+    const int gstride = 3 + 3 * A.kseg;
+    for (int blk = blockIdx.x * kPlanWaves + wv; blk < nblk; blk += gridDim.x * kPlanWaves) {
+        const Block B = A.blocks[blk];
+        const PlanSample &P = A.ps[B.sample];
+        const Grid &g = P.g;
+        double lo[3], hi[3];
+        {
+            const double *r = P.srec + 8 * (int64_t)(B.s0 + (lane < B.ns ? lane : 0));
+#pragma unroll
+            for (int k = 0; k < 3; ++k) lo[k] = hi[k] = r[k];
+        }
+        for (int d = kWave / 2; d > 0; d >>= 1)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = fmin(lo[k], __shfl_xor(lo[k], d));
+                hi[k] = fmax(hi[k], __shfl_xor(hi[k], d));
+            }
+        if (lane < 3) {
+            A.bbox[6 * (int64_t)blk + 2 * lane] = lane == 0 ? lo[0] : (lane == 1 ? lo[1] : lo[2]);
+            A.bbox[6 * (int64_t)blk + 2 * lane + 1] = lane == 0 ? hi[0] : (lane == 1 ? hi[1] : hi[2]);
+        }
+        const double m = g.margin, rr = P.reach_r + 4 * m;
+        int cnt[3];
+        // lane i of a pass holds the i-th column (slab) of the axis with its
+        // state (index | class << 12 | sub-box << 16, -1: out of reach); a
+        // segment starts where the state does not continue the one before
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            uint16_t *half = (uint16_t *)seg[wv][ax];
+            int u0 = 0, W = g.nz;
+            const int n = ax < 2 ? P.ncp : g.nz;
+            if (ax < 2) {
+                const int a0 = (int)floor((lo[ax] - rr) / P.fw) - 1, a1 = (int)floor((hi[ax] + rr) / P.fw) + 1;
+                u0 = a0;
+                W = a1 - a0 + 1;
+                if (W >= n || !P.periodic) {
+                    u0 = 0;
+                    W = n;
+                }
+            }
+            auto state = [&](int i) {
+                if (i < 0 || i >= W) return -1;
+                int j = u0 + i;
+                int cls;
+                if (ax < 2) {
+                    j = j < 0 ? j + n : (j >= n ? j - n : j);
+                    double dmin;
+                    axis_class(lo[ax] - (j + 1) * P.fw - 2 * m, hi[ax] - j * P.fw + 2 * m, g.L, g.half, P.periodic,
+                               dmin, cls);
+                    if (!(dmin < rr)) return -1;
+                    return j | (cls << 12) | (j / (g.ncj * g.m) << 16);
+                }
+                if (!slab_in(P, lo[2], hi[2], j, cls)) return -1;
+                return j | (cls << 12) | (j / g.nzj << 16);
+            };
+            // b continues a: the next index of the same class and sub-box
+            auto cont = [](int a, int b) { return a >= 0 && b >= 0 && b == a + 1; };
+            int c = 0;
+            for (int i0 = 0; i0 < W; i0 += kWave) {
+                const int i = i0 + lane;
+                const int s = state(i);
+                const bool st = s >= 0 && !cont(state(i - 1), s), en = s >= 0 && !cont(s, state(i + 1));
+                const uint64_t ms = __ballot(st);
+                const int at = c + __popcll(ms & ((2ull << lane) - 1)) - 1;
+                if (st && at < A.kseg) half[2 * at] = (uint16_t)(s & 0x3fff);
+                if (en && at < A.kseg) half[2 * at + 1] = (uint16_t)(s & 0xfff);
+                c += __popcll(ms);
+            }
+            // (kseg bounds the segments of any reach; see kSegExtra)
+            cnt[ax] = c < A.kseg ? c : A.kseg;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        uint32_t *G = A.geo + (int64_t)gstride * blk;
+        if (lane < 3) G[lane] = lane == 0 ? cnt[0] : (lane == 1 ? cnt[1] : cnt[2]);
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax)
+            if (lane < cnt[ax]) G[3 + ax * A.kseg + lane] = seg[wv][ax][lane];
+        const int kb = B.sample * A.K1 * A.K1;
+        int same = 0;
+        for_rects(P, B.rs, A.K1, cnt[0], cnt[1], cnt[2], seg[wv][0], seg[wv][1], seg[wv][2], lane,
+                  [&](int, int key, int items, uint32_t, uint32_t, uint32_t, int) {
+                      if (A.K1 == 1)
+                          same += items;
+                      else
+                          atomicAdd(&A.key_count[kb + key], (unsigned long long)items);
+                  });
+        if (A.K1 == 1) {
+            for (int d = kWave / 2; d > 0; d >>= 1) same += __shfl_xor(same, d);
+            if (lane == 0 && same) atomicAdd(&A.key_count[kb], (unsigned long long)same);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // seg is reused
+    }
+}
+
+// One wave per shape block: its items, counting-sorted by key (sample, R_s,
+// R_p).  Items beyond the capacity are not written and raise the overflow flag
+// (the host then grows the capacity and counts again).
+__global__ __launch_bounds__(kPlanThreads) void k_emit_items(PlanLaunch A) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int nblk = A.boff[A.ncells];
+    const int gstride = 3 + 3 * A.kseg;
+    for (int blk = blockIdx.x * kPlanWaves + wv; blk < nblk; blk += gridDim.x * kPlanWaves) {
+        const Block B = A.blocks[blk];
+        const PlanSample &P = A.ps[B.sample];
+        const uint32_t *G = A.geo + (int64_t)gstride * blk;
+        const int kb = B.sample * A.K1 * A.K1;
+        for_rects(P, B.rs, A.K1, G[0], G[1], G[2], G + 3, G + 3 + A.kseg, G + 3 + 2 * A.kseg, lane,
+                  [&](int t, int key, int n, uint32_t a, uint32_t b, uint32_t r, int rp) {
+                      const int64_t slot =
+                          A.key_off[kb + key] + (int64_t)atomicAdd(&A.key_cursor[kb + key], (unsigned long long)n);
+                      if (slot + n > A.cap) {
+                          atomicOr(A.overflow, 1ull);
+                          return;
+                      }
+                      const int ca = seg_cls(a), cb = seg_cls(b), cz = r == ~0u ? 3 : seg_cls(r);
+                      // mixed shift classes take the per-pair minimum-image wrap; a
+                      // non-periodic box never wraps (classes are always 0 there, and
+                      // the tail's "any line-of-sight value" class means no shift)
+                      const bool wrap = P.periodic && ((ca == 3) || (cb == 3) || (cz == 3));
+                      const int sh = (ca == 3 ? 0 : ca) | ((cb == 3 ? 0 : cb) << 2) | ((cz == 3 ? 0 : cz) << 4) |
+                                     (wrap ? 64 : 0);
+                      const int cols = (seg_j1(a) - seg_j0(a) + 1) * (seg_j1(b) - seg_j0(b) + 1);
+                      Item it;
+                      it.blk = blk;
+                      it.w = (rp & 0xffff) | (sh << 16) | (cz << 24);
+                      it.ja = (uint16_t)seg_j0(a);
+                      it.jb = (uint16_t)seg_j0(b);
+                      it.wb = (uint16_t)(seg_j1(b) - seg_j0(b) + 1);
+                      it.k0 = (uint16_t)(r == ~0u ? P.g.nz : seg_j0(r));
+                      it.k1 = (uint16_t)(r == ~0u ? P.g.nz + 1 : seg_j1(r) + 1);
+                      it.np = 0;
+                      it.key = kb + key;
+                      for (int i = 0; i < n; ++i) {
+                          it.c0 = i * P.cpi;
+                          it.nc = (uint16_t)(cols - it.c0 < P.cpi ? cols - it.c0 : P.cpi);
+                          A.items[slot + i] = it;
+                          if (A.sort_key)
+                              A.sort_key[slot + i] = ((unsigned long long)(kb + key) << A.sort_shift) |
+                                                     ((unsigned long long)blk * (kMaxSegs * kMaxSegs * (kMaxSegs + 1)) + t);
+                      }
+                  });
+    }
+}
+
+// The lane's column of an item, and its positions.
+__device__ __forceinline__ void item_column(const ColumnView &v, const double *bb, int ja, int jb, int wb, int nc,
+                                            int c0, int k0, int k1, int cz, int lane, int &pb, int &n) {
+    pb = 0;
+    n = 0;
+    if (lane < nc) {
+        const int c = c0 + lane, row = c / wb;
+        column_positions(v, bb[0], bb[1], bb[2], bb[3], bb[4], bb[5], ja + row, jb + (c - row * wb), k0, k1, cz, pb, n);
+    }
+}
+
+// One wave per item: its positions and balancing cost.
+__global__ __launch_bounds__(kPlanThreads) void k_item_cost(const PlanSample *ps, const Block *blocks,
+                                                            const double *bbox, const int64_t *n_items, Item *items,
+                                                            int64_t *cost, unsigned long long *candidates) {
+    __shared__ unsigned long long cand_l;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (threadIdx.x == 0) cand_l = 0;
     __syncthreads();
+    const int64_t n = *n_items;
+    unsigned long long cand = 0;
+    for (int64_t i = (int64_t)blockIdx.x * kPlanWaves + wv; i < n; i += (int64_t)gridDim.x * kPlanWaves) {
+        const Item it = items[i];
+        const Block &B = blocks[it.blk];
+        const ColumnView v = column_view(ps + B.sample);
+        int pb, np;
+        item_column(v, bbox + 6 * (int64_t)it.blk, it.ja, it.jb, it.wb, it.nc, it.c0, it.k0, it.k1, (it.w >> 24) & 3,
+                    lane, pb, np);
+        for (int d = kWave / 2; d > 0; d >>= 1) np += __shfl_xor(np, d);
+        if (lane == 0) {
+            items[i].np = np;
+            // a wave pays for whole 64-lane position batches plus a fixed
+            // per-item overhead, whatever the item's true pair count
+            cost[i] = (int64_t)B.ns * (((np + kWave - 1) / kWave) * kWave) + kItemOverhead;
+            cand += (unsigned long long)B.ns * np;
+        }
+    }
     if (cand) atomicAdd(&cand_l, cand);
     __syncthreads();
-    if (threadIdx.x == 0 && cand_l) atomicAdd(A.candidates, cand_l);
+    if (threadIdx.x == 0 && cand_l) atomicAdd(candidates, cand_l);
 }
 
 // Shape blocks: per (column, slab group) cell of every sample, the number of
 // blocks of at most bsz shapes (count), then the blocks themselves at the
-// scanned offsets (emit) with their bounding boxes and, for (r_p, pi), their
-// slab runs (kBlockRuns + 1 ints per block: the count, -1 if they do not fit,
-// then k0 | k1 << 11 | class << 22 per run).  cell0[S + 1] locates each
-// sample's cells.
+// scanned offsets (emit).  cell0[S + 1] locates each sample's cells.
 __global__ void k_blocks(const PlanSample *ps, const int64_t *cell0, int S, int bsz,
-                         int32_t *nb, const int32_t *boff, Block *blocks, double *bbox, int32_t *bruns) {
+                         int32_t *nb, const int32_t *boff, Block *blocks) {
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= cell0[S]) return;
     const int s = find_sample(cell0, S, c);
@@ -733,33 +557,6 @@ __global__ void k_blocks(const PlanSample *ps, const int64_t *cell0, int S, int 
         B.sample = s;
         B.rs = rs;
         blocks[o + b] = B;
-        // bounding box {a_lo, a_hi, b_lo, b_hi, l_lo, l_hi} of the block's shapes
-        double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-        for (int j = 0; j < B.ns; ++j) {
-            const double *r = P.srec + 8 * (int64_t)(B.s0 + j);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                lo[k] = fmin(lo[k], r[k]);
-                hi[k] = fmax(hi[k], r[k]);
-            }
-        }
-        double *bb = bbox + 6 * (int64_t)(o + b);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            bb[2 * k] = lo[k];
-            bb[2 * k + 1] = hi[k];
-        }
-        if (bruns) {
-            int32_t *br = bruns + (kBlockRuns + 1) * (int64_t)(o + b);
-            // (r, mu): the runs of a column at zero transverse distance, the
-            // widest reach of any column
-            int nr = 0;
-            slab_runs(P, lo[2], hi[2], 0.0, P.reach_r + 4 * g.margin, [&](int k0, int k1, int cls) {
-                if (nr < kBlockRuns) br[1 + nr] = k0 | (k1 << 11) | (cls << 22);
-                ++nr;
-            });
-            br[0] = nr <= kBlockRuns ? nr : -1;
-        }
     }
 }
 
@@ -928,27 +725,28 @@ __global__ void k_finalize_det(const FinSample *fs, const int64_t *fin0, int S, 
 
 struct PairArgs {
     const Item *items;
-    const Range *ranges;         // range records of the multi-range items
+    const PlanSample *ps;        // position columns of every sample
+    const double *bbox;          // bounding boxes of the blocks' shapes
     const unsigned long long *overflow;  // planner's capacity flag
     const Block *blocks;
     const int64_t *n_items;      // device: work items in the list
     int n_waves;
-    const int64_t *bounds;       // schedule unit -> first item, n_waves * kScheduleUnits + 3
+    const int64_t *key_off;      // first item of every key
+    const int64_t *bounds;       // schedule unit -> first item, groups * kScheduleUnits + 3
     int *queue;                  // tail-chunk counter, zero at launch
     int mode, n_r, n_2, weighted, var, nbins;
     const double *T, *X;         // exact thresholds (global copy)
     double T0, Tn, X0, Xn;       // domain bounds (rppi: s and pi; rmu: r^2)
     float lgs, lgc;              // r bin guess: log2(v) * lgs + lgc
-    float xs;                    // mu: (mu + 1) * xs
+    float xs, xc;                // mu: (mu + 1) * xs + xc
     double xs64, xc64;           // pi: pi * xs64 + xc64
-    float dr;                    // guard bands: exact path when |guess - nearest integer| < d
-    float d2;
+    float dr, d2f;               // guard bands: exact path when the fraction of a guess is below
+    double d2;
     int scan;                    // 1: the exact path scans every threshold (guard band of a whole bin)
     const SampleDev *samples;
-    int hist_stride;             // bytes per wave histogram
+    int hist_stride;             // bytes of a histogram
+    int shared, copies;          // the waves of a workgroup share `copies` histograms (else one per wave)
     int bin_off, nbins_out;      // this pass's first output bin (r0 * n_2) and the output's B
-    int copies_log2;             // each bin is kept in 2^copies_log2 interleaved copies
-    int off_sp, off_sx, off_dd, off_var; // byte offsets inside a wave histogram
     unsigned long long *rechecks;
     // wall-clock span of the launch's busy waves: [0] max of ~start, [1] max of end
     unsigned long long *clock;
@@ -964,49 +762,55 @@ struct PairArgs {
     double *slot_sp, *slot_sx, *slot_dd, *slot_var;
 };
 
-// Wave histogram layout (C = 2^copies_log2 interleaved copies of B bins;
-// slot h = bin * C + copy).  Separate arrays keep the FP64 slots 8 bytes
-// apart, so the lanes of one ds_add_f64 spread over all 16 bank pairs.
-//   u32     cnt[B*C]   at 0
-//   double  sp[B*C]    at off_sp    (S+D)
-//   double  sx[B*C]    at off_sx    (SxD)
-//   double  dd[B*C]    at off_dd    (weighted samples)
-//   double  var[B*C]   at off_var   (variance requested)
+// One bin of a wave's histogram.  A pending run keeps its slot's address and
+// the fields lie at constant offsets from it, so a flush computes no
+// addresses.
+template <bool WEIGHTED, bool VAR>
+struct Slot {
+    double sp, sx;                       // S+D, SxD
+    double more[WEIGHTED + VAR];         // DD (weighted samples), sum of e+^2 (variance requested)
+    uint32_t c, pad;
+};
+static_assert(sizeof(Slot<false, false>) == 24 && sizeof(Slot<true, true>) == 40, "Slot layout");
+constexpr size_t slot_bytes(bool weighted, bool var) {
+    return sizeof(Slot<false, false>) + 8 * (size_t)(weighted + var);
+}
 
 // Shape record {a, b, l, ax, ay, e*w, w, 2*e*w} read through the scalar cache:
 // the inner loop is uniform over shapes, so every field lands in SGPRs.
 typedef const __attribute__((address_space(4))) double *ShapePtr;
 
-__device__ void flush_hist(const PairArgs &P, char *hist, const SampleDev &S, int rs, int rp,
-                           int lane) {
-    uint32_t *cnt = (uint32_t *)hist;
-    double *sp = (double *)(hist + P.off_sp);
-    double *sx = (double *)(hist + P.off_sx);
-    double *dd = P.weighted ? (double *)(hist + P.off_dd) : nullptr;
-    double *vr = P.var ? (double *)(hist + P.off_var) : nullptr;
+// One bin of a histogram, summed over its copies and cleared.
+template <bool WEIGHTED, bool VAR>
+__device__ __forceinline__ Slot<WEIGHTED, VAR> take_bin(const PairArgs &P, char *hist, int copies, int b) {
+    typedef Slot<WEIGHTED, VAR> BinSlot;
+    BinSlot t{};
+    for (int k = 0; k < copies; ++k, hist += P.hist_stride) {
+        BinSlot *s = (BinSlot *)hist + b;
+        if (s->c == 0) continue;
+        t.c += s->c;
+        t.sp += s->sp;
+        t.sx += s->sx;
+        if constexpr (WEIGHTED) t.more[0] += s->more[0];
+        if constexpr (VAR) t.more[WEIGHTED ? 1 : 0] += s->more[WEIGHTED ? 1 : 0];
+        *s = BinSlot{};
+    }
+    return t;
+}
+
+template <bool WEIGHTED, bool VAR>
+__device__ void flush_hist(const PairArgs &P, char *hist, int copies, const SampleDev &S, int rs, int rp, int tid,
+                           int nthr) {
+    const bool dd = WEIGHTED, vr = VAR;
     const int B = P.nbins;
     const int BO = P.nbins_out;
-    const int C = 1 << P.copies_log2;
-    for (int b = lane; b < B; b += kWave) {
-        uint32_t c = 0;
-        double vsp = 0.0, vsx = 0.0, vdd = 0.0, vvr = 0.0;
-        for (int k = 0; k < C; ++k) {
-            int h = b * C + k;
-            c += cnt[h];
-            vsp += sp[h];
-            vsx += sx[h];
-            cnt[h] = 0;
-            sp[h] = 0.0;
-            sx[h] = 0.0;
-            if (dd) {
-                vdd += dd[h];
-                dd[h] = 0.0;
-            }
-            if (vr) {
-                vvr += vr[h];
-                vr[h] = 0.0;
-            }
-        }
+    for (int b = tid; b < B; b += nthr) {
+        const Slot<WEIGHTED, VAR> t = take_bin<WEIGHTED, VAR>(P, hist, copies, b);
+        const uint32_t c = t.c;
+        const double vsp = t.sp, vsx = t.sx;
+        double vdd = 0.0, vvr = 0.0;
+        if constexpr (WEIGHTED) vdd = t.more[0];
+        if constexpr (VAR) vvr = t.more[WEIGHTED ? 1 : 0];
         if (c == 0) continue;
         const int gb = b + P.bin_off;  // the pass's local bin in the output grid
         atomicAdd(&S.npairs[gb], (unsigned long long)c);
@@ -1037,42 +841,19 @@ __device__ __forceinline__ int64_t slot_key_of(int sample, int rs, int rp) {
 
 // The deterministic flush: the wave's histogram (every bin of the pass, the
 // empty ones too) is stored into its slot instead of added by atomics.
-__device__ void flush_slot(const PairArgs &P, char *hist, int64_t slot, int64_t key, int lane) {
+template <bool WEIGHTED, bool VAR>
+__device__ void flush_slot(const PairArgs &P, char *hist, int copies, int64_t slot, int64_t key, int tid, int nthr) {
     if (slot >= P.slot_cap) return;  // cannot happen: the slot plan counts every flush
-    uint32_t *cnt = (uint32_t *)hist;
-    double *sp = (double *)(hist + P.off_sp);
-    double *sx = (double *)(hist + P.off_sx);
-    double *dd = P.weighted ? (double *)(hist + P.off_dd) : nullptr;
-    double *vr = P.var ? (double *)(hist + P.off_var) : nullptr;
-    const int C = 1 << P.copies_log2;
-    for (int b = lane; b < P.nbins; b += kWave) {
-        uint32_t c = 0;
-        double vsp = 0.0, vsx = 0.0, vdd = 0.0, vvr = 0.0;
-        for (int k = 0; k < C; ++k) {
-            const int h = b * C + k;
-            c += cnt[h];
-            vsp += sp[h];
-            vsx += sx[h];
-            cnt[h] = 0;
-            sp[h] = 0.0;
-            sx[h] = 0.0;
-            if (dd) {
-                vdd += dd[h];
-                dd[h] = 0.0;
-            }
-            if (vr) {
-                vvr += vr[h];
-                vr[h] = 0.0;
-            }
-        }
+    for (int b = tid; b < P.nbins; b += nthr) {
+        const Slot<WEIGHTED, VAR> t = take_bin<WEIGHTED, VAR>(P, hist, copies, b);
         const int64_t o = slot * P.nbins_out + P.bin_off + b;
-        P.slot_np[o] = c;
-        P.slot_sp[o] = vsp;
-        P.slot_sx[o] = vsx;
-        if (dd) P.slot_dd[o] = vdd;
-        if (vr) P.slot_var[o] = vvr;
+        P.slot_np[o] = t.c;
+        P.slot_sp[o] = t.sp;
+        P.slot_sx[o] = t.sx;
+        if constexpr (WEIGHTED) P.slot_dd[o] = t.more[0];
+        if constexpr (VAR) P.slot_var[o] = t.more[WEIGHTED ? 1 : 0];
     }
-    if (lane == 0) P.slot_key[slot] = key;
+    if (tid == 0) P.slot_key[slot] = key;
 }
 
 
@@ -1139,22 +920,23 @@ enum { SH_NONE = 0, SH_CONST = 1, SH_WRAP = 2 };
 // summed in registers and reach the LDS histogram as one atomic per run,
 // which cuts the same-address collisions of the hot (outer r) bins.
 struct Pend {
-    int b;
+    uint32_t at;  // LDS address of the slot
     uint32_t c;
     double sp, sx, dd, vr;
 };
 
+#define MIA_LDS __attribute__((address_space(3)))
+
 template <bool WEIGHTED, bool VAR>
-__device__ __forceinline__ void hist_add(const PairArgs &P, char *hist, int b, uint32_t c, double sp,
-                                         double sx, double dd, double vr) {
-    uint32_t *cnt = (uint32_t *)hist;
-    atomicAdd(&cnt[b], c);
-    double *hsp = (double *)(hist + P.off_sp);
-    double *hsx = (double *)(hist + P.off_sx);
-    atomicAdd(&hsp[b], sp);
-    atomicAdd(&hsx[b], sx);
-    if (WEIGHTED) atomicAdd(&((double *)(hist + P.off_dd))[b], dd);
-    if (VAR) atomicAdd(&((double *)(hist + P.off_var))[b], vr);
+__device__ __forceinline__ void hist_add(const Pend &p) {
+    typedef MIA_LDS Slot<WEIGHTED, VAR> LdsSlot;
+    LdsSlot *s = (LdsSlot *)p.at;
+    __hip_atomic_fetch_add(&s->c, p.c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(&s->sp, p.sp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(&s->sx, p.sx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if constexpr (WEIGHTED)
+        __hip_atomic_fetch_add(&s->more[0], p.dd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if constexpr (VAR) __hip_atomic_fetch_add(&s->more[WEIGHTED ? 1 : 0], p.vr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 template <int MODE, int SH, bool WEIGHTED, bool VAR, bool LZ>
@@ -1162,8 +944,8 @@ __device__ __forceinline__ void one_pair(const PairArgs &P, const SampleView &S,
                                          double pa, double pb, double pl, double pw, double qa,
                                          double qb, double ql, double qax, double qay, double qew,
                                          double qw, double q2ew, double sha, double shb, double shl,
-                                         char *hist, const double *T, const double *X,
-                                         uint32_t &nre, Pend &pd, float vlgc, double vxc) {
+                                         uint32_t hist, uint32_t row, const double *T, const double *X,
+                                         uint32_t &nre, Pend &pd, float vlgc, float vlg2, double vxs, double vxc) {
     const int n_r = P.n_r, n_2 = P.n_2;
     // the reference's own FP64 separation (measure_w_box_jk.py:159-162)
     double da = qa - pa, db = qb - pb, dl = ql - pl;
@@ -1192,24 +974,30 @@ __device__ __forceinline__ void one_pair(const PairArgs &P, const SampleView &S,
         // within the guard band of a bin edge (every edge, the domain edges
         // included, so no clamping is needed)
         float rv32 = (float)rv;
-        float gr = __fmaf_rn(__log2f(rv32), P.lgs, vlgc);
+        const float gr = __fmaf_rn(__log2f(rv32), P.lgs, vlgc);
+        const bool near_r = __builtin_amdgcn_fractf(gr) < P.dr;
         // pi: an FP64 guess (one FMA; its error is ~1e-14 bins, so a 1e-9 guard
-        // band); mu = pi / r: an FP32 guess from rsqrt
+        // band); mu = pi / r: an FP32 guess from rsqrt.  The constants of the
+        // guesses hold half the guard band, so a guess close to an edge on
+        // either side has a fraction below the whole band
+        int i2;
         double g2;
         bool near2;
         if (MODE == MIA_RPPI) {
-            g2 = fma(dl, P.xs64, vxc);
-            near2 = fabs(g2 - rint(g2)) < P.d2;
+            g2 = fma(dl, vxs, vxc);
+            near2 = __builtin_amdgcn_fract(g2) < P.d2;
+            i2 = (int)g2;
         } else {
-            float g2f = __fmaf_rn((float)dl, __builtin_amdgcn_rsqf(rv32), 1.0f) * P.xs;
-            near2 = fabsf(g2f - rintf(g2f)) < P.d2;
+            const float g2f = __fmaf_rn(__fmaf_rn((float)dl, __builtin_amdgcn_rsqf(rv32), 1.0f), P.xs, vlg2);
+            near2 = __builtin_amdgcn_fractf(g2f) < P.d2f;
+            i2 = (int)g2f;
             g2 = g2f;
         }
         // truncation is floor for the non-negative guesses; a guess within
         // the guard band of an integer (an edge, or a slightly negative
         // guess at the lower domain edge) takes the exact path
-        int ir = (int)gr, i2 = (int)g2;
-        bool near = ((int)(fabsf(gr - rintf(gr)) < P.dr) | (int)near2) != 0;
+        int ir = (int)gr;
+        const bool near = near_r | near2;
         if (near) {
             if (P.scan) {
                 ir = count_edges(T, n_r, rv);
@@ -1256,16 +1044,16 @@ __device__ __forceinline__ void one_pair(const PairArgs &P, const SampleView &S,
             ep = pw * ep;
             ex = pw * ex;
         }
-        int b = __mul24(ir, n_2) + i2;
+        const uint32_t at = __umul24(ir, row) + (__umul24(i2, (uint32_t)sizeof(Slot<WEIGHTED, VAR>)) + hist);
         double dd = WEIGHTED ? pw * qw : 0.0;
         double vr = VAR ? ep * ep : 0.0;
         // a new slot flushes the pending run; the run then restarts from this
         // pair: keep = 0 drops the old sums (fma(0, sum, x) = x, fma(1, sum, x)
         // = sum + x, both exactly as the plain assignment and addition)
-        const bool nw = b != pd.b;
-        if (nw & (pd.b >= 0)) hist_add<WEIGHTED, VAR>(P, hist, pd.b, pd.c, pd.sp, pd.sx, pd.dd, pd.vr);
+        const bool nw = at != pd.at;
+        if (nw) hist_add<WEIGHTED, VAR>(pd);
         const double keep = nw ? 0.0 : 1.0;
-        pd.b = b;
+        pd.at = at;
         pd.c = (nw ? 0u : pd.c) + 1u;
         pd.sp = fma_into(keep, pd.sp, ep);
         pd.sx = fma_into(keep, pd.sx, ex);
@@ -1274,9 +1062,53 @@ __device__ __forceinline__ void one_pair(const PairArgs &P, const SampleView &S,
     }
 }
 
+// An item's np positions lie in the columns of its lanes (lane c: positions
+// [pb, pb + n)); item coordinate k runs over them column by column.  Lane l
+// takes coordinates l * nb .. l * nb + nb - 1, one per batch: a batch then
+// spans all columns and the whole line-of-sight range of the item, and its
+// pairs spread over many (r, pi) bins (64 consecutive positions mostly share a
+// few: with them same-address LDS atomics bound the kernel, 9.9 against 8.6 ms on
+// a million clustered positions, 200,000 shapes).
+struct ColumnWalk {
+    int pb, end;        // own column: first position minus its first coordinate; end coordinate
+    int c, base, ce;    // the column the lane reads from
+    int np, nb;
+
+    __device__ __forceinline__ void begin(int lane, int pb_, int n) {
+        end = n;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const int o = __shfl_up(end, d);
+            end += lane >= d ? o : 0;
+        }
+        pb = pb_ - (end - n);
+        np = __builtin_amdgcn_readlane(end, kWave - 1);
+        nb = (np + kWave - 1) / kWave;
+        // the first column that ends past the lane's first coordinate
+        const int k = lane * nb < np ? lane * nb : np - 1;
+        c = 0;
+#pragma unroll
+        for (int d = kWave / 2; d > 0; d >>= 1) c += __shfl(end, c + d - 1) <= k ? d : 0;
+        base = __shfl(pb, c);
+        ce = __shfl(end, c);
+    }
+    // the lane's position of batch bt (a lane past the end gets a valid one)
+    __device__ __forceinline__ int position(int bt, int lane, bool &v) {
+        int k = bt + lane * nb;
+        v = k < np;
+        k = v ? k : np - 1;
+        while (__any(k >= ce)) {  // every lane takes part: a shuffle reads active lanes only
+            c += k >= ce ? 1 : 0;
+            base = __shfl(pb, c);
+            ce = __shfl(end, c);
+        }
+        return base + k;
+    }
+};
+
 template <int MODE, int SH, bool WEIGHTED, bool VAR, bool LZ>
-__device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S, int p0, int np, int nr,
-                                         int shifts, ShapePtr shp, int ns, char *hist,
+__device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S, int cpb, int cn,
+                                         int shifts, ShapePtr shp, int ns, uint32_t hist,
                                          const double *T, const double *X, int lane,
                                          uint32_t &nre, uint64_t &iterations) {
     const double L = S.L;
@@ -1286,56 +1118,31 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
     // the additive constants of the FP32 bin guesses, held in VGPRs for the
     // whole item (a VOP3 FMA reads one scalar operand; the other would be
     // copied into a VGPR on every pair)
-    float vlgc;
-    double vxc;
+    float vlgc, vlg2 = 0.0f;
+    double vxs = 0.0, vxc = 0.0;
     asm volatile("v_mov_b32 %0, %1" : "=v"(vlgc) : "s"(P.lgc));
-    asm volatile("v_mov_b64 %0, %1" : "=v"(vxc) : "s"(P.xc64));
-    // Strided lane -> position map: lane l of batch b takes position b + l*nb,
-    // so one batch spans the whole line-of-sight range of the item and its
-    // pairs spread over more (r, pi) bins (fewer same-address LDS atomics).
-    const int nb = (np + kWave - 1) / kWave;
-    iterations += (uint64_t)nb * ns;
-    // The lane's current range: item coordinate k < ce is position cb + k.
-    // Lane l walks k = l*nb .. l*nb + nb - 1, so it starts in the range
-    // holding l*nb (found from the item's range records, scalar loads live
-    // only here) and steps to the next record when k reaches ce.
-    int cb = p0, ce = np, ci = 0;
-    const int2 *rg = (const int2 *)(P.ranges + (nr > 1 ? p0 : 0));
-    if (nr > 1) {
-        const MIA_CONST int32_t *rr = (const MIA_CONST int32_t *)rg;
-        const int kf = lane * nb < np ? lane * nb : np - 1;
-        cb = rr[0];
-        ce = rr[1];
-#pragma unroll
-        for (int i = 1; i < kItemRanges; ++i)
-            if (i < nr && kf >= rr[2 * i - 1]) {
-                ci = i;
-                cb = rr[2 * i];
-                ce = rr[2 * i + 1];
-            }
+    if (MODE == MIA_RPPI) {
+        asm volatile("v_mov_b64 %0, %1" : "=v"(vxs) : "s"(P.xs64));
+        asm volatile("v_mov_b64 %0, %1" : "=v"(vxc) : "s"(P.xc64));
+    } else {
+        asm volatile("v_mov_b32 %0, %1" : "=v"(vlg2) : "s"(P.xc));
     }
-    // the lane's position of batch bt (a lane past the item's end reads a
-    // valid position, its range's last)
-    auto position = [&](int bt, bool &v) {
-        const int k = bt + lane * nb;
-        v = k < np;
-        while (v && k >= ce) {
-            const int2 r = rg[++ci];
-            cb = r.x;
-            ce = r.y;
-        }
-        return (const double2 *)(S.prec + 4 * (int64_t)(cb + (v ? k : ce - 1)));
-    };
-    Pend pd{-1, 0, 0, 0, 0, 0};
+    ColumnWalk walk;
+    walk.begin(lane, cpb, cn);
+    const int nb = walk.nb;
+    iterations += (uint64_t)nb * ns;
+    // the slot past the last bin takes the zeros of the empty run
+    const uint32_t row = (uint32_t)(P.n_2 * sizeof(Slot<WEIGHTED, VAR>));
+    Pend pd{hist + (uint32_t)(P.nbins * sizeof(Slot<WEIGHTED, VAR>)), 0, 0, 0, 0, 0};
     // positions are loaded one batch ahead
     bool vn;
-    const double2 *prn = position(0, vn);
+    const double2 *prn = (const double2 *)(S.prec + 4 * (int64_t)walk.position(0, lane, vn));
     double2 abn = prn[0], lwn = prn[1];
     for (int bt = 0; bt < nb; ++bt) {
         const bool v0 = vn;
         const double2 ab = abn, lw = lwn;
         if (bt + 1 < nb) {
-            prn = position(bt + 1, vn);
+            prn = (const double2 *)(S.prec + 4 * (int64_t)walk.position(bt + 1, lane, vn));
             abn = prn[0];
             lwn = prn[1];
         }
@@ -1355,12 +1162,12 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
             const double b0 = r1[0], b1 = r1[1], b2 = r1[2], b3 = r1[3], b4 = r1[4], b5 = r1[5],
                          b6 = r1[6], b7 = r1[7];
             one_pair<MODE, SH, WEIGHTED, VAR, LZ>(P, S, v0, pa0, pb0, pl0, pw0, qa, qb, ql, qax, qay, qew, qw,
-                                         q2ew, sha, shb, shl, hist, T, X, nre, pd, vlgc, vxc);
+                                         q2ew, sha, shb, shl, hist, row, T, X, nre, pd, vlgc, vlg2, vxs, vxc);
             ShapePtr r2 = (ShapePtr)((const MIA_CONST char *)shp + (o + 128u < olast ? o + 128u : olast));
             const double c0 = r2[0], c1 = r2[1], c2 = r2[2], c3 = r2[3], c4 = r2[4], c5 = r2[5],
                          c6 = r2[6], c7 = r2[7];
             one_pair<MODE, SH, WEIGHTED, VAR, LZ>(P, S, v0, pa0, pb0, pl0, pw0, b0, b1, b2, b3, b4, b5, b6,
-                                         b7, sha, shb, shl, hist, T, X, nre, pd, vlgc, vxc);
+                                         b7, sha, shb, shl, hist, row, T, X, nre, pd, vlgc, vlg2, vxs, vxc);
             qa = c0;
             qb = c1;
             ql = c2;
@@ -1372,106 +1179,174 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
         }
         if (j < ns)
             one_pair<MODE, SH, WEIGHTED, VAR, LZ>(P, S, v0, pa0, pb0, pl0, pw0, qa, qb, ql, qax, qay, qew, qw,
-                                         q2ew, sha, shb, shl, hist, T, X, nre, pd, vlgc, vxc);
+                                         q2ew, sha, shb, shl, hist, row, T, X, nre, pd, vlgc, vlg2, vxs, vxc);
     }
-    if (pd.b >= 0) hist_add<WEIGHTED, VAR>(P, hist, pd.b, pd.c, pd.sp, pd.sx, pd.dd, pd.vr);
+    hist_add<WEIGHTED, VAR>(pd);
 }
 
 // An item's pair loop for its periodic-shift variant.
 template <int MODE, bool WEIGHTED, bool VAR, bool LZ>
-__device__ __forceinline__ void run_shifted(const PairArgs &P, const SampleView &S, int p0, int np, int nr,
-                                            int shifts, ShapePtr shp, int ns, char *hist, const double *T,
+__device__ __forceinline__ void run_shifted(const PairArgs &P, const SampleView &S, int cpb, int cn,
+                                            int shifts, ShapePtr shp, int ns, uint32_t hist, const double *T,
                                             const double *X, int lane, uint32_t &nre, uint64_t &iterations) {
     if (shifts & 64)
-        run_item<MODE, SH_WRAP, WEIGHTED, VAR, LZ>(P, S, p0, np, nr, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_WRAP, WEIGHTED, VAR, LZ>(P, S, cpb, cn, shifts, shp, ns, hist, T, X, lane, nre,
                                                    iterations);
     else if (shifts & 63)
-        run_item<MODE, SH_CONST, WEIGHTED, VAR, LZ>(P, S, p0, np, nr, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_CONST, WEIGHTED, VAR, LZ>(P, S, cpb, cn, shifts, shp, ns, hist, T, X, lane, nre,
                                                     iterations);
     else
-        run_item<MODE, SH_NONE, WEIGHTED, VAR, LZ>(P, S, p0, np, nr, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_NONE, WEIGHTED, VAR, LZ>(P, S, cpb, cn, shifts, shp, ns, hist, T, X, lane, nre,
                                                    iterations);
 }
 
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// Persistent groups of waves over the cost-balanced, key-sorted items.  A group
+// works on the items of one key at a time and adds into its histogram, which
+// goes to the key's sums when the key changes.  A group is one wave; or, where
+// private histograms would leave too few waves per CU (P.shared), the four
+// waves of a workgroup, which take a key's items from a counter in LDS and
+// share P.copies copies of one histogram, a lane adding into the copy of its
+// place (so neighbouring lanes, which often hit one bin, hit different
+// addresses).
 template <int MODE, bool WEIGHTED, bool VAR>
-__global__ __launch_bounds__(kThreads) void k_pairs(PairArgs P) {
+__global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs P) {
     extern __shared__ __align__(16) char lds[];
+    __shared__ int s_next[2], s_chunk;
     const int lane = threadIdx.x & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    // exact thresholds for the rare FP64 bin path (shared by the block's waves)
+    const bool shared = P.shared != 0;
+    // exact thresholds for the rare FP64 bin path
     double *T = (double *)lds;
     double *X = T + (P.n_r + 1);
     int nx = P.n_2 + 1;
     for (int i = threadIdx.x; i < P.n_r + 1; i += blockDim.x) T[i] = P.T[i];
     for (int i = threadIdx.x; i < nx; i += blockDim.x) X[i] = P.X[i];
     size_t thr_bytes = ((size_t)(P.n_r + 1 + nx) * 8 + 15) & ~(size_t)15;
-    char *hist = lds + thr_bytes + (size_t)wv * P.hist_stride;
-    for (int i = lane * 4; i < P.hist_stride; i += kWave * 4) *(uint32_t *)(hist + i) = 0u;
+    typedef Slot<WEIGHTED, VAR> BinSlot;
+    char *hist0 = lds + thr_bytes;
+    const int nhist = shared ? P.copies : (int)(blockDim.x / kWave);
+    for (int i = threadIdx.x * 4; i < nhist * P.hist_stride; i += blockDim.x * 4) *(uint32_t *)(hist0 + i) = 0u;
+    if (threadIdx.x < 2) s_next[threadIdx.x] = 0;
     __syncthreads();
 
     // runs of neighbouring items of the key-sorted list (which read the same
     // position cells) stay on one XCD
-    const int w = xcd_run_block() * (blockDim.x / kWave) + wv;
+    const int wpb = blockDim.x / kWave, wg = xcd_run_block();
     const int64_t n_items = *(const MIA_CONST int64_t *)P.n_items;
+    const int wave = wg * wpb + wv;
     // a plan that overflowed its capacities is counted again by the host
-    if (w >= P.n_waves || n_items == 0 || *(const MIA_CONST unsigned long long *)P.overflow) return;
+    if (n_items == 0 || *(const MIA_CONST unsigned long long *)P.overflow) return;
+    if (!shared && wave >= P.n_waves) return;
     if (lane == 0) atomicMax(&P.clock[0], ~(unsigned long long)wall_clock64());
+    const int tid = shared ? threadIdx.x : lane, nthr = shared ? blockDim.x : kWave;
+    char *hist = hist0 + (shared ? 0 : wv * P.hist_stride);
+    const int place = ((lane & 7) << 3) | (lane >> 3);
+    const uint32_t hist_at = (uint32_t)(uintptr_t)(MIA_LDS char *)(hist + (shared ? place % P.copies : 0) * P.hist_stride);
     // a contiguous share of the cost-sorted items, then tail chunks from the counter
-    const WaveSchedule sch = make_schedule(P.bounds, P.n_waves);
+    const WaveSchedule sch = make_schedule(P.bounds, shared ? (int)gridDim.x : P.n_waves);
     int64_t it0, it1;
-    sch.first(w, it0, it1);
+    sch.first(shared ? wg : wave, it0, it1);
     const MIA_CONST int32_t *items = (const MIA_CONST int32_t *)P.items;
     const MIA_CONST int32_t *blocks = (const MIA_CONST int32_t *)P.blocks;
-    int cur_key_s = -1, cur_rs = -1, cur_rp = -1;
-    const SampleDev *Sp = nullptr;
-    SampleView S{};
-    int64_t slot = P.det ? P.slot0[w] : 0;
+    int cur_key = -1, flushes = 0, par = 0;
     uint32_t nre = 0;
     uint64_t iterations = 0;  // wave-uniform
-    do {
-        for (int64_t i = it0; i < it1; ++i) {
-            const MIA_CONST int32_t *ip = items + 4 * i;
-            const int blk = ip[0], p0 = ip[1], np = ip[2], w3 = ip[3];
-            const int rp = (int16_t)(w3 & 0xffff);
-            const int shifts = (w3 >> 16) & 0xff;
-            const int nr = (w3 >> 24) & 0xff;
-            const MIA_CONST int32_t *bp = blocks + 6 * (int64_t)blk;
-            const int s0 = bp[0], ns = bp[1], sample = bp[4], rs = bp[5];
-            if (sample != cur_key_s || rs != cur_rs || rp != cur_rp) {
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                if (Sp) {
-                    if (P.det)
-                        flush_slot(P, hist, slot++, slot_key_of(cur_key_s, cur_rs, cur_rp), lane);
-                    else
-                        flush_hist(P, hist, *Sp, cur_rs, cur_rp, lane);
-                }
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                if (sample != cur_key_s) {
-                    Sp = &P.samples[sample];
-                    S = load_view(Sp);
-                }
-                cur_key_s = sample;
-                cur_rs = rs;
-                cur_rp = rp;
-            }
-            ShapePtr shp = (ShapePtr)(S.srec + 8 * (int64_t)s0);
-            // (r, mu) sums r^2 in an order fixed by the line of sight: one
-            // loop per order, so the pair loop holds no branch on it
-            if (MODE == MIA_RMU && S.los != 2)
-                run_shifted<MODE, WEIGHTED, VAR, false>(P, S, p0, np, nr, shifts, shp, ns, hist, T, X, lane, nre,
-                                                        iterations);
-            else
-                run_shifted<MODE, WEIGHTED, VAR, true>(P, S, p0, np, nr, shifts, shp, ns, hist, T, X, lane, nre,
-                                                       iterations);
-        }
-    } while (sch.next(P.queue, lane, it0, it1));
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    if (Sp) {
-        if (P.det)
-            flush_slot(P, hist, slot, slot_key_of(cur_key_s, cur_rs, cur_rp), lane);
+
+    auto sync = [&]() {
+        if (shared)
+            __syncthreads();
         else
-            flush_hist(P, hist, *Sp, cur_rs, cur_rp, lane);
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    };
+    // the histogram goes to its key's sums, the next adds are for `key` (every
+    // thread of the group, with no adds in flight)
+    auto turn_to = [&](int key) {
+        if (cur_key >= 0) {
+            sync();
+            const int kk = P.K1 * P.K1;
+            const int sample = cur_key / kk, in = cur_key - sample * kk;
+            const int rs = in / P.K1, rp = in - rs * P.K1;
+            const int n = shared ? P.copies : 1;
+            if (P.det)
+                flush_slot<WEIGHTED, VAR>(P, hist, n, P.slot0[wave] + flushes++, slot_key_of(sample, rs, rp), tid, nthr);
+            else
+                flush_hist<WEIGHTED, VAR>(P, hist, n, P.samples[sample], rs, rp, tid, nthr);
+            sync();
+        }
+        cur_key = key;
+    };
+
+    while (true) {
+        for (int64_t it = it0; it < it1;) {
+            // the items [it, se) of one key
+            const int key = __builtin_amdgcn_readfirstlane(items[8 * it + 7]);
+            const int64_t ke = ((const MIA_CONST int64_t *)P.key_off)[key + 1];
+            const int64_t se = uniform64(ke < it1 ? ke : it1);
+            if (key != cur_key) turn_to(key);
+            int64_t i = it;
+            while (true) {
+                if (shared) {
+                    int t = 0;
+                    if (lane == 0) t = wave < P.n_waves ? atomicAdd(&s_next[par], 1) : 0x7fffffff;
+                    i = it + __builtin_amdgcn_readfirstlane(t);
+                }
+                // (the compiler does not see that i is wave-uniform; vector
+                // loads of the shape records would cost 70 registers)
+                i = uniform64(i);
+                if (i >= se) break;
+                const MIA_CONST int32_t *ip = items + 8 * i;
+                ++i;
+                if (ip[6] == 0) continue;  // no column of the item is in reach
+                const int blk = ip[0], w = ip[1], jj = ip[2], wn = ip[3], c0 = ip[4], kk = ip[5];
+                const int shifts = (w >> 16) & 0xff;
+                const MIA_CONST int32_t *bp = blocks + 6 * (int64_t)blk;
+                const int s0 = bp[0], ns = bp[1], sample = bp[4];
+                const SampleView S = load_view(P.samples + sample);
+                ShapePtr shp = (ShapePtr)(S.srec + 8 * (int64_t)s0);
+                int cpb, cn;
+                {
+                    const MIA_CONST double *bc = (const MIA_CONST double *)P.bbox + 6 * (int64_t)blk;
+                    const double bb[6] = {bc[0], bc[1], bc[2], bc[3], bc[4], bc[5]};
+                    item_column(column_view((const MIA_CONST PlanSample *)P.ps + sample), bb, jj & 0xffff,
+                                (jj >> 16) & 0xffff, wn & 0xffff, (wn >> 16) & 0xffff, c0, kk & 0xffff,
+                                (kk >> 16) & 0xffff, (w >> 24) & 3, lane, cpb, cn);
+                }
+                // (r, mu) sums r^2 in an order fixed by the line of sight: one
+                // loop per order, so the pair loop holds no branch on it
+                if (MODE == MIA_RMU && S.los != 2)
+                    run_shifted<MODE, WEIGHTED, VAR, false>(P, S, cpb, cn, shifts, shp, ns, hist_at, T, X, lane, nre,
+                                                            iterations);
+                else
+                    run_shifted<MODE, WEIGHTED, VAR, true>(P, S, cpb, cn, shifts, shp, ns, hist_at, T, X, lane, nre,
+                                                           iterations);
+            }
+            if (shared) {
+                __syncthreads();
+                // (the other counter serves the next key, and a barrier lies
+                // between this reset and this counter's next use)
+                if (threadIdx.x == 0) s_next[par] = 0;
+                par ^= 1;
+            }
+            it = se;
+        }
+        if (!shared) {
+            if (!sch.next(P.queue, lane, it0, it1)) break;
+        } else {
+            if (sch.tail == 0) break;
+            if (threadIdx.x == 0) s_chunk = atomicAdd(P.queue, 1);
+            __syncthreads();
+            const int k = __builtin_amdgcn_readfirstlane(s_chunk);
+            __syncthreads();
+            if (!sch.chunk(k, it0, it1)) break;
+        }
     }
+    turn_to(-1);
     if (nre) atomicAdd(P.rechecks, (unsigned long long)nre);
     if (lane == 0) {
         if (iterations) atomicAdd(P.iterations, (unsigned long long)iterations);
@@ -1502,10 +1377,7 @@ void launch_pairs_mode(const PairArgs &A, unsigned grid, int wpb, size_t lds, hi
 
 // LDS bytes of one wave's histogram (one copy) and of the block's thresholds.
 size_t wave_hist_bytes(const mia_bins &bins, bool weighted) {
-    const size_t B = (size_t)bins.n_r * bins.n_2;
-    size_t off = (4 * B + 15) & ~(size_t)15;
-    off += 16 * B + (weighted ? 8 * B : 0) + (bins.accumulate_variance ? 8 * B : 0);
-    return (off + 15) & ~(size_t)15;
+    return (((size_t)bins.n_r * bins.n_2 + 1) * slot_bytes(weighted, bins.accumulate_variance) + 15) & ~(size_t)15;
 }
 
 size_t threshold_bytes(const mia_bins &bins) {
@@ -1518,15 +1390,47 @@ inline unsigned nblk(int64_t n, int t) { return (unsigned)((n + t - 1) / t < 1 ?
 // bands, passes over r-bin ranges, histogram copies and offsets, waves.
 struct PairConfig {
     PairArgs A{};        // pointers unset
-    int nrp = 0, npass = 0, wpb = 0, waves = 0;
+    int nrp = 0, npass = 0, wpb = 0, waves = 0, groups = 0;
     unsigned grid = 0;
     size_t lds = 0;
-    double l0 = 0, lgs = 0;
+    double l0 = 0, lgs = 0, shift_r = 0;
 };
 
-PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia_tuning *tuning, int cu_count) {
+// The pair kernel of a count.
+const void *pair_kernel(int mode, bool weighted, bool var) {
+#define MIA_PICK(M) \
+    (weighted ? (var ? (const void *)k_pairs<M, true, true> : (const void *)k_pairs<M, true, false>) \
+              : (var ? (const void *)k_pairs<M, false, true> : (const void *)k_pairs<M, false, false>))
+    return mode == MIA_RPPI ? MIA_PICK(MIA_RPPI) : MIA_PICK(MIA_RMU);
+#undef MIA_PICK
+}
+
+// Workgroups of that kernel a CU holds at once (registers and LDS).
+int resident_workgroups(int mode, bool weighted, bool var, int wpb, size_t lds) {
+    int n = 0;
+    MIA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pair_kernel(mode, weighted, var), kWave * wpb, lds));
+    return std::max(1, n);
+}
+
+// Waves per CU whose histograms (hs bytes) and thresholds LDS holds, with a
+// histogram per wave (workgroups of 4, 2 or 1 waves) or per workgroup of 4.
+int private_waves(size_t thr_bytes, size_t hs) {
+    int w = kMaxWavesPerBlock;
+    while (w > 1 && thr_bytes + hs * w + kPairStaticLds > kLdsBytes) w /= 2;
+    const size_t l = thr_bytes + hs * w + kPairStaticLds;
+    return l > kLdsBytes ? 0 : (int)std::min<size_t>(32 / w, kLdsBytes / l) * w;
+}
+int shared_waves(size_t thr_bytes, size_t hs) {
+    const size_t l = thr_bytes + hs + kPairStaticLds;
+    return l > kLdsBytes ? 0 : (int)std::min<size_t>(32 / kMaxWavesPerBlock, kLdsBytes / l) * kMaxWavesPerBlock;
+}
+
+// candidates: expected (shape, position) pairs of the count.
+PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia_tuning *tuning, int cu_count,
+                       double candidates) {
     PairConfig C;
     PairArgs &A = C.A;
+    const bool det = tuning && tuning->deterministic != 0;
     const int n_r = bins.n_r, n_2 = bins.n_2, B = n_r * n_2;
     A.mode = bins.mode;
     A.n_r = n_r;
@@ -1545,7 +1449,6 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     C.l0 = l0;
     C.lgs = lgs;
     A.lgs = (float)lgs;
-    A.lgc = (float)(-l0 * lgs);
     const double u = std::ldexp(1.0, -23);  // FP32 ulp of 1
     // (+ 2u n_r for a pass's shifted constant -l0 lgs - r0)
     double err_r = (4 * u * std::fmax(std::fabs(l0), std::fabs(ln)) + 4 * u) * lgs + 4 * u * n_r;
@@ -1573,8 +1476,15 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     double dr = std::fmax(1e-4, 20 * err_r);
     // pathological binnings (guard band > 5% of a bin): every pair takes the exact path
     bool exact_only = dr > 0.05 || d2 > 0.05;
-    A.dr = exact_only ? 1.0f : (float)dr;
-    A.d2 = exact_only ? 1.0f : (float)d2;
+    // the guesses are raised by the half width d, and an edge within d of one
+    // then leaves it a fraction below 2 d
+    A.dr = exact_only ? 2.0f : (float)(2.0 * dr);
+    A.d2 = exact_only ? 2.0 : 2.0 * d2;
+    A.d2f = (float)A.d2;
+    C.shift_r = exact_only ? 0.0 : dr;
+    const double shift_2 = exact_only ? 0.0 : d2;
+    A.xc64 += shift_2;
+    A.xc = (float)shift_2;
     A.scan = exact_only ? 1 : 0;
     // Passes over r-bin ranges.  Pass [r0, r0 + nrp) takes the pairs with
     // T[r0] <= r^2 < T[r0 + nrp] (exact FP64 comparisons, so every pair lands
@@ -1593,11 +1503,8 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
         auto waves_per_cu = [&](int nr_) {
             part.n_r = nr_;
             const size_t hs = wave_hist_bytes(part, any_w);
-            int w = kMaxWavesPerBlock;  // as the launch below: 4, 2 or 1 waves per workgroup
-            while (w > 1 && thr_bytes + hs * w > kLdsBytes) w /= 2;
-            const size_t l = thr_bytes + hs * w;
-            if (l > kLdsBytes) return 0;
-            return (int)std::min<size_t>(32 / w, kLdsBytes / l) * w;
+            const int w = private_waves(thr_bytes, hs);
+            return det ? w : std::max(w, shared_waves(thr_bytes, hs));
         };
         if (tuning && tuning->r_bins_per_pass > 0) {
             // as asked, but no more than one wave's histogram can hold
@@ -1630,33 +1537,49 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     // one histogram copy per wave: the pending-slot registers already absorb
     // most same-address collisions, and one copy leaves LDS for 8 waves per
     // SIMD (2 copies measured 20 % slower); mia_tuning.hist_copies is ignored
-    const int copies_log2 = 0;
-    A.copies_log2 = copies_log2;
-    const int BC = Bp << copies_log2;
-    int off = 4 * BC;
-    off = (off + 15) & ~15;
-    A.off_sp = off;
-    off += 8 * BC;
-    A.off_sx = off;
-    off += 8 * BC;
-    A.off_dd = off;
-    if (A.weighted) off += 8 * BC;
-    A.off_var = off;
-    if (A.var) off += 8 * BC;
-    A.hist_stride = (off + 15) & ~15;
-    // waves per block: 4, or fewer when the histograms of 4 waves do not fit
+    // (and the slot an empty pending run adds its zeros to)
+    A.hist_stride = (int)((((size_t)Bp + 1) * slot_bytes(A.weighted, A.var) + 15) & ~(size_t)15);
+    // A private histogram per wave (one copy: the pending-slot registers already
+    // absorb most same-address collisions), or one per workgroup, shared by its
+    // four waves, in as many copies (at most 4) as leave room for
+    // kPairWavesPerSimd waves per SIMD.  Sharing keeps the SIMDs full where
+    // private histograms leave LDS for few waves (600 bins: 2 waves per SIMD
+    // private, 7 shared; 3,000,000 positions to 100 Mpc/h 317 against 201 ms),
+    // but a group of four waits for its slowest wave wherever the key or the
+    // chunk changes (200 bins, 28 private waves per CU, 1,000,000 positions: 8.5
+    // against 11.7 ms).  So it is taken below kSharedBelow private waves per CU,
+    // and where the registers allow more waves than LDS while the launch is too
+    // small for tail chunks (317,811 weighted positions with variances, 20
+    // private waves: 2.65 against 1.9 ms) or so large that its chunks hold many
+    // items (2,000,000 positions, 300 bins: 205 against 200 ms; but twelve
+    // samples of 10,000 to 800,000, 24 private waves: 21 against 31 ms).  Never where the reduction is
+    // deterministic, since a shared histogram's sums depend on timing.
+    // mia_tuning.hist_copies is ignored.
     int wpb = kMaxWavesPerBlock;
-    while (wpb > 1 && thr_bytes + (size_t)A.hist_stride * wpb > kLdsBytes) wpb /= 2;
-    C.lds = thr_bytes + (size_t)A.hist_stride * wpb;
-    if (C.lds > kLdsBytes)
+    const size_t hs = A.hist_stride;
+    const int pw = private_waves(thr_bytes, hs), most = std::min(4 * kPairWavesPerSimd, shared_waves(thr_bytes, hs));
+    const bool small = candidates < kTailMinCost * pw * cu_count;
+    const bool large = candidates > 10 * kTailMinCost * pw * cu_count;
+    A.shared = !det && pw < most && (pw < kSharedBelow || small || large);
+    if (A.shared) {
+        const size_t share = kLdsBytes / kPairWavesPerSimd - kPairStaticLds;
+        A.copies = share > thr_bytes + hs ? (int)std::min<size_t>(4, (share - thr_bytes) / hs) : 1;
+        C.lds = thr_bytes + hs * A.copies;
+    } else {
+        while (wpb > 1 && thr_bytes + hs * wpb + kPairStaticLds > kLdsBytes) wpb /= 2;
+        A.copies = 1;
+        C.lds = thr_bytes + hs * wpb;
+    }
+    if (C.lds + kPairStaticLds > kLdsBytes)
         throw Error{MIA_E_UNSUPPORTED, "histogram too large for LDS (n_r*n_2 too big for MIA_FAST)"};
     C.wpb = wpb;
-    // at most 8 waves per SIMD (32 per CU)
-    int blocks_per_cu = (int)std::max<size_t>(1, std::min<size_t>(32 / wpb, kLdsBytes / C.lds));
+    // as many workgroups as are resident at once
+    const int blocks_per_cu = resident_workgroups(bins.mode, any_w, any_var, wpb, C.lds);
     int waves = tuning && tuning->waves > 0 ? std::min(tuning->waves, kMaxWaves) : cu_count * blocks_per_cu * wpb;
     C.waves = std::max(1, waves);
     A.n_waves = C.waves;
     C.grid = (unsigned)((C.waves + wpb - 1) / wpb);
+    C.groups = A.shared ? (int)C.grid : C.waves;
     return C;
 }
 
@@ -1668,7 +1591,7 @@ bool fast_path_fits(const mia_bins &bins, bool weighted, int jk) {
     // larger binnings run in passes over r-bin ranges: one r row must fit
     mia_bins row = bins;
     row.n_r = 1;
-    return threshold_bytes(bins) + wave_hist_bytes(row, weighted) <= kLdsBytes;
+    return threshold_bytes(bins) + wave_hist_bytes(row, weighted) + kPairStaticLds <= kLdsBytes;
 }
 
 // Sets the dynamic-LDS limit of every pair-kernel variant (once per process).
@@ -1679,13 +1602,9 @@ void pair_kernels_init() {
     MIA_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(mu);
     if (dev < 64 && (done >> dev & 1)) return;
-    const void *fns[] = {
-        (const void *)k_pairs<MIA_RPPI, false, false>, (const void *)k_pairs<MIA_RPPI, false, true>,
-        (const void *)k_pairs<MIA_RPPI, true, false>,  (const void *)k_pairs<MIA_RPPI, true, true>,
-        (const void *)k_pairs<MIA_RMU, false, false>,  (const void *)k_pairs<MIA_RMU, false, true>,
-        (const void *)k_pairs<MIA_RMU, true, false>,   (const void *)k_pairs<MIA_RMU, true, true>};
-    for (const void *f : fns)
-        MIA_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
+    for (int i = 0; i < 8; ++i)
+        MIA_HIP(hipFuncSetAttribute(pair_kernel(i & 4 ? MIA_RMU : MIA_RPPI, i & 2, i & 1),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kLdsBytes - kPairStaticLds)));
     if (dev < 64) done |= 1ull << dev;
 }
 
@@ -1694,8 +1613,8 @@ void pair_kernels_init() {
 
 struct CountPlan {
     int S = 0;
-    int K1 = 1, plan_local = 0, bsz = kMaxBlockShapes;
-    int64_t ncells = 0, nthreads = 0, nthreads_r = 0, nkeys = 0, fin_total = 0, item_cap = 0, range_cap = 0;
+    int K1 = 1, kseg = 0, bsz = kMaxBlockShapes;
+    int64_t ncells = 0, nblk_cap = 0, nkeys = 0, fin_total = 0, item_cap = 0;
     int64_t acc_total = 0;           // accumulator words (u64 / f64) of all samples
     double margin = 0;               // largest geometric slack of the samples' grids
     PairConfig pc;
@@ -1706,14 +1625,13 @@ struct CountPlan {
     std::vector<PlanSample> ps;
     std::vector<SampleDev> sd;
     std::vector<FinSample> fs;
-    std::vector<int64_t> cell0, t0, t0r, fin0;
+    std::vector<int64_t> cell0, fin0;
     std::vector<int64_t> acc0;       // first accumulator word of each sample
     std::vector<int> Bs;             // per sample: K
     // bound workspace
     char *param_dev = nullptr;
     std::vector<char> param;         // host image of the parameter block
-    size_t off_T = 0, off_X = 0, off_cell0 = 0, off_t0 = 0, off_t0r = 0, off_fin0 = 0, off_ps = 0, off_sd = 0,
-           off_fs = 0;
+    size_t off_T = 0, off_X = 0, off_cell0 = 0, off_fin0 = 0, off_ps = 0, off_sd = 0, off_fs = 0;
     size_t param_bytes = 0;
     unsigned long long *zero_begin = nullptr;
     size_t zero_words = 0;
@@ -1722,12 +1640,9 @@ struct CountPlan {
     unsigned long long *kc = nullptr, *kcur = nullptr;
     int64_t *ko = nullptr;
     Item *items = nullptr;
-    Range *ranges = nullptr;
-    RawRange *raw = nullptr;
-    int32_t *roff = nullptr, *rcnt = nullptr;
     int64_t *cost = nullptr, *cpre = nullptr, *n_items = nullptr, *bounds = nullptr;
     double *bbox = nullptr;
-    int32_t *bruns = nullptr;
+    uint32_t *geo = nullptr;
     unsigned long long *words = nullptr;   // [kCountReadback] read back after the count
     int *queue = nullptr;
     unsigned long long *acc = nullptr;
@@ -1751,7 +1666,6 @@ int count_bsz(const CountPlan &p) { return p.bsz; }
 bool count_det(const CountPlan &p) { return p.det; }
 int count_G(const CountPlan &p, int s) { return p.G[s]; }
 int64_t count_item_cap(const CountPlan &p) { return p.item_cap; }
-int64_t count_range_cap(const CountPlan &p) { return p.range_cap; }
 std::string count_key(const CountPlan &p) { return p.key; }
 size_t count_param_bytes(const CountPlan &p) { return p.param_bytes; }
 const void *count_param_image(const CountPlan &p) { return p.param.data(); }
@@ -1759,13 +1673,26 @@ void *count_param_dev(const CountPlan &p) { return p.param_dev; }
 const unsigned long long *count_readback(const CountPlan &p) { return p.words; }
 void free_plan(CountPlan *p) { delete p; }
 
-// Expected work items and multi-range records of a sample (mia_grid.hip's
-// uniform-density model).
-double estimate_items(const Grid &g, int G, double reach_r, double reach_z, bool rmu, int64_t ns, int64_t np,
-                      int pmax, double *ranges);
+// Expected work items of a sample (mia_grid.hip's uniform-density model).
+double estimate_items(const Grid &g, int G, int cpi, double reach_r, double reach_z, bool rmu, int64_t ns, int64_t np,
+                      int64_t blk_cap);
+
+// Deterministic item sort key: planner key, then block and rectangle (the low
+// det_low_bits bits).
+int det_low_bits(const CountPlan &p) {
+    const int64_t n = p.nblk_cap * (kMaxSegs * kMaxSegs * (kMaxSegs + 1));
+    int b = 1;
+    while (b < 62 && ((int64_t)1 << b) < n) ++b;
+    return b;
+}
+int det_key_bits(const CountPlan &p) {
+    int b = 1;
+    while (b < 31 && ((int64_t)1 << b) < p.nkeys + 1) ++b;
+    return det_low_bits(p) + b;
+}
 
 CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_bins &bins,
-                      const mia_tuning *tuning, int64_t item_cap, int64_t range_cap, bool cap_exact) {
+                      const mia_tuning *tuning, int64_t item_cap, bool cap_exact) {
     pair_kernels_init();
     std::unique_ptr<CountPlan> P(new CountPlan());
     CountPlan &p = *P;
@@ -1783,10 +1710,18 @@ CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_b
     p.X.assign(n_2 + 1, 3.0);
     for (int i = 0; i < nx2; ++i) p.X[i] = bins.x2_edges[i];
     p.bsz = tuning && tuning->block_shapes > 0 ? std::min(tuning->block_shapes, kMaxBlockShapes) : kMaxBlockShapes;
-    const int pmax_set = tuning && tuning->item_positions > 0 ? tuning->item_positions : 0;
     p.any_var = bins.accumulate_variance != 0;
     for (const auto &x : ss) p.any_w = p.any_w || x.weighted;
-    p.pc = pair_config(bins, p.any_w, p.any_var, tuning, ctx.cu_count);
+    // (shape, position) pairs within reach at the mean densities, half as many
+    // again for the blocks' extents
+    double candidates = 0;
+    for (const auto &x : ss) {
+        const double L = x.g.L, pi = 3.14159265358979;
+        const double v = bins.mode == MIA_RPPI ? pi * reach_r * reach_r * std::min(L, 2 * reach_z)
+                                               : 4.0 / 3.0 * pi * reach_r * reach_r * reach_r;
+        candidates += 1.5 * (double)x.n_shape * (double)x.n_pos * std::min(1.0, v / (L * L * L));
+    }
+    p.pc = pair_config(bins, p.any_w, p.any_var, tuning, ctx.cu_count, candidates);
     p.det = tuning && tuning->deterministic != 0;
 
     p.ps.resize(S);
@@ -1794,11 +1729,10 @@ CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_b
     p.fs.resize(S);
     p.G.resize(S);
     p.cell0.assign(S + 1, 0);
-    p.t0.assign(S + 1, 0);
-    p.t0r.assign(S + 1, 0);
     p.fin0.assign(S + 1, 0);
     p.acc0.assign(S + 1, 0);
-    double est_items = 0, est_ranges = 0;
+    double est_items = 0;
+    int jk_max = 1;
     for (int si = 0; si < S; ++si) {
         const SortedSample &x = ss[si];
         const Grid &g = x.g;
@@ -1826,53 +1760,46 @@ CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_b
         Q.periodic = x.periodic;
         Q.ng = g.nz / G;
         Q.G = G;
-        Q.kx = (int)std::ceil((reach_r + 4 * g.margin) / g.cw) + 1;
-        Q.nxw = std::min(g.nc, 2 * Q.kx + 1);
-        Q.pmax = pmax_set > 0 ? pmax_set : (g.pmax > 0 ? g.pmax : 1024);
+        Q.ncp = g.nc * g.m;
+        Q.pbits = x.pbits;
+        Q.fw = g.cw / g.m;
+        Q.hq = g.hz / (double)(1 << x.pbits);
+        // columns per item: about kItemPositions positions at the mean density
+        // (mia_tuning.item_positions), at most one column per lane
+        const double per_col = (double)x.n_pos / ((double)Q.ncp * Q.ncp) *
+                               std::min(1.0, 2.0 * reach_z / std::max(g.L, 1e-300));
+        const double want_pos = tuning && tuning->item_positions > 0 ? tuning->item_positions : kItemPositions;
+        Q.cpi = (int)std::max(1.0, std::min((double)kWave, std::floor(want_pos / std::max(per_col, 1e-9) + 0.5)));
+        jk_max = std::max(jk_max, g.jk);
         Q.reach_r = reach_r;
         Q.reach_z = reach_z;
         Q.x_lo = bins.mode == MIA_RPPI ? bins.x2_edges[0] : -reach_r;
         Q.x_hi = bins.mode == MIA_RPPI ? bins.x2_edges[n_2] : reach_r;
         Q.sstart = x.sstart;
-        Q.pstart = x.pstart;
         Q.ncells = (int64_t)g.nc * g.nc * (Q.ng + 1);
         Q.cell0 = p.cell0[si];
         p.cell0[si + 1] = Q.cell0 + Q.ncells;
         const int64_t blk_cap = (x.n_shape + p.bsz - 1) / p.bsz + std::min<int64_t>(Q.ncells, x.n_shape);
-        Q.ngc = (Q.nxw * Q.nxw + kGroupColumns - 1) / kGroupColumns;
-        Q.nt = blk_cap * Q.ngc;
-        Q.t0 = p.t0[si];
-        p.t0[si + 1] = Q.t0 + (Q.nt + kPlanThreads - 1) / kPlanThreads * kPlanThreads;
-        Q.ntr = blk_cap * Q.nxw * Q.nxw;
-        Q.t0r = p.t0r[si];
-        p.t0r[si + 1] = Q.t0r + (Q.ntr + kPlanThreads - 1) / kPlanThreads * kPlanThreads;
+        p.nblk_cap += blk_cap;
         const int K = x.K;
         p.fin0[si + 1] = p.fin0[si] + (int64_t)(1 + K) * B + K;
         // accumulators: npairs, sp, dd ((1+K) B each), sx, var (B each)
         p.acc0[si + 1] = p.acc0[si] + 3 * (int64_t)(1 + K) * B + 2 * (int64_t)B;
-        double er = 0;
-        est_items += estimate_items(g, G, reach_r, reach_z, bins.mode == MIA_RMU, x.n_shape, x.n_pos, Q.pmax, &er);
-        est_ranges += er;
+        est_items += estimate_items(g, G, Q.cpi, reach_r, reach_z, bins.mode == MIA_RMU, x.n_shape, x.n_pos, blk_cap);
     }
+    p.kseg = std::min(jk_max + kSegExtra, kMaxSegs);
     p.ncells = p.cell0[S];
-    p.nthreads = p.t0[S];
-    p.nthreads_r = p.t0r[S];
     p.fin_total = p.fin0[S];
     p.acc_total = p.acc0[S];
     MIA_REQUIRE((double)S * p.K1 * p.K1 < 2e9, "too many planner keys (samples x regions^2)");
     p.nkeys = (int64_t)S * p.K1 * p.K1;
     p.slot_cap = p.det ? (int64_t)p.pc.waves + p.nkeys : 0;
-    MIA_REQUIRE(!p.det || p.nthreads < ((int64_t)1 << 32), "plan too large for the deterministic item order");
-    const size_t plan_lds = (size_t)p.K1 * p.K1 * (sizeof(int64_t) + sizeof(int32_t));
-    p.plan_local = plan_lds <= 64 * 1024 ? 1 : 0;
-    // item capacity: the caller's (grown after an overflow), at least 3x the
-    // uniform-density estimate plus a margin; range capacity (the planner's
-    // ranges and the items' range records): 1.25x the estimate, which runs
-    // 1.3-2x above the counts of the clustered benchmark samples
-    p.item_cap = cap_exact ? item_cap : std::max<int64_t>(item_cap, (int64_t)(3.0 * est_items) + 65536);
+    MIA_REQUIRE(p.nblk_cap < ((int64_t)1 << 31), "too many shape blocks");
+    MIA_REQUIRE(!p.det || det_key_bits(p) <= 64, "plan too large for the deterministic item order");
+    // item capacity: the caller's (grown after an overflow), at least twice
+    // the uniform-density estimate plus a margin
+    p.item_cap = cap_exact ? item_cap : std::max<int64_t>(item_cap, (int64_t)(2.0 * est_items) + 65536);
     p.item_cap = std::min<int64_t>(p.item_cap, (int64_t)1 << 31);
-    p.range_cap = cap_exact ? range_cap : std::max<int64_t>(range_cap, (int64_t)(1.25 * est_ranges) + 65536);
-    p.range_cap = std::min<int64_t>(p.range_cap, ((int64_t)1 << 31) - kItemRanges);
 
     // the launch-sequence key: everything the launches depend on except the
     // caller's pointers (which live in the parameter block)
@@ -1884,10 +1811,9 @@ CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_b
     put(p.X.data(), sizeof(double) * p.X.size());
     if (tuning) put(tuning, sizeof(*tuning));
     put(&p.item_cap, sizeof(p.item_cap));
-    put(&p.range_cap, sizeof(p.range_cap));
     for (int si = 0; si < S; ++si) {
         PlanSample q = p.ps[si];
-        q.sstart = q.pstart = q.pfine = nullptr;
+        q.sstart = q.pfine = q.flags = nullptr;
         q.srec = nullptr;
         put(&q, sizeof(q));
         put(&ss[si].n_pos, sizeof(int64_t));
@@ -1896,13 +1822,6 @@ CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_b
         put(&ss[si].weighted, sizeof(int));
     }
     return P.release();
-}
-
-// bits of the deterministic item sort key: 32 of plan thread + the key index
-int det_key_bits(const CountPlan &p) {
-    int b = 1;
-    while (b < 31 && ((int64_t)1 << b) < p.nkeys + 1) ++b;
-    return 32 + b;
 }
 
 size_t count_bytes(const CountPlan &p) {
@@ -1922,8 +1841,6 @@ void count_bind(CountPlan &p, Carve &c, const std::vector<SortedSample> &ss, con
     p.off_T = pc.off; pc.take<double>(n_r + 1);
     p.off_X = pc.off; pc.take<double>(n_2 + 1);
     p.off_cell0 = pc.off; pc.take<int64_t>(S + 1);
-    p.off_t0 = pc.off; pc.take<int64_t>(S + 1);
-    p.off_t0r = pc.off; pc.take<int64_t>(S + 1);
     p.off_fin0 = pc.off; pc.take<int64_t>(S + 1);
     p.off_ps = pc.off; pc.take<PlanSample>(S);
     p.off_sd = pc.off; pc.take<SampleDev>(S);
@@ -1944,24 +1861,18 @@ void count_bind(CountPlan &p, Carve &c, const std::vector<SortedSample> &ss, con
     p.nb = c.take<int32_t>(p.ncells + 1);
     p.boff = c.take<int32_t>(p.ncells + 1);
     scan_carve<int32_t>(c, p.ncells, p.scan_nb);
-    int64_t blk_total = 0;
-    for (int si = 0; si < S; ++si) blk_total += p.ps[si].nt / p.ps[si].ngc;
-    p.blocks = c.take<Block>(std::max<int64_t>(blk_total, 1));
-    p.bbox = c.take<double>(6 * std::max<int64_t>(blk_total, 1));
-    p.bruns = c.take<int32_t>((kBlockRuns + 1) * std::max<int64_t>(blk_total, 1));
+    const int64_t blk_total = std::max<int64_t>(p.nblk_cap, 1);
+    p.blocks = c.take<Block>(blk_total);
+    p.bbox = c.take<double>(6 * blk_total);
+    p.geo = c.take<uint32_t>((3 + 3 * (int64_t)p.kseg) * blk_total);
     p.ko = c.take<int64_t>(p.nkeys + 1);
     scan_carve<int64_t>(c, p.nkeys, p.scan_keys);
     p.items = c.take<Item>(p.item_cap);
-    // kItemRanges records of slack: the pair kernel loads a full set per item
-    p.ranges = c.take<Range>(p.range_cap + kItemRanges);
-    p.raw = c.take<RawRange>(p.range_cap);
-    p.roff = c.take<int32_t>(std::max<int64_t>(p.nthreads_r, 1));
-    p.rcnt = c.take<int32_t>(std::max<int64_t>(p.nthreads_r, 1));
     p.cost = c.take<int64_t>(p.item_cap + 1);
     p.cpre = c.take<int64_t>(p.item_cap + 1);
     scan_carve<int64_t>(c, p.item_cap, p.scan_cost);
     p.n_items = c.take<int64_t>(1);
-    p.bounds = c.take<int64_t>((size_t)p.pc.waves * kScheduleUnits + 3);
+    p.bounds = c.take<int64_t>((size_t)p.pc.groups * kScheduleUnits + 3);
     if (p.det) {
         const int64_t W = p.pc.waves, sw = p.slot_cap * B;
         p.runs = c.take<int64_t>(W + 1);
@@ -1998,8 +1909,6 @@ void count_bind(CountPlan &p, Carve &c, const std::vector<SortedSample> &ss, con
     std::memcpy(img + p.off_T, p.T.data(), sizeof(double) * (n_r + 1));
     std::memcpy(img + p.off_X, p.X.data(), sizeof(double) * (n_2 + 1));
     std::memcpy(img + p.off_cell0, p.cell0.data(), sizeof(int64_t) * (S + 1));
-    std::memcpy(img + p.off_t0, p.t0.data(), sizeof(int64_t) * (S + 1));
-    std::memcpy(img + p.off_t0r, p.t0r.data(), sizeof(int64_t) * (S + 1));
     std::memcpy(img + p.off_fin0, p.fin0.data(), sizeof(int64_t) * (S + 1));
     unsigned long long *acc = p.acc;
     double *accd = (double *)p.acc;
@@ -2010,15 +1919,13 @@ void count_bind(CountPlan &p, Carve &c, const std::vector<SortedSample> &ss, con
         const int64_t a0 = p.acc0[si];
         PlanSample &Q = p.ps[si];
         Q.sstart = x.sstart;
-        Q.pstart = x.pstart;
         Q.pfine = x.pfine;
-        Q.sbits = x.sbits;
+        Q.flags = x.flags;
         Q.srec = x.srec;
         SampleDev &D = p.sd[si];
         std::memset(&D, 0, sizeof(D));
         D.prec = x.prec;
         D.srec = x.srec;
-        D.pstart = x.pstart;
         D.L = x.g.L;
         D.half = x.g.half;
         D.los = x.g.los;
@@ -2054,73 +1961,41 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
     const char *pd = p.param_dev;
     const PlanSample *ps = (const PlanSample *)(pd + p.off_ps);
     const int64_t *cell0 = (const int64_t *)(pd + p.off_cell0);
-    const int64_t *t0 = (const int64_t *)(pd + p.off_t0);
-    const int64_t *t0r = (const int64_t *)(pd + p.off_t0r);
     const int64_t *fin0 = (const int64_t *)(pd + p.off_fin0);
     if (ev) MIA_HIP(hipEventRecord(ev[0], st));
     fill<unsigned long long>(p.zero_begin, 0ull, (int64_t)p.zero_words, st);
     // shape blocks of every (column, slab group) cell
     hipLaunchKernelGGL(k_blocks, dim3(nblk(p.ncells, 256)), dim3(256), 0, st, ps, cell0, S, p.bsz, p.nb,
-                       (const int32_t *)nullptr, (Block *)nullptr, (double *)nullptr, (int32_t *)nullptr);
+                       (const int32_t *)nullptr, (Block *)nullptr);
     MIA_HIP(hipGetLastError());
     scan_ws<int32_t>(p.nb, p.boff, p.ncells, nullptr, p.scan_nb, st);
     hipLaunchKernelGGL(k_blocks, dim3(nblk(p.ncells, 256)), dim3(256), 0, st, ps, cell0, S, p.bsz, p.nb,
-                       (const int32_t *)p.boff, p.blocks, p.bbox, p.bruns);
+                       (const int32_t *)p.boff, p.blocks);
     MIA_HIP(hipGetLastError());
-    // the position ranges of every (block, stencil column) pair
-    RangeLaunch R{};
-    R.ps = ps;
-    R.t0r = t0r;
-    R.S = S;
-    R.K1 = p.K1;
-    R.boff = p.boff;
-    R.blocks = p.blocks;
-    R.bbox = p.bbox;
-    R.bruns = p.bruns;
-    R.raw = p.raw;
-    R.raw_cursor = p.words + 8;
-    R.raw_cap = p.range_cap;
-    R.roff = p.roff;
-    R.rcnt = p.rcnt;
-    R.overflow = p.words + 2;
-    const int64_t nvwg_r = (p.nthreads_r + kPlanThreads - 1) / kPlanThreads;
-    const unsigned rgrid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(nvwg_r, 256 * kPlanGridPerCu));
-    hipLaunchKernelGGL(k_plan_ranges, dim3(rgrid), dim3(kPlanThreads), 0, st, R);
-    MIA_HIP(hipGetLastError());
-    // work items packed from the ranges, counting-sorted by (sample, R_s, R_p)
+    // their reach, and the items per key
     PlanLaunch L{};
     L.ps = ps;
-    L.t0 = t0;
-    L.S = S;
+    L.ncells = p.ncells;
     L.K1 = p.K1;
+    L.kseg = p.kseg;
     L.boff = p.boff;
     L.blocks = p.blocks;
-    L.raw = p.raw;
-    L.roff = p.roff;
-    L.rcnt = p.rcnt;
+    L.bbox = p.bbox;
+    L.geo = p.geo;
     L.key_count = p.kc;
     L.key_cursor = p.kcur;
     L.key_off = p.ko;
     L.items = p.items;
-    L.cost = p.cost;
     L.cap = p.item_cap;
-    L.ranges = p.ranges;
-    L.range_cursor = p.words + 7;
-    L.range_cap = p.range_cap;
     L.overflow = p.words + 2;
-    L.candidates = p.words + 1;
-    L.local = p.plan_local;
-    const size_t plan_lds = p.plan_local ? (size_t)p.K1 * p.K1 * 12 : 0;
-    const int64_t nvwg = (p.nthreads + kPlanThreads - 1) / kPlanThreads;
-    const unsigned pgrid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(nvwg, 256 * kPlanGridPerCu));
-    L.emit = 0;
-    hipLaunchKernelGGL(k_plan_items, dim3(pgrid), dim3(kPlanThreads), plan_lds, st, L);
+    const unsigned bgrid = (unsigned)std::max<int64_t>(
+        1, std::min<int64_t>((p.nblk_cap + kPlanWaves - 1) / kPlanWaves, 256 * kPlanGridPerCu));
+    hipLaunchKernelGGL(k_block_geom, dim3(bgrid), dim3(kPlanThreads), 0, st, L);
     MIA_HIP(hipGetLastError());
     scan_ws<int64_t>((const int64_t *)p.kc, p.ko, p.nkeys, nullptr, p.scan_keys, st);
     hipLaunchKernelGGL(k_items_total, dim3(1), dim3(64), 0, st, (const int64_t *)p.ko, p.nkeys, p.item_cap,
                        p.n_items, p.words + 3);
     MIA_HIP(hipGetLastError());
-    L.emit = 1;
     const Item *items = p.items;
     const int64_t *cost = p.cost;
     if (p.det) {
@@ -2128,8 +2003,14 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
         hipLaunchKernelGGL(k_iota, dim3(nblk(p.item_cap, 256)), dim3(256), 0, st, p.sidx, p.item_cap);
         MIA_HIP(hipGetLastError());
         L.sort_key = p.skey;
+        L.sort_shift = det_low_bits(p);
     }
-    hipLaunchKernelGGL(k_plan_items, dim3(pgrid), dim3(kPlanThreads), plan_lds, st, L);
+    hipLaunchKernelGGL(k_emit_items, dim3(bgrid), dim3(kPlanThreads), 0, st, L);
+    MIA_HIP(hipGetLastError());
+    const unsigned igrid = (unsigned)std::max<int64_t>(
+        1, std::min<int64_t>((p.item_cap + kPlanWaves - 1) / kPlanWaves, 256 * kPlanGridPerCu));
+    hipLaunchKernelGGL(k_item_cost, dim3(igrid), dim3(kPlanThreads), 0, st, ps, (const Block *)p.blocks,
+                       (const double *)p.bbox, (const int64_t *)p.n_items, p.items, p.cost, p.words + 1);
     MIA_HIP(hipGetLastError());
     if (p.det) {
         // items of one key in (plan thread, emission) order: a stable sort of
@@ -2146,7 +2027,7 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
         cost = p.cost2;
     }
     scan_ws<int64_t>(cost, p.cpre, p.item_cap, p.n_items, p.scan_cost, st);
-    schedule_bounds(p.cpre, p.n_items, p.pc.waves, p.bounds, st, p.det);
+    schedule_bounds(p.cpre, p.n_items, p.pc.groups, p.bounds, st, p.det, p.pc.A.shared ? p.pc.wpb : 1);
     if (p.det) {
         // slot numbers of every wave's flushes (slot0[W] = slots in all)
         hipLaunchKernelGGL(k_key_nonempty, dim3(nblk(p.nkeys, 256)), dim3(256), 0, st, (const int64_t *)p.ko,
@@ -2162,11 +2043,13 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
     // pair kernel, one launch per r-bin pass
     PairArgs A = p.pc.A;
     A.items = items;
-    A.ranges = p.ranges;
+    A.ps = ps;
+    A.bbox = p.bbox;
     A.overflow = p.words + 2;
     A.blocks = p.blocks;
     A.n_items = p.n_items;
     A.bounds = p.bounds;
+    A.key_off = p.ko;
     A.T = (const double *)(pd + p.off_T);
     A.X = (const double *)(pd + p.off_X);
     A.samples = (const SampleDev *)(pd + p.off_sd);
@@ -2192,7 +2075,7 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
         A.T = (const double *)(pd + p.off_T) + r0;
         A.T0 = p.T[r0];
         A.Tn = p.T[r1];
-        A.lgc = (float)(-p.pc.l0 * p.pc.lgs - r0);
+        A.lgc = (float)(-p.pc.l0 * p.pc.lgs - r0 + p.pc.shift_r);
         A.queue = p.queue + pass;
         if (A.mode == MIA_RPPI)
             launch_pairs_mode<MIA_RPPI>(A, p.pc.grid, p.pc.wpb, p.pc.lds, st);

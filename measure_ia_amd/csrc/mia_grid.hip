@@ -1,20 +1,21 @@
-// Grid autotuner: columns per side, slabs per side and slabs per shape block.
+// Grid autotuner: columns per side, slabs per side, slabs per shape block and
+// position columns per column.
 //
-// The count's time (pair kernel + planning) is, to within a few percent over
-// the measured range,
-//     t = t0 + a * candidates + b * items
-// (t0: the in-domain pairs, fixed by the data; candidates = (shape, position)
-// pairs the work items evaluate; items = packed work items).  For a grid the
-// last two are estimated on the host for uniform densities -- the expected
-// number of positions in the cells each shape block reaches, and the items the
-// planner packs from each group of stencil columns -- and the grid with the
-// lowest a*cand + b*items is taken.  The candidate estimate is ~10 % high on
-// clustered samples (the same for every grid); the item estimate is scaled by
-// its measured ratio (0.7).  a and b were fitted on MI355X sweeps of a
-// 1M-position w_gg/w_g+ count and a 2M-position multipole count: a = 0.58 ps
-// (r_p, pi) and 0.85 ps (r, mu) per candidate, b = 1.0 ns (r_p, pi) and
-// 1.3 ns (r, mu) per item.  Choices are cached per (box, binning reach,
-// jackknife, sizes).
+// The time of the planner and the pair kernel on a grid, for uniform densities:
+//   tests : every shape against the positions of the position columns within
+//           reach of its block, in batches of 64 lanes (half a batch of every
+//           item is idle);
+//   runs  : once per block and position, the lane's pending histogram run ends;
+//   bodies: the pairs whose column touches the domain of their shape (bins,
+//           e+ and ex, the histogram);
+//   items : the column lookup and the planner's work per item.
+// Thin position columns cut tests and bodies near the edge of the domain and
+// add items (at most 64 columns each); small blocks cut tests and add runs and
+// items.  The areas that columns of width f cover around a block or a shape are
+// those of the Minkowski sums (for a convex outline of area A and perimeter p
+// on a square grid, on average A + (2/pi) p f + f^2).  The constants are a fit
+// to eight grids of a million clustered positions (200,000 shapes, reach 20 by
+// 60), 8.7 to 9.8 ms: within 3 %, the best grid 2 % from the one it picks.
 #include "mia_common.hpp"
 
 #include <algorithm>
@@ -26,90 +27,73 @@ namespace mia {
 
 namespace {
 
-constexpr double kCandCostW = 0.58e-12;  // s per candidate, (r_p, pi)
-constexpr double kCandCostMu = 0.85e-12; // s per candidate, (r, mu)
-constexpr double kItemCostW = 1.0e-9;    // s per work item, (r_p, pi)
-constexpr double kItemCostMu = 1.3e-9;   // s per work item, (r, mu)
-constexpr double kItemScale = 0.7;       // measured items / estimated items
+constexpr double kTestCost = 1.15e-12;   // s per tested (shape, position) pair
+constexpr double kRunCost = 1.1e-12;     // s per tested (block, position) pair
+constexpr double kBodyCost = 1.0e-12;    // s per pair of the columns that touch a shape's domain
+constexpr double kItemCost = 1.5e-9;     // s per work item
 constexpr int kBlockShapes = 64;
-constexpr int kItemPositions = 1024;
-// Dense columns split their position runs into many 1024-position items;
-// 2048 halves those splits.  Measured: large20M (runs of thousands of
-// positions) 1.5 % faster at 2048, the 1M/2M boxes and the batch within
-// 0.5 % either way.  Taken when it cuts the estimated items by a tenth.
-constexpr int kItemPositionsDense = 2048;
+constexpr int kItemPositions = 8192;
+constexpr int kMaxPosColumns = 4096;     // position columns per side (12-bit indices)
 
 struct Choice {
-    int ncj, nzj, G, pmax;
+    int ncj, nzj, G, m;
 };
 
-// Expected candidates, work items and position ranges of one grid (uniform
-// densities).  Per shape block: every reached stencil column holds
-// `pos` positions in (1 + win/jspan + win/L) line-of-sight runs (jackknife
-// slab and periodic-wrap splits); the planner packs the runs of each group of
-// kGroupColumns columns into items of at most pmax positions and kItemRanges
-// runs, one item per (region, shift) class at least.
-void estimate(double L, int jk, int ncj, int nzj, int G, double R, double Z, bool rmu, double Ns,
-              double Np, double &cand, double &items, double *ranges = nullptr, int pmax = kItemPositions) {
-    const int nc = ncj * jk, nz = nzj * jk;
-    const double cw = L / nc, hz = L / nz;
-    int kx = (int)std::ceil(R / cw) + 1;
-    int lo = -kx, hi = kx;
-    if (2 * kx + 1 >= nc) {  // the stencil covers the plane: each column once
-        lo = -(nc / 2);
-        hi = lo + nc - 1;
-    }
-    const int nxw = hi - lo + 1;
-    const double cell_p = Np / ((double)nc * nc * nz);
-    const double jspan = L / jk;
-    double zsum = 0.0, per_block = 0.0, rec = 0.0;
-    double g_pos = 0.0, g_runs = 0.0, g_cls = 0.0;
-    int g_at = -1;
-    auto close_group = [&]() {
-        if (g_cls > 0.0) {
-            const double n = std::max({g_cls, std::ceil(g_pos / pmax) + g_cls - 1.0, std::ceil(g_runs / kItemRanges)});
-            per_block += n;
-            rec += g_runs;
-        }
-        g_pos = g_runs = g_cls = 0.0;
-    };
-    for (int i = lo; i <= hi; ++i) {
-        int ai = std::abs(i);
-        if (2 * kx + 1 >= nc) ai = std::min(ai, nc - ai);
-        double u = std::max(ai - 1, 0) * cw;
-        for (int j = lo; j <= hi; ++j) {
-            const int grp = ((i - lo) * nxw + (j - lo)) / kGroupColumns;
-            if (grp != g_at) {
-                close_group();
-                g_at = grp;
-            }
-            int aj = std::abs(j);
-            if (2 * kx + 1 >= nc) aj = std::min(aj, nc - aj);
-            double v = std::max(aj - 1, 0) * cw;
-            double d2 = u * u + v * v;
-            if (d2 >= R * R) continue;
-            double reach = rmu ? std::sqrt(R * R - d2) : Z;
-            int nsl = std::min(G + 2 * (int)std::ceil(reach / hz), nz);
-            zsum += nsl;
-            double win = nsl * hz;
-            double pos = cell_p * nsl;
-            const double cls = 1.0 + win / jspan + win / L;
-            g_pos += pos;
-            g_runs += cls * std::max(1.0, std::ceil(pos / pmax));
-            g_cls = std::max(g_cls, cls);
-        }
-    }
-    close_group();
-    cand = Ns * cell_p * zsum;
-    const double groups = (double)nc * nc * (nz / G);
+// Expected cost and work items of one grid.
+double grid_cost(double L, int jk, const Choice &c, double R, double Z, bool rmu, double Ns, double Np,
+                 double *items_out = nullptr) {
+    const double pi = 3.14159265358979;
+    const int nc = c.ncj * jk, nz = c.nzj * jk;
+    const double cw = L / nc, h = L / nz * c.G, f = cw / c.m;
+    const double rho = Np / (L * L * L);
+    const double groups = (double)nc * nc * (nz / c.G);
     const double lam = Ns / groups;
     const double nblocks = groups * (1.0 - std::exp(-lam)) * std::max(1.0, lam / kBlockShapes);
-    items = kItemScale * nblocks * per_block;
-    if (ranges) *ranges = nblocks * rec;
+    const double per_block = Ns / std::max(nblocks, 1e-300);
+    // a block of few shapes is smaller than its cells
+    const double shrink = per_block > 1.0 ? (per_block - 1.0) / (per_block + 1.0) : 0.0;
+    const double bw = cw * shrink, bh = h * shrink;
+    // position columns of width g around a square block of side w
+    auto area = [&](double w, double g) {
+        const double a = w * w + 4.0 * w * R + pi * R * R, p = 4.0 * w + 2.0 * pi * R;
+        return std::min(L * L, a + 2.0 / pi * p * g + g * g);
+    };
+    // mean line-of-sight window over those columns
+    const double win = std::min(L, (rmu ? 4.0 / 3.0 * R : 2.0 * Z) + bh);
+    const double per_col = rho * f * f * win;
+    const double tests = Ns * rho * area(bw, f) * win;
+    const double columns = area(bw, f) / (f * f);
+    const double cpi = std::max(1.0, std::min((double)kWave, kItemPositions / std::max(per_col, 1e-9)));
+    // rectangles of one sub-box and shift class the reach falls into
+    const double side = bw + 2.0 * R + f;
+    const double sx = 1.0 + std::min(side, L) / (L / jk), sz = 1.0 + win / (L / jk) + win / L;
+    const double rects = sx * sx * sz;
+    const double items = nblocks * std::max(rects, 1.27 * columns * sz / cpi + 0.5 * rects);
+    if (items_out) *items_out = items;
+    const double idle = items * 32.0 * per_block;
+    return kTestCost * (tests + idle) + kRunCost * tests / std::max(per_block, 1.0) +
+           kBodyCost * Ns * rho * area(0.0, f) * win + kItemCost * items;
 }
 
 std::mutex g_mu;
 std::map<std::tuple<double, int, double, double, int, int64_t, int64_t>, Choice> g_cache;
+
+// Position columns per column: the cheapest of 1 .. 8.
+int best_m(double L, int jk, Choice c, double R, double Z, bool rmu, double Ns, double Np, double *cost) {
+    int best = 1;
+    double best_t = -1.0;
+    for (c.m = 1; c.m <= 8; ++c.m) {
+        const double n = (double)c.ncj * jk * c.m;
+        if (c.m > 1 && (n > kMaxPosColumns || n * n * (c.nzj * jk + 1.0) > 8.0 * Np + 262144.0)) break;
+        const double t = grid_cost(L, jk, c, R, Z, rmu, Ns, Np);
+        if (best_t < 0 || t < best_t) {
+            best_t = t;
+            best = c.m;
+        }
+    }
+    *cost = best_t;
+    return best;
+}
 
 Choice search(double L, int jk, double R, double Z, bool rmu, int64_t ns, int64_t np) {
     auto key = std::make_tuple(L, jk, R, Z, (int)rmu, ns, np);
@@ -121,33 +105,25 @@ Choice search(double L, int jk, double R, double Z, bool rmu, int64_t ns, int64_
     const double Ns = (double)std::max<int64_t>(ns, 1), Np = (double)std::max<int64_t>(np, 1);
     const double span = L / jk;
     const double zr = rmu ? R : Z;
-    const double a = rmu ? kCandCostMu : kCandCostW;
-    const double b = rmu ? kItemCostMu : kItemCostW;
     // column widths in [R/12, R/2], slab heights in [zr/12, max(zr, R)/2], at most 512 per side
     int c0 = std::max(1, (int)std::floor(span / (R / 2.0)));
     int c1 = std::max(c0, std::min(512 / jk, (int)std::ceil(span / (R / 12.0))));
     int z0 = std::max(1, (int)std::floor(span / (std::max(zr, R) / 2.0)));
     int z1 = std::max(z0, std::min(512 / jk, (int)std::ceil(span / (zr / 12.0))));
-    Choice best{c0, z0, 1, 0};
+    Choice best{c0, z0, 1, 1};
     double best_t = -1.0;
     for (int ncj = c0; ncj <= c1; ++ncj)
         for (int nzj = z0; nzj <= z1; ++nzj)
             for (int G = 1; G <= 4 && G <= nzj; ++G) {
                 if (nzj % G) continue;
-                double cand, items;
-                estimate(L, jk, ncj, nzj, G, R, Z, rmu, Ns, Np, cand, items);
-                double t = a * cand + b * items;
+                Choice c{ncj, nzj, G, 1};
+                double t;
+                c.m = best_m(L, jk, c, R, Z, rmu, Ns, Np, &t);
                 if (best_t < 0 || t < best_t) {
                     best_t = t;
-                    best = Choice{ncj, nzj, G, 0};
+                    best = c;
                 }
             }
-    {
-        double cand, items, items2;
-        estimate(L, jk, best.ncj, best.nzj, best.G, R, Z, rmu, Ns, Np, cand, items);
-        estimate(L, jk, best.ncj, best.nzj, best.G, R, Z, rmu, Ns, Np, cand, items2, nullptr, kItemPositionsDense);
-        if (items2 < 0.9 * items) best.pmax = kItemPositionsDense;
-    }
     std::lock_guard<std::mutex> lk(g_mu);
     g_cache[key] = best;
     return best;
@@ -155,15 +131,20 @@ Choice search(double L, int jk, double R, double Z, bool rmu, int64_t ns, int64_
 
 }  // namespace
 
-double estimate_items(const Grid &g, int G, double reach_r, double reach_z, bool rmu, int64_t ns, int64_t np,
-                      int pmax, double *ranges) {
+// Expected work items (at most what the block capacity allows).
+double estimate_items(const Grid &g, int G, int cpi, double reach_r, double reach_z, bool rmu, int64_t ns, int64_t np,
+                      int64_t blk_cap) {
+    if (ns <= 0 || np <= 0) return 0.0;
     const int jk = g.jk > 0 ? g.jk : 1;
-    double cand = 0, items = 0, rec = 0;
-    estimate(g.L, jk, g.ncj, g.nzj, std::max(1, G), reach_r, reach_z, rmu, (double)std::max<int64_t>(ns, 1),
-             (double)std::max<int64_t>(np, 1), cand, items, &rec, pmax);
-    const bool any = ns > 0 && np > 0;
-    if (ranges) *ranges = any ? rec : 0.0;
-    return any ? items : 0.0;
+    const double fw = g.cw / g.m;
+    const double groups = (double)g.nc * g.nc * (g.nz / std::max(1, G));
+    const double lam = (double)ns / groups;
+    const double nblocks =
+        std::min((double)blk_cap, groups * (1.0 - std::exp(-lam)) * std::max(1.0, lam / kBlockShapes) + 1.0);
+    const double side = std::min(g.L, g.cw + 2.0 * reach_r + fw), win = std::min(g.L, 2.0 * reach_z + G * g.hz);
+    const double sx = 1.0 + side / (g.L / jk) + side / g.L, sz = 1.0 + win / (g.L / jk) + win / g.L;
+    const double cols = (side / fw + 1.0) * (side / fw + 1.0);
+    return nblocks * sz * (cols / cpi + sx * sx);
 }
 
 Grid make_grid(const mia_sample &s, const mia_bins &bins, const mia_tuning *t) {
@@ -199,7 +180,6 @@ Grid make_grid(const mia_sample &s, const mia_bins &bins, const mia_tuning *t) {
         ncj = c.ncj;
         nzj = c.nzj;
         G = c.G;
-        g.pmax = c.pmax;
     }
     if (t && t->columns_per_side > 0) ncj = std::max(1, t->columns_per_side / jk_eff);
     if (t && t->slabs_per_side > 0) nzj = std::max(1, t->slabs_per_side / jk_eff);
@@ -212,6 +192,12 @@ Grid make_grid(const mia_sample &s, const mia_bins &bins, const mia_tuning *t) {
     g.cw = g.L / g.nc;
     g.hz = g.L / g.nz;
     g.margin = 1e-9 * g.L + 1e-12;
+    {
+        Choice c{ncj, nzj, G > 0 && nzj % G == 0 ? G : 1, 1};
+        double t;
+        g.m = best_m(g.L, jk_eff, c, reach_r, reach_z, rmu, (double)std::max<int64_t>(s.n_shape, 1),
+                     (double)std::max<int64_t>(s.n_pos, 1), &t);
+    }
     g.G = (G > 0 && nzj % G == 0) ? G : 0;
     return g;
 }

@@ -63,6 +63,8 @@ struct PrepSeg {
     int64_t key0;             // first cell key of the sample in the concatenated key arrays
     int64_t wg0;              // first workgroup of the segment
     Grid g;
+    int ncj, nc;              // columns per sub-box and side: the grid's, or (positions) g.m times as many
+    double cw;
     int kind, K, sample, sbits;
     int32_t *cnt;             // key counters of the kind
     const int32_t *start;     // scanned key starts of the kind
@@ -71,7 +73,7 @@ struct PrepSeg {
     double *rsum;             // [2K] of the sample: sum w_s, sum w_s (1 - e^2/2) per region
     double *prec;
     double *srec;
-    int *oor;                 // the sample's out-of-box flag
+    int *oor;                 // the sample's flags: 1 a coordinate out of the box, 2 a position in a column's tail
 };
 
 __device__ __forceinline__ int find_seg(const int64_t *tab, int n, int64_t v) {
@@ -131,7 +133,7 @@ __global__ __launch_bounds__(kStageThreads) void k_stage_classify(const PrepSeg 
         }
         __syncthreads();
     }
-    bool bad = false;
+    bool bad = false, tail = false;
     const int64_t base = (int64_t)(blockIdx.x - G.wg0) * kStageWg + threadIdx.x;
     const int lane = threadIdx.x & (kWave - 1);
     // 1: every item's coordinates -> region and cell key (all loads in flight
@@ -168,13 +170,14 @@ __global__ __launch_bounds__(kStageThreads) void k_stage_classify(const PrepSeg 
 #pragma unroll
             for (int c = 0; c < 3; ++c) ji[c] = strict_axis_index(x[c], g.jk_sub, g.jk);
             anom = ji[0] < 0 || ji[1] < 0 || ji[2] < 0;
+            tail = tail || (anom && valid[it]);
             if (!anom) region[it] = ji[0] * g.jk * g.jk + ji[1] * g.jk + ji[2];
         }
-        const int ca = stage_axis_cell(x[g.ax_a], anom ? -1 : ji[g.ax_a], g.jk_sub, g.ncj, g.cw, g.nc);
-        const int cb = stage_axis_cell(x[g.ax_b], anom ? -1 : ji[g.ax_b], g.jk_sub, g.ncj, g.cw, g.nc);
+        const int ca = stage_axis_cell(x[g.ax_a], anom ? -1 : ji[g.ax_a], g.jk_sub, G.ncj, G.cw, G.nc);
+        const int cb = stage_axis_cell(x[g.ax_b], anom ? -1 : ji[g.ax_b], g.jk_sub, G.ncj, G.cw, G.nc);
         int sub = 0;
         const int cl = stage_axis_cell(x[g.los], anom ? -1 : ji[g.los], g.jk_sub, g.nzj, g.hz, g.nz, &sub, G.sbits);
-        const int64_t cell = G.key0 + (int64_t)(ca * g.nc + cb) * (g.nz + 1) + (anom ? g.nz : cl);
+        const int64_t cell = G.key0 + ((int64_t)ca * G.nc + cb) * (g.nz + 1) + (anom ? g.nz : cl);
         // fine key (cell << sbits) + part of the slab (0 in the tail slot)
         key[it] = (int)((cell << G.sbits) + (anom ? 0 : sub));
         // per-region sums of shapes: w and w (1 - e^2/2)
@@ -233,6 +236,7 @@ __global__ __launch_bounds__(kStageThreads) void k_stage_classify(const PrepSeg 
         }
     }
     if (bad) atomicOr(G.oor, 1);
+    if (tail && G.kind == 0) atomicOr(G.oor, 2);
     if (lds) {
         __syncthreads();
         for (int r = threadIdx.x; r < K; r += blockDim.x) {
@@ -415,17 +419,18 @@ struct PrepPlan {
     std::vector<Grid> grids;
     std::vector<PrepSeg> segs;      // 2S: positions of s at 2s, shapes at 2s + 1
     std::vector<int64_t> wg0;       // 2S + 1
-    std::vector<int64_t> key0, rs0; // per sample: first key, first region-stat word
-    int64_t keys = 0, npos = 0, nshp = 0, rstat = 0;
+    std::vector<int64_t> key0, rs0; // per sample: first shape key, first region-stat word
+    std::vector<int64_t> pkey0;     // first position key
+    int64_t keys = 0, pkeys = 0, npos = 0, nshp = 0, rstat = 0;
     int lds_regions = 0;
     // bound
     size_t off_segs = 0, off_wg0 = 0, param_bytes = 0;
     char *param_dev = nullptr;
     std::vector<char> param;
-    int32_t *pcnt = nullptr, *scnt = nullptr, *pstart = nullptr, *sstart = nullptr;
+    int32_t *pcnt = nullptr, *scnt = nullptr, *sstart = nullptr;
     int32_t *pfine = nullptr;  // positions: starts of the fine keys
     int32_t *sfine = nullptr;  // shapes: starts of the fine keys (cell << sbits) + part of the slab
-    int sbits = kSubBits;
+    int sbits = kSubBits, pbits = kSubBits;
     ScanBufs<int32_t> scan_p, scan_s;
     int2 *pkr = nullptr, *skr = nullptr;
     double *prec = nullptr, *srec = nullptr;
@@ -450,23 +455,41 @@ void prep_plan(PrepPlan &p, int S, const mia_sample *samples, const mia_bins &bi
     p.segs.assign(2 * S, PrepSeg{});
     p.wg0.assign(2 * S + 1, 0);
     p.key0.assign(S + 1, 0);
+    p.pkey0.assign(S + 1, 0);
     p.rs0.assign(S + 1, 0);
-    int kmax = 0;
+    int kmax = 0, mmax = 1;
+    int64_t pk = 0;
+    for (int s = 0; s < S; ++s) {
+        p.grids[s] = make_grid(samples[s], bins, tuning);
+        mmax = std::max(mmax, p.grids[s].m);
+        pk += p.grids[s].pkeys();
+    }
+    // the positions' line-of-sight parts: coarser for thinner columns, so that
+    // the fine keys stay of the order of the shapes'
+    p.pbits = mmax == 1 ? kSubBits : (mmax == 2 ? 4 : (mmax <= 4 ? 3 : 2));
+    while (p.pbits > 0 && (pk << p.pbits) >= (1ll << 31)) --p.pbits;
+    if (pk >= (1ll << 31))
+        for (Grid &g : p.grids) g.m = 1;
     for (int s = 0; s < S; ++s) {
         const mia_sample &m = samples[s];
-        Grid &g = p.grids[s] = make_grid(m, bins, tuning);
+        const Grid &g = p.grids[s];
         const int K = g.jk > 0 ? g.jk * g.jk * g.jk : 0;
         kmax = std::max(kmax, K);
         p.key0[s + 1] = p.key0[s] + g.keys();
+        p.pkey0[s + 1] = p.pkey0[s] + g.pkeys();
         p.rs0[s + 1] = p.rs0[s] + 2 * (int64_t)K;
         for (int kind = 0; kind < 2; ++kind) {
             PrepSeg &G = p.segs[2 * s + kind];
             std::memset(&G, 0, sizeof(G));
             G.n = kind ? m.n_shape : m.n_pos;
             G.obj0 = kind ? p.nshp : p.npos;
-            G.key0 = p.key0[s];
+            G.key0 = kind ? p.key0[s] : p.pkey0[s];
             G.g = g;
             G.kind = kind;
+            const int fine = kind ? 1 : g.m;
+            G.ncj = g.ncj * fine;
+            G.nc = g.nc * fine;
+            G.cw = g.cw / fine;
             G.K = K;
             G.sample = s;
             const int j = 2 * s + kind;
@@ -480,8 +503,9 @@ void prep_plan(PrepPlan &p, int S, const mia_sample *samples, const mia_bins &bi
                 "samples of one call hold more than 2^31 objects or cell keys");
     p.sbits = kSubBits;
     while (p.sbits > 0 && (p.key0[S] << p.sbits) >= (1ll << 31)) --p.sbits;
-    for (PrepSeg &G : p.segs) G.sbits = p.sbits;
+    for (PrepSeg &G : p.segs) G.sbits = G.kind ? p.sbits : p.pbits;
     p.keys = p.key0[S];
+    p.pkeys = p.pkey0[S];
     p.rstat = p.rs0[S];
     p.lds_regions = kmax <= kLdsRegions ? kmax : 0;
     p.kmax = kmax;
@@ -507,18 +531,17 @@ std::vector<SortedSample> prep_bind(PrepPlan &p, Carve &c, const mia_sample *sam
     p.param_bytes = pc.off;
     p.param_dev = c.take<char>(p.param_bytes);
     char *z0 = c.dry ? nullptr : c.base + c.off;
-    p.pcnt = c.take<int32_t>((p.keys << p.sbits) + 1);
+    p.pcnt = c.take<int32_t>((p.pkeys << p.pbits) + 1);
     p.scnt = c.take<int32_t>((p.keys << p.sbits) + 1);
     p.rcnt = c.take<unsigned long long>(p.rstat);
     p.rsum = c.take<double>(p.rstat);
     p.oor = c.take<int>(S);
     p.zero_begin = (unsigned long long *)z0;
     p.zero_words = c.dry ? 0 : (size_t)((c.base + c.off) - z0) / 8;
-    p.pstart = c.take<int32_t>(p.keys + 1);
-    p.pfine = c.take<int32_t>((p.keys << p.sbits) + 1);
+    p.pfine = c.take<int32_t>((p.pkeys << p.pbits) + 1);
     p.sstart = c.take<int32_t>(p.keys + 1);
     p.sfine = c.take<int32_t>((p.keys << p.sbits) + 1);
-    scan_carve<int32_t>(c, p.keys << p.sbits, p.scan_p);
+    scan_carve<int32_t>(c, p.pkeys << p.pbits, p.scan_p);
     scan_carve<int32_t>(c, p.keys << p.sbits, p.scan_s);
     p.pkr = c.take<int2>(p.npos);
     p.skr = c.take<int2>(p.nshp);
@@ -533,7 +556,8 @@ std::vector<SortedSample> prep_bind(PrepPlan &p, Carve &c, const mia_sample *sam
         size_t bytes = 0;
         MIA_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, (const int32_t *)nullptr, (int32_t *)nullptr,
                                                    (const int32_t *)nullptr, (int32_t *)nullptr, (int)nmax, 0,
-                                                   key_bits((p.keys << p.sbits) + 1), (hipStream_t)0));
+                                                   key_bits(std::max(p.keys << p.sbits, p.pkeys << p.pbits) + 1),
+                                                   (hipStream_t)0));
         p.dtmp_bytes = std::max<size_t>(bytes, 256);
         p.dtmp = c.take<char>(p.dtmp_bytes);
         p.dcell = c.take<double>(2 * (p.keys + 1));
@@ -549,12 +573,12 @@ std::vector<SortedSample> prep_bind(PrepPlan &p, Carve &c, const mia_sample *sam
         x.K = g.jk > 0 ? g.jk * g.jk * g.jk : 0;
         x.periodic = m.periodic;
         x.weighted = (m.pos_w != nullptr || m.shp_w != nullptr) ? 1 : 0;
+        x.pbits = p.pbits;
         if (c.dry) continue;
         x.prec = p.prec;
         x.srec = p.srec;
-        x.pstart = p.pstart + p.key0[s];
-        x.pfine = p.pfine + (p.key0[s] << p.sbits);
-        x.sbits = p.sbits;
+        x.pfine = p.pfine + (p.pkey0[s] << p.pbits);
+        x.flags = p.oor + s;
         x.sstart = p.sstart + p.key0[s];
         x.rcnt = p.rcnt + p.rs0[s];
         x.rsum = p.rsum + p.rs0[s];
@@ -600,10 +624,7 @@ void prep_enqueue(const PrepPlan &p, hipStream_t st) {
                            p.lds_regions);
         MIA_HIP(hipGetLastError());
     }
-    scan_ws<int32_t>(p.pcnt, p.pfine, p.keys << p.sbits, nullptr, p.scan_p, st);
-    hipLaunchKernelGGL(k_coarse_starts, dim3((unsigned)((p.keys + 1 + 255) / 256)), dim3(256), 0, st,
-                       (const int32_t *)p.pfine, p.keys, p.sbits, p.pstart);
-    MIA_HIP(hipGetLastError());
+    scan_ws<int32_t>(p.pcnt, p.pfine, p.pkeys << p.pbits, nullptr, p.scan_p, st);
     scan_ws<int32_t>(p.scnt, p.sfine, p.keys << p.sbits, nullptr, p.scan_s, st);
     hipLaunchKernelGGL(k_coarse_starts, dim3((unsigned)((p.keys + 1 + 255) / 256)), dim3(256), 0, st,
                        (const int32_t *)p.sfine, p.keys, p.sbits, p.sstart);
@@ -619,7 +640,7 @@ void prep_enqueue(const PrepPlan &p, hipStream_t st) {
             size_t bytes = p.dtmp_bytes;
             MIA_HIP(hipcub::DeviceRadixSort::SortPairs(p.dtmp, bytes, (const int32_t *)p.dkey, p.dkey_s,
                                                        (const int32_t *)p.didx, p.didx_s, (int)n, 0,
-                                                       key_bits((p.keys << p.sbits) + 1), st));
+                                                       key_bits((kind ? p.keys << p.sbits : p.pkeys << p.pbits) + 1), st));
             hipLaunchKernelGGL(k_stage_rank, dim3(g), dim3(256), 0, st, (const int32_t *)p.dkey_s,
                                (const int32_t *)p.didx_s, n, (const int32_t *)(kind ? p.sfine : p.pfine), kr);
             MIA_HIP(hipGetLastError());
@@ -846,16 +867,13 @@ void stage_release(Ctx &ctx) {
     ctx.ws_bytes = ctx.pinned_bytes = 0;
 }
 
-// After a count whose plan overflowed: larger item and range capacities for
-// the next attempt (a quarter of headroom over what the count needed).
+// After a count whose plan overflowed: a larger item capacity for the next attempt
+// (a quarter of headroom over what the count needed).
 void grow_caps(Ctx &ctx, const RunOut &r, int attempt) {
     if (attempt >= 3)
-        throw Error{MIA_E_UNSUPPORTED, "work items exceed the workspace capacity (" + std::to_string(r.words[3]) +
-                                           " items, " + std::to_string(std::max(r.words[7], r.words[8])) +
-                                           " range records)"};
+        throw Error{MIA_E_UNSUPPORTED,
+                    "work items exceed the workspace capacity (" + std::to_string(r.words[3]) + " items)"};
     ctx.item_cap = std::max<int64_t>(ctx.item_cap, (int64_t)(r.words[3] + r.words[3] / 4 + 1024));
-    const unsigned long long need = std::max(r.words[7], r.words[8]);
-    ctx.range_cap = std::max<int64_t>(ctx.range_cap, (int64_t)(need + need / 4 + 1024));
 }
 
 void stage_count(Ctx &ctx, int n, const mia_sample *samples, const mia_bins &bins, const mia_counts *outs,
@@ -868,20 +886,18 @@ void stage_count(Ctx &ctx, int n, const mia_sample *samples, const mia_bins &bin
         Carve dry;
         std::vector<SortedSample> proto = prep_bind(prep, dry, samples);
         const size_t pbytes = dry.off;
-        PlanPtr cp(plan_count(ctx, proto, bins, tuning, ctx.item_cap, ctx.range_cap, false));
+        PlanPtr cp(plan_count(ctx, proto, bins, tuning, ctx.item_cap, false));
         size_t total = pbytes + count_bytes(*cp);
         char *base;
         if (mode == STAGE_STATIC) {
             MIA_REQUIRE(ctx.scratch != nullptr, "no static workspace on this device");
             const size_t room = (size_t)stage_static_bytes();
             if (total > room) {
-                // fewer work-item slots (32 bytes each with their costs and
-                // scan) and ranges (24 bytes: planner range and item record),
-                // down to a floor; a count that needs more reports it
-                const int64_t over = (int64_t)((total - room) / 56) + 4096;
-                const int64_t cap = count_item_cap(*cp) - over, rcap = count_range_cap(*cp) - over;
-                if (cap >= 65536 && rcap >= 65536) {
-                    cp.reset(plan_count(ctx, proto, bins, tuning, cap, rcap, true));
+                // fewer work-item slots (48 bytes each with their costs and
+                // scan), down to a floor; a count that needs more reports it
+                const int64_t cap = count_item_cap(*cp) - ((int64_t)((total - room) / 48) + 4096);
+                if (cap >= 65536) {
+                    cp.reset(plan_count(ctx, proto, bins, tuning, cap, true));
                     total = pbytes + count_bytes(*cp);
                 }
             }
@@ -901,17 +917,14 @@ void stage_count(Ctx &ctx, int n, const mia_sample *samples, const mia_bins &bin
         RunOut r;
         upload_and_run(ctx, &prep, *cp, st, mode, r);
         for (int s = 0; s < n; ++s)
-            if (r.oor[s])
+            if (r.oor[s] & 1)
                 throw Error{MIA_E_RANGE, "coordinates outside [0, boxsize] (or NaN) in sample " + std::to_string(s)};
         if (r.words[2]) {
-            // more work items or range records than the capacity: grow it and count again
+            // more work items than the capacity: grow it and count again
             if (mode == STAGE_STATIC)
                 throw Error{MIA_E_UNSUPPORTED, "the count needs " + std::to_string(r.words[3]) +
-                                                   " work items and " +
-                                                   std::to_string(std::max(r.words[7], r.words[8])) +
-                                                   " range records; the static workspace holds " +
-                                                   std::to_string(count_item_cap(*cp)) + " and " +
-                                                   std::to_string(count_range_cap(*cp)) +
+                                                   " work items; the static workspace holds " +
+                                                   std::to_string(count_item_cap(*cp)) +
                                                    " (mia_count allocates what it needs)"};
             grow_caps(ctx, r, attempt);
             continue;
@@ -945,7 +958,7 @@ PreparedSample *stage_prepare(Ctx &ctx, const mia_sample &s, const mia_bins &bin
         int *flag = (int *)(stage + ((prep.param_bytes + 255) & ~(size_t)255));
         MIA_HIP(hipMemcpyAsync(flag, prep.oor, sizeof(int), hipMemcpyDeviceToHost, st));
         MIA_HIP(hipStreamSynchronize(st));
-        if (*flag) throw Error{MIA_E_RANGE, "coordinates outside [0, boxsize] (or NaN)"};
+        if (*flag & 1) throw Error{MIA_E_RANGE, "coordinates outside [0, boxsize] (or NaN)"};
         h->s = ss[0];
     } catch (...) {
         (void)hipFree(h->mem);
@@ -963,7 +976,7 @@ void stage_count_prepared(Ctx &ctx, int n, const PreparedSample *const *hs, cons
         ss[i] = hs[i]->s;
     }
     for (int attempt = 0;; ++attempt) {
-        PlanPtr cp(plan_count(ctx, ss, bins, tuning, ctx.item_cap, ctx.range_cap, false));
+        PlanPtr cp(plan_count(ctx, ss, bins, tuning, ctx.item_cap, false));
         Carve c;
         c.dry = false;
         c.base = (char *)workspace(ctx, count_bytes(*cp));
