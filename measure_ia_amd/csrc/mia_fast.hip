@@ -50,10 +50,13 @@ constexpr int kMaxWavesPerBlock = 4;
 constexpr int kThreads = kWave * kMaxWavesPerBlock;
 constexpr size_t kLdsBytes = 160 * 1024;         // LDS per CU (gfx950)
 constexpr size_t kPairStaticLds = 64;            // the pair kernel's own LDS words, at most
+constexpr int kStatCopies = 32, kStatStride = 16;  // copies of the pair kernel's statistics, words apart
 constexpr int kSharedBelow = 16;                 // private waves per CU below which histograms are shared
 constexpr int kPairWavesPerSimd = 6;             // waves per SIMD the pair kernel's registers allow
 constexpr int64_t kMaxKeysPerSample = 1 << 24;   // K^2 planner keys per sample (K regions)
 constexpr double kSinExact = 1e-5;  // FP64 arccos-domain check when |sin phi| < 1e-5 |cos phi|
+
+#define MIA_CONST __attribute__((address_space(4)))
 
 struct Block {
     int32_t s0, ns;
@@ -500,19 +503,24 @@ __global__ __launch_bounds__(kPlanThreads) void k_item_cost(const PlanSample *ps
     const int64_t n = *n_items;
     unsigned long long cand = 0;
     for (int64_t i = (int64_t)blockIdx.x * kPlanWaves + wv; i < n; i += (int64_t)gridDim.x * kPlanWaves) {
-        const Item it = items[i];
-        const Block &B = blocks[it.blk];
-        const ColumnView v = column_view(ps + B.sample);
+        // (wave-uniform: read through the scalar cache)
+        const MIA_CONST int32_t *ip = (const MIA_CONST int32_t *)items + 8 * i;
+        const int blk = ip[0], w = ip[1], jj = ip[2], wn = ip[3], c0 = ip[4], kk = ip[5];
+        const MIA_CONST int32_t *bp = (const MIA_CONST int32_t *)blocks + 6 * (int64_t)blk;
+        const MIA_CONST double *bc = (const MIA_CONST double *)bbox + 6 * (int64_t)blk;
+        const double bb[6] = {bc[0], bc[1], bc[2], bc[3], bc[4], bc[5]};
+        const int ns = bp[1];
         int pb, np;
-        item_column(v, bbox + 6 * (int64_t)it.blk, it.ja, it.jb, it.wb, it.nc, it.c0, it.k0, it.k1, (it.w >> 24) & 3,
-                    lane, pb, np);
+        item_column(column_view((const MIA_CONST PlanSample *)ps + bp[4]), bb, jj & 0xffff, (jj >> 16) & 0xffff,
+                    wn & 0xffff, (wn >> 16) & 0xffff, c0, kk & 0xffff, (kk >> 16) & 0xffff, (w >> 24) & 3, lane, pb,
+                    np);
         for (int d = kWave / 2; d > 0; d >>= 1) np += __shfl_xor(np, d);
         if (lane == 0) {
             items[i].np = np;
             // a wave pays for whole 64-lane position batches plus a fixed
             // per-item overhead, whatever the item's true pair count
-            cost[i] = (int64_t)B.ns * (((np + kWave - 1) / kWave) * kWave) + kItemOverhead;
-            cand += (unsigned long long)B.ns * np;
+            cost[i] = (int64_t)ns * (((np + kWave - 1) / kWave) * kWave) + kItemOverhead;
+            cand += (unsigned long long)ns * np;
         }
     }
     if (cand) atomicAdd(&cand_l, cand);
@@ -587,9 +595,31 @@ __global__ void k_gather_items(const int32_t *order, const int64_t *n_dev, const
     cost_out[i] = cost[o];
 }
 
+// The pair kernel's statistics, summed over their copies into the words the
+// host reads back (one wave).
+__device__ __forceinline__ void collect_stats(const unsigned long long *stat, unsigned long long *words) {
+    const int lane = threadIdx.x;
+    unsigned long long v[4] = {0, 0, 0, 0};
+    if (lane < kStatCopies)
+        for (int k = 0; k < 4; ++k) v[k] = stat[lane * kStatStride + k];
+    for (int d = kWave / 2; d > 0; d >>= 1)
+        for (int k = 0; k < 4; ++k) {
+            const unsigned long long o = __shfl_down(v[k], d);
+            v[k] = k < 2 ? v[k] + o : (o > v[k] ? o : v[k]);
+        }
+    if (lane == 0) {
+        words[0] = v[0];
+        words[6] = v[1];
+        words[4] = v[2];
+        words[5] = v[3];
+    }
+}
+
 // Caller outputs from the accumulators: counts, DD (the pair count itself for
 // unit weights), S+D, their tallies, SxD, the variance and the region stats.
-__global__ void k_finalize(const FinSample *fs, const int64_t *fin0, int S) {
+__global__ void k_finalize(const FinSample *fs, const int64_t *fin0, int S, const unsigned long long *stat,
+                           unsigned long long *words) {
+    if (blockIdx.x == 0 && threadIdx.x < kWave) collect_stats(stat, words);
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= fin0[S]) return;
     const int s = find_sample(fin0, S, i);
@@ -659,15 +689,99 @@ __device__ __forceinline__ void neumaier(double &s, double &c, double v) {
     s = t;
 }
 
-// Deterministic reduction, step 2: caller outputs from the slots.  Output
-// element (tally t, bin b) of a sample sums, in slot order, the slots of that
-// sample whose key (R_s, R_p) includes region t - 1 (every slot for t = 0),
-// with compensated FP64 sums; region stats as k_finalize.
-__global__ void k_finalize_det(const FinSample *fs, const int64_t *fin0, int S, const int64_t *slot_total,
-                               const int64_t *slot_key, const unsigned long long *slot_np,
-                               const double *slot_sp, const double *slot_sx, const double *slot_dd,
-                               const double *slot_var, int BO) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Deterministic reduction, step 2: the slots of one key are consecutive; the
+// first one (its head) takes their sum, and the second, where there is one, the
+// sum's compensation, bin by bin.
+__device__ __forceinline__ void sum_run(double *slot, int64_t o, int64_t step, int n) {
+    double s = slot[o], c = 0.0;
+    for (int k = 1; k < n; ++k) neumaier(s, c, slot[o + k * step]);
+    slot[o] = s;
+    slot[o + step] = c;
+}
+
+__global__ __launch_bounds__(256) void k_sum_slots(const int64_t *slot_total, const int64_t *slot_key,
+                                                   unsigned long long *slot_np, double *slot_sp, double *slot_sx,
+                                                   double *slot_dd, double *slot_var, int BO) {
+    const int64_t n = *slot_total;
+    for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
+        const int64_t key = slot_key[q];
+        if (q > 0 && slot_key[q - 1] == key) continue;
+        int run = 1;
+        while (q + run < n && slot_key[q + run] == key) ++run;
+        if (run == 1) continue;
+        for (int b = threadIdx.x; b < BO; b += blockDim.x) {
+            const int64_t o = q * BO + b;
+            unsigned long long c = slot_np[o];
+            for (int k = 1; k < run; ++k) c += slot_np[o + (int64_t)k * BO];
+            slot_np[o] = c;
+            sum_run(slot_sp, o, BO, run);
+            sum_run(slot_sx, o, BO, run);
+            if (slot_dd) sum_run(slot_dd, o, BO, run);
+            if (slot_var) sum_run(slot_var, o, BO, run);
+        }
+    }
+}
+
+// The heads in slot order: heads[i] = slot << 1 | whether a second slot follows,
+// *n_heads of them (one workgroup).
+__global__ __launch_bounds__(1024) void k_slot_heads(const int64_t *slot_total, const int64_t *slot_key,
+                                                     int64_t *heads, int64_t *n_heads) {
+    __shared__ int s_cnt[1024 / kWave];
+    const int64_t n = *slot_total;
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    int64_t base = 0;
+    for (int64_t q0 = 0; q0 < n; q0 += blockDim.x) {
+        const int64_t q = q0 + threadIdx.x;
+        const bool head = q < n && (q == 0 || slot_key[q - 1] != slot_key[q]);
+        const uint64_t m = __ballot(head);
+        if (lane == 0) s_cnt[wv] = __popcll(m);
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int k = 0; k < 1024 / kWave; ++k) {
+            before += k < wv ? s_cnt[k] : 0;
+            all += s_cnt[k];
+        }
+        if (head) {
+            const bool two = q + 1 < n && slot_key[q + 1] == slot_key[q];
+            heads[base + before + __popcll(m & ((1ull << lane) - 1))] = (q << 1) | (two ? 1 : 0);
+        }
+        base += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *n_heads = base;
+}
+
+// Step 3: caller outputs from the keys' sums, one wave per output.  Output
+// element (tally t, bin b) of a sample sums the heads of that sample whose key
+// (R_s, R_p) includes region t - 1 (every head for t = 0): lane l every 64th
+// from the l-th, then the lanes pairwise, all with compensated FP64 sums, in an
+// order fixed by the heads.  Region stats as k_finalize.  (One thread per
+// output over all slots took 8.5 ms for 8,000 slots of 200 bins and 28 tallies,
+// waiting on one slot after the other.)
+struct DetSum {
+    double s, c;
+    __device__ __forceinline__ void add(const double *slot, int64_t at, int64_t second) {
+        neumaier(s, c, slot[at]);
+        if (second >= 0) c += slot[second];
+    }
+    __device__ __forceinline__ void reduce() {
+        for (int d = kWave / 2; d > 0; d >>= 1) {
+            const double os = __shfl_down(s, d), oc = __shfl_down(c, d);
+            neumaier(s, c, os);
+            c += oc;
+        }
+    }
+};
+
+__global__ __launch_bounds__(256) void k_finalize_det(const FinSample *fs, const int64_t *fin0, int S,
+                                                      const int64_t *heads, const int64_t *n_heads,
+                                                      const int64_t *slot_key, const unsigned long long *slot_np,
+                                                      const double *slot_sp, const double *slot_sx,
+                                                      const double *slot_dd, const double *slot_var, int BO,
+                                                      const unsigned long long *stat, unsigned long long *words) {
+    if (blockIdx.x == 0 && threadIdx.x < kWave) collect_stats(stat, words);
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t i = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
     if (i >= fin0[S]) return;
     const int s = find_sample(fin0, S, i);
     const FinSample &F = fs[s];
@@ -675,7 +789,7 @@ __global__ void k_finalize_det(const FinSample *fs, const int64_t *fin0, int S, 
     const int64_t nb = (int64_t)(1 + F.K) * F.B;
     if (j >= nb) {
         const int64_t k = j - nb;  // region k < K
-        if (F.out.region_stats) {
+        if (F.out.region_stats && lane == 0) {
             double *r = F.out.region_stats + 4 * k;
             r[0] = (double)F.rcnt[k];
             r[1] = (double)F.rcnt[F.K + k];
@@ -685,38 +799,47 @@ __global__ void k_finalize_det(const FinSample *fs, const int64_t *fin0, int S, 
         return;
     }
     const int t = (int)(j / F.B), b = (int)(j % F.B);
-    // the sample's slots: keys [s << 32, (s + 1) << 32) of the ascending key list
-    const int64_t n = *slot_total;
-    int64_t lo = 0, hi = n;
-    while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (slot_key[mid] < ((int64_t)s << 32))
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
+    // the sample's heads: keys [s << 32, (s + 1) << 32) of the ascending key list
+    const int64_t n = *n_heads;
+    auto first_of = [&](int64_t key) {
+        int64_t lo = 0, hi = n;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if (slot_key[heads[mid] >> 1] < key)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        return lo;
+    };
+    const int64_t h0 = first_of((int64_t)s << 32), h1 = first_of((int64_t)(s + 1) << 32);
     unsigned long long c = 0;
-    double sp = 0.0, spc = 0.0, dd = 0.0, ddc = 0.0, sx = 0.0, sxc = 0.0, vr = 0.0, vrc = 0.0;
-    for (int64_t q = lo; q < n; ++q) {
-        const int64_t key = slot_key[q];
-        if ((key >> 32) != s) break;
+    DetSum sp{0.0, 0.0}, dd{0.0, 0.0}, sx{0.0, 0.0}, vr{0.0, 0.0};
+    for (int64_t h = h0 + lane; h < h1; h += kWave) {
+        const int64_t e = heads[h], key = slot_key[e >> 1];
         const int rs = (int)((key >> 16) & 0xffff), rp = (int)(key & 0xffff);
         if (t > 0 && rs != t - 1 && rp != t - 1) continue;
-        const int64_t o = q * BO + b;
-        c += slot_np[o];
-        neumaier(sp, spc, slot_sp[o]);
-        if (F.weighted) neumaier(dd, ddc, slot_dd[o]);
+        const int64_t at = (e >> 1) * BO + b, second = (e & 1) ? at + BO : -1;
+        c += slot_np[at];
+        sp.add(slot_sp, at, second);
+        if (F.weighted) dd.add(slot_dd, at, second);
         if (t == 0) {
-            neumaier(sx, sxc, slot_sx[o]);
-            if (F.var_on) neumaier(vr, vrc, slot_var[o]);
+            sx.add(slot_sx, at, second);
+            if (F.var_on) vr.add(slot_var, at, second);
         }
     }
+    for (int d = kWave / 2; d > 0; d >>= 1) c += __shfl_down(c, d);
+    sp.reduce();
+    dd.reduce();
+    sx.reduce();
+    vr.reduce();
+    if (lane) return;
     F.out.npairs[j] = c;
-    if (F.out.dd) F.out.dd[j] = F.weighted ? dd + ddc : (double)c;
-    F.out.splus[j] = sp + spc;
+    if (F.out.dd) F.out.dd[j] = F.weighted ? dd.s + dd.c : (double)c;
+    F.out.splus[j] = sp.s + sp.c;
     if (t == 0) {
-        F.out.scross[b] = sx + sxc;
-        if (F.out.variance) F.out.variance[b] = F.var_on ? vr + vrc : 0.0;
+        F.out.scross[b] = sx.s + sx.c;
+        if (F.out.variance) F.out.variance[b] = F.var_on ? vr.s + vr.c : 0.0;
     }
 }
 
@@ -747,10 +870,10 @@ struct PairArgs {
     int hist_stride;             // bytes of a histogram
     int shared, copies;          // the waves of a workgroup share `copies` histograms (else one per wave)
     int bin_off, nbins_out;      // this pass's first output bin (r0 * n_2) and the output's B
-    unsigned long long *rechecks;
-    // wall-clock span of the launch's busy waves: [0] max of ~start, [1] max of end
-    unsigned long long *clock;
-    unsigned long long *iterations;  // wave-iterations (a 64-lane position batch against one shape)
+    // kStatCopies copies of: pairs binned exactly, wave-iterations (a 64-lane
+    // position batch against one shape), and the wall-clock span of the busy
+    // workgroups: max of ~start, max of end
+    unsigned long long *stat;
     // deterministic reduction: the j-th histogram flush of wave w goes to
     // slot slot0[w] + j (all output bins of the pass, plain stores) with its
     // planner key; k_finalize_det sums the slots in slot order
@@ -889,7 +1012,6 @@ __device__ __forceinline__ int edge_near(const double *E, int n, double v, doubl
     return e - 1 + (E[e] <= v ? 1 : 0);
 }
 
-#define MIA_CONST __attribute__((address_space(4)))
 
 // Per-sample values the pair loop needs, read once per item through the
 // scalar cache (they are wave-uniform and end up in SGPRs).
@@ -1217,7 +1339,8 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
 template <int MODE, bool WEIGHTED, bool VAR>
 __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs P) {
     extern __shared__ __align__(16) char lds[];
-    __shared__ int s_next[2], s_chunk;
+    __shared__ int s_next[2], s_chunk, s_left;
+    __shared__ unsigned long long s_stat[3];
     const int lane = threadIdx.x & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const bool shared = P.shared != 0;
@@ -1232,7 +1355,14 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     char *hist0 = lds + thr_bytes;
     const int nhist = shared ? P.copies : (int)(blockDim.x / kWave);
     for (int i = threadIdx.x * 4; i < nhist * P.hist_stride; i += blockDim.x * 4) *(uint32_t *)(hist0 + i) = 0u;
-    if (threadIdx.x < 2) s_next[threadIdx.x] = 0;
+    if (threadIdx.x < 2) {
+        s_next[threadIdx.x] = 0;
+        s_stat[threadIdx.x] = 0;
+    }
+    if (threadIdx.x == 0) {
+        s_left = blockDim.x / kWave;
+        s_stat[2] = wall_clock64();
+    }
     __syncthreads();
 
     // runs of neighbouring items of the key-sorted list (which read the same
@@ -1242,8 +1372,6 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     const int wave = wg * wpb + wv;
     // a plan that overflowed its capacities is counted again by the host
     if (n_items == 0 || *(const MIA_CONST unsigned long long *)P.overflow) return;
-    if (!shared && wave >= P.n_waves) return;
-    if (lane == 0) atomicMax(&P.clock[0], ~(unsigned long long)wall_clock64());
     const int tid = shared ? threadIdx.x : lane, nthr = shared ? blockDim.x : kWave;
     char *hist = hist0 + (shared ? 0 : wv * P.hist_stride);
     const int place = ((lane & 7) << 3) | (lane >> 3);
@@ -1251,7 +1379,10 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     // a contiguous share of the cost-sorted items, then tail chunks from the counter
     const WaveSchedule sch = make_schedule(P.bounds, shared ? (int)gridDim.x : P.n_waves);
     int64_t it0, it1;
-    sch.first(shared ? wg : wave, it0, it1);
+    sch.first(shared ? wg : (wave < P.n_waves ? wave : 0), it0, it1);
+    if (!shared && wave >= P.n_waves) it1 = it0;
+    it0 = uniform64(it0);
+    it1 = uniform64(it1);
     const MIA_CONST int32_t *items = (const MIA_CONST int32_t *)P.items;
     const MIA_CONST int32_t *blocks = (const MIA_CONST int32_t *)P.blocks;
     int cur_key = -1, flushes = 0, par = 0;
@@ -1336,7 +1467,7 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
             it = se;
         }
         if (!shared) {
-            if (!sch.next(P.queue, lane, it0, it1)) break;
+            if (wave >= P.n_waves || !sch.next(P.queue, lane, it0, it1)) break;
         } else {
             if (sch.tail == 0) break;
             if (threadIdx.x == 0) s_chunk = atomicAdd(P.queue, 1);
@@ -1347,10 +1478,19 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
         }
     }
     turn_to(-1);
-    if (nre) atomicAdd(P.rechecks, (unsigned long long)nre);
+    // Statistics: the last wave of the workgroup adds them, to one of
+    // kStatCopies copies a cache line apart (four atomics of every wave on one
+    // line took 0.1 ms of a count of 2,000 galaxies).
+    if (nre) atomicAdd(&s_stat[0], (unsigned long long)nre);
     if (lane == 0) {
-        if (iterations) atomicAdd(P.iterations, (unsigned long long)iterations);
-        atomicMax(&P.clock[1], (unsigned long long)wall_clock64());
+        if (iterations) atomicAdd(&s_stat[1], (unsigned long long)iterations);
+        if (__hip_atomic_fetch_add(&s_left, -1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 1 && s_stat[1]) {
+            unsigned long long *st = P.stat + (wg % kStatCopies) * kStatStride;
+            atomicAdd(&st[0], s_stat[0]);
+            atomicAdd(&st[1], s_stat[1]);
+            atomicMax(&st[2], ~s_stat[2]);
+            atomicMax(&st[3], (unsigned long long)wall_clock64());
+        }
     }
 }
 
@@ -1644,8 +1784,10 @@ struct CountPlan {
     double *bbox = nullptr;
     uint32_t *geo = nullptr;
     unsigned long long *words = nullptr;   // [kCountReadback] read back after the count
+    unsigned long long *stat = nullptr;    // the pair kernel's statistics, kStatCopies copies
     int *queue = nullptr;
     unsigned long long *acc = nullptr;
+    int64_t *heads = nullptr, *n_heads = nullptr;
     int64_t *runs = nullptr, *slot0 = nullptr, *slot_key = nullptr, *ne = nullptr, *ne_pre = nullptr;
     unsigned long long *skey = nullptr, *skey2 = nullptr;   // deterministic item order
     int32_t *sidx = nullptr, *sidx2 = nullptr;
@@ -1854,6 +1996,7 @@ void count_bind(CountPlan &p, Carve &c, const std::vector<SortedSample> &ss, con
     p.kc = c.take<unsigned long long>(p.nkeys + 1);
     p.kcur = c.take<unsigned long long>(p.nkeys + 1);
     p.words = c.take<unsigned long long>(kCountReadback);
+    p.stat = c.take<unsigned long long>(kStatCopies * kStatStride);
     p.queue = c.take<int>(kMaxBinsR);
     p.zero_begin = (unsigned long long *)z0;
     p.zero_words = dry ? 0 : (size_t)((c.base + c.off) - z0) / 8;
@@ -1882,6 +2025,8 @@ void count_bind(CountPlan &p, Carve &c, const std::vector<SortedSample> &ss, con
         p.ne_pre = c.take<int64_t>(p.nkeys + 1);
         scan_carve<int64_t>(c, p.nkeys, p.scan_ne);
         p.slot_key = c.take<int64_t>(p.slot_cap);
+        p.heads = c.take<int64_t>(p.slot_cap);
+        p.n_heads = c.take<int64_t>(1);
         p.slot_np = c.take<unsigned long long>(sw);
         p.slot_sp = c.take<double>(sw);
         p.slot_sx = c.take<double>(sw);
@@ -2053,9 +2198,7 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
     A.T = (const double *)(pd + p.off_T);
     A.X = (const double *)(pd + p.off_X);
     A.samples = (const SampleDev *)(pd + p.off_sd);
-    A.rechecks = p.words;
-    A.clock = p.words + 4;
-    A.iterations = p.words + 6;
+    A.stat = p.stat;
     A.det = p.det ? 1 : 0;
     A.K1 = p.K1;
     A.slot_cap = p.slot_cap;
@@ -2083,15 +2226,25 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
             launch_pairs_mode<MIA_RMU>(A, p.pc.grid, p.pc.wpb, p.pc.lds, st);
     }
     if (ev) MIA_HIP(hipEventRecord(ev[2], st));
-    if (p.det)
-        hipLaunchKernelGGL(k_finalize_det, dim3(nblk(p.fin_total, 256)), dim3(256), 0, st,
-                           (const FinSample *)(pd + p.off_fs), fin0, S, (const int64_t *)(p.slot0 + p.pc.waves),
-                           (const int64_t *)p.slot_key, (const unsigned long long *)p.slot_np,
-                           (const double *)p.slot_sp, (const double *)p.slot_sx, (const double *)p.slot_dd,
-                           (const double *)p.slot_var, n_r * n_2);
-    else
+    if (p.det) {
+        const int64_t *slots = p.slot0 + p.pc.waves;  // their number
+        const unsigned sgrid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(p.slot_cap, 8192));
+        hipLaunchKernelGGL(k_sum_slots, dim3(sgrid), dim3(256), 0, st, slots, (const int64_t *)p.slot_key, p.slot_np,
+                           p.slot_sp, p.slot_sx, p.slot_dd, p.slot_var, n_r * n_2);
+        MIA_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_slot_heads, dim3(1), dim3(1024), 0, st, slots, (const int64_t *)p.slot_key, p.heads,
+                           p.n_heads);
+        MIA_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_finalize_det, dim3(nblk(p.fin_total, 256 / kWave)), dim3(256), 0, st,
+                           (const FinSample *)(pd + p.off_fs), fin0, S, (const int64_t *)p.heads,
+                           (const int64_t *)p.n_heads, (const int64_t *)p.slot_key,
+                           (const unsigned long long *)p.slot_np, (const double *)p.slot_sp, (const double *)p.slot_sx,
+                           (const double *)p.slot_dd, (const double *)p.slot_var, n_r * n_2,
+                           (const unsigned long long *)p.stat, p.words);
+    } else {
         hipLaunchKernelGGL(k_finalize, dim3(nblk(p.fin_total, 256)), dim3(256), 0, st,
-                           (const FinSample *)(pd + p.off_fs), fin0, S);
+                           (const FinSample *)(pd + p.off_fs), fin0, S, (const unsigned long long *)p.stat, p.words);
+    }
     MIA_HIP(hipGetLastError());
     if (ev) MIA_HIP(hipEventRecord(ev[3], st));
 }
