@@ -409,6 +409,13 @@ __device__ __forceinline__ int strict_axis_index(double x, double Lsub, int jk) 
     return -1;
 }
 
+// A wave-uniform value in scalar registers.
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
 // The reference's minimum-image wrap (measure_w_box_jk.py:160-162).
 __device__ __forceinline__ double wrap_sep(double d, double L, double half) {
     if (d > half) d -= L;

@@ -1253,9 +1253,9 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
     walk.begin(lane, cpb, cn);
     const int nb = walk.nb;
     iterations += (uint64_t)nb * ns;
-    // the slot past the last bin takes the zeros of the empty run
+    // an empty run adds its zeros to some bin, another one for every lane
     const uint32_t row = (uint32_t)(P.n_2 * sizeof(Slot<WEIGHTED, VAR>));
-    Pend pd{hist + (uint32_t)(P.nbins * sizeof(Slot<WEIGHTED, VAR>)), 0, 0, 0, 0, 0};
+    Pend pd{hist + (uint32_t)((lane < P.nbins ? lane : 0) * sizeof(Slot<WEIGHTED, VAR>)), 0, 0, 0, 0, 0};
     // positions are loaded one batch ahead
     bool vn;
     const double2 *prn = (const double2 *)(S.prec + 4 * (int64_t)walk.position(0, lane, vn));
@@ -1320,12 +1320,6 @@ __device__ __forceinline__ void run_shifted(const PairArgs &P, const SampleView 
     else
         run_item<MODE, SH_NONE, WEIGHTED, VAR, LZ>(P, S, cpb, cn, shifts, shp, ns, hist, T, X, lane, nre,
                                                    iterations);
-}
-
-__device__ __forceinline__ int64_t uniform64(int64_t v) {
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
 // Persistent groups of waves over the cost-balanced, key-sorted items.  A group
@@ -1517,7 +1511,7 @@ void launch_pairs_mode(const PairArgs &A, unsigned grid, int wpb, size_t lds, hi
 
 // LDS bytes of one wave's histogram (one copy) and of the block's thresholds.
 size_t wave_hist_bytes(const mia_bins &bins, bool weighted) {
-    return (((size_t)bins.n_r * bins.n_2 + 1) * slot_bytes(weighted, bins.accumulate_variance) + 15) & ~(size_t)15;
+    return ((size_t)bins.n_r * bins.n_2 * slot_bytes(weighted, bins.accumulate_variance) + 15) & ~(size_t)15;
 }
 
 size_t threshold_bytes(const mia_bins &bins) {
@@ -1677,8 +1671,7 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     // one histogram copy per wave: the pending-slot registers already absorb
     // most same-address collisions, and one copy leaves LDS for 8 waves per
     // SIMD (2 copies measured 20 % slower); mia_tuning.hist_copies is ignored
-    // (and the slot an empty pending run adds its zeros to)
-    A.hist_stride = (int)((((size_t)Bp + 1) * slot_bytes(A.weighted, A.var) + 15) & ~(size_t)15);
+    A.hist_stride = (int)(((size_t)Bp * slot_bytes(A.weighted, A.var) + 15) & ~(size_t)15);
     // A private histogram per wave (one copy: the pending-slot registers already
     // absorb most same-address collisions), or one per workgroup, shared by its
     // four waves, in as many copies (at most 4) as leave room for

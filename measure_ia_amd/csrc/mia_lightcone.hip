@@ -57,7 +57,7 @@ namespace {
 
 constexpr int kLcWavesPerBlock = 4;
 constexpr int kLcThreads = kWave * kLcWavesPerBlock;
-constexpr size_t kLcLds = 160 * 1024;
+constexpr size_t kLcLds = 160 * 1024 - 64;  // LDS per CU (gfx950) less the pair kernel's own words
 constexpr double kPiC = 3.141592653589793;  // numpy's np.pi
 constexpr double kDeg = kPiC / 180.0;
 constexpr int kLcMaxPatches = 4096;           // patch pairs stay below 2^24 keys
@@ -673,7 +673,7 @@ struct LcPairArgs {
     float lgs, lgc, xs, xc, dr, d2;
     int scan;                    // 1: the exact path scans every threshold (guard band of a whole bin)
     int bin_off, nbins_out;      // this pass's first output bin; bins per output row (B)
-    int hist_stride, off_dd, off_sp, off_sx;
+    int hist_stride;
     unsigned long long *npairs;  // (1+P)*B
     double *dd, *sp, *sx;        // (1+P)*B (sp, sx NULL for pair counts)
     unsigned long long *rechecks;
@@ -682,39 +682,67 @@ struct LcPairArgs {
 typedef const __attribute__((address_space(4))) double *CPtrD;
 typedef const __attribute__((address_space(4))) int32_t *CPtrI;
 
+#define MIA_LDS __attribute__((address_space(3)))
+
+// One bin of a wave's histogram: the pair count, with shapes S+D and SxD, with
+// weights DD (unit weights: DD is the count itself, so random-random counts
+// touch four bytes per bin).  A pending run keeps its slot's address and the
+// fields lie at constant offsets from it.
+template <bool SHAPES, bool WEIGHTED>
+struct LcSlot {
+    double v[(SHAPES ? 2 : 0) + (WEIGHTED ? 1 : 0)];  // [S+D, SxD], [DD]
+    uint32_t c, pad;
+};
+template <>
+struct LcSlot<false, false> {
+    uint32_t c;
+};
+static_assert(sizeof(LcSlot<false, false>) == 4 && sizeof(LcSlot<true, false>) == 24 &&
+                  sizeof(LcSlot<true, true>) == 32 && sizeof(LcSlot<false, true>) == 16,
+              "LcSlot layout");
+constexpr size_t lc_slot_bytes(bool shapes, bool weighted) {
+    return shapes || weighted ? 8 + (shapes ? 16 : 0) + (weighted ? 8 : 0) : 4;
+}
+
 struct LcPend {
-    int b;
+    uint32_t at;  // LDS address of the slot
     uint32_t c;
     double dd, sp, sx;
 };
 
-template <bool SHAPES>
-__device__ __forceinline__ void lc_hist_add(const LcPairArgs &P, char *hist, const LcPend &p) {
-    atomicAdd(&((uint32_t *)hist)[p.b], p.c);
-    atomicAdd(&((double *)(hist + P.off_dd))[p.b], p.dd);
-    if (SHAPES) {
-        atomicAdd(&((double *)(hist + P.off_sp))[p.b], p.sp);
-        atomicAdd(&((double *)(hist + P.off_sx))[p.b], p.sx);
-    }
+template <class T>
+__device__ __forceinline__ void lds_add(MIA_LDS T *p, T v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-template <bool SHAPES>
+template <bool SHAPES, bool WEIGHTED>
+__device__ __forceinline__ void lc_hist_add(const LcPend &p) {
+    typedef MIA_LDS LcSlot<SHAPES, WEIGHTED> S;
+    S *s = (S *)p.at;
+    lds_add(&s->c, p.c);
+    if constexpr (SHAPES) {
+        lds_add(&s->v[0], p.sp);
+        lds_add(&s->v[1], p.sx);
+    }
+    if constexpr (WEIGHTED) lds_add(&s->v[SHAPES ? 2 : 0], p.dd);
+}
+
+template <bool SHAPES, bool WEIGHTED>
 __device__ void lc_flush(const LcPairArgs &P, char *hist, int pn, int ps, int lane) {
-    uint32_t *cnt = (uint32_t *)hist;
-    double *hdd = (double *)(hist + P.off_dd);
-    double *hsp = (double *)(hist + P.off_sp);
-    double *hsx = (double *)(hist + P.off_sx);
+    typedef LcSlot<SHAPES, WEIGHTED> Slot;
+    Slot *slots = (Slot *)hist;
     const int B = P.nbins, BO = P.nbins_out;
     for (int b = lane; b < B; b += kWave) {
-        uint32_t c = cnt[b];
+        const Slot t = slots[b];
+        const uint32_t c = t.c;
         if (c == 0) continue;
-        double vdd = hdd[b], vsp = SHAPES ? hsp[b] : 0.0, vsx = SHAPES ? hsx[b] : 0.0;
-        cnt[b] = 0;
-        hdd[b] = 0.0;
-        if (SHAPES) {
-            hsp[b] = 0.0;
-            hsx[b] = 0.0;
+        slots[b] = Slot{};
+        double vsp = 0.0, vsx = 0.0, vdd = (double)c;
+        if constexpr (SHAPES) {
+            vsp = t.v[0];
+            vsx = t.v[1];
         }
+        if constexpr (WEIGHTED) vdd = t.v[SHAPES ? 2 : 0];
         int tgt[3] = {0, -1, -1};
         if (P.P > 0) {
             tgt[1] = 1 + pn;
@@ -751,11 +779,11 @@ __device__ __forceinline__ int lc_edge_near(const double *E, int n, double v, fl
     return e - 1 + (E[e] <= v ? 1 : 0);
 }
 
-template <int MODE, bool SHAPES>
+template <int MODE, bool SHAPES, bool WEIGHTED>
 __device__ __forceinline__ void lc_pair(const LcPairArgs &P, bool valid, double qra, double qdec,
                                         double qchi, double qc2, double qs2, double qw, double pra,
                                         double pdec, double pchi, double pax, double pay, double pw,
-                                        double pcos, char *hist, const double *T, const double *X,
+                                        double pcos, uint32_t hist, uint32_t row, const double *T, const double *X,
                                         uint32_t &nre, LcPend &pd, float vlgc, float vxc) {
     const int n_r = P.n_r, n_2 = P.n_2;
     const double dra = qra - pra, ddec = qdec - pdec;
@@ -776,9 +804,11 @@ __device__ __forceinline__ void lc_pair(const LcPairArgs &P, bool valid, double 
     float rv32 = (float)rv, pif = (float)pi;
     float gr = __fmaf_rn(__log2f(rv32), P.lgs, vlgc);
     float g2 = MODE == MIA_RPPI ? __fmaf_rn(pif, P.xs, vxc)
-                                : __fmaf_rn(pif, __builtin_amdgcn_rsqf(rv32), 1.0f) * P.xs;
+                                : __fmaf_rn(__fmaf_rn(pif, __builtin_amdgcn_rsqf(rv32), 1.0f), P.xs, vxc);
     int ir = (int)gr, i2 = (int)g2;
-    bool near = ((int)(fabsf(gr - rintf(gr)) < P.dr) | (int)(fabsf(g2 - rintf(g2)) < P.d2)) != 0;
+    // the guesses are raised by half their guard band: close to an edge, on
+    // either side, the fraction is below the whole band
+    bool near = ((int)(__builtin_amdgcn_fractf(gr) < P.dr) | (int)(__builtin_amdgcn_fractf(g2) < P.d2)) != 0;
     if (MODE == MIA_RMU) near |= s * (P.h * P.h) <= P.cut_hi;
     if (near) {
         // the reference's operation order (measure_w_lightcone.py:143-150)
@@ -811,33 +841,40 @@ __device__ __forceinline__ void lc_pair(const LcPairArgs &P, bool valid, double 
         const double B2 = 2.0 * dx * dy;
         const double r0 = __builtin_amdgcn_rcp(s);
         const double inv = fma(r0, fma(-s, r0, 1.0), r0);
-        ep = fma(qc2, A, qs2 * B2) * inv * pw;
-        ex = fma(qs2, A, -(qc2 * B2)) * inv * pw;
+        ep = fma(qc2, A, qs2 * B2) * inv;
+        ex = fma(qs2, A, -(qc2 * B2)) * inv;
+        if (WEIGHTED) {
+            ep = ep * pw;
+            ex = ex * pw;
+        }
         if (MODE == MIA_RMU && !(s > 0.0)) {
             // zero projected separation (only reachable with rp_cut < 0): NaN e+ -> 0
             ep = 0.0;
             ex = 0.0;
         }
     }
-    const int b = __mul24(ir, n_2) + i2;
+    const uint32_t at = __umul24(ir, row) + (__umul24(i2, (uint32_t)sizeof(LcSlot<SHAPES, WEIGHTED>)) + hist);
     // a new slot flushes the pending run, which then restarts from this pair:
     // keep = 0 drops the old sums (fma(0, sum, x) = x and fma(1, sum, x) =
     // sum + x, exactly as the plain assignment and addition)
-    const bool nw = b != pd.b;
-    if (nw & (pd.b >= 0)) lc_hist_add<SHAPES>(P, hist, pd);
-    const double keep = nw ? 0.0 : 1.0;
-    pd.b = b;
+    const bool nw = at != pd.at;
+    if (nw) lc_hist_add<SHAPES, WEIGHTED>(pd);
+    pd.at = at;
     pd.c = (nw ? 0u : pd.c) + 1u;
-    pd.dd = fma_into(keep, pd.dd, pw * qw);
-    if (SHAPES) {
-        pd.sp = fma_into(keep, pd.sp, ep);
-        pd.sx = fma_into(keep, pd.sx, ex);
+    if (SHAPES || WEIGHTED) {
+        const double keep = nw ? 0.0 : 1.0;
+        if (WEIGHTED) pd.dd = fma_into(keep, pd.dd, pw * qw);
+        if (SHAPES) {
+            pd.sp = fma_into(keep, pd.sp, ep);
+            pd.sx = fma_into(keep, pd.sx, ex);
+        }
     }
 }
 
-template <int MODE, bool SHAPES>
-__global__ __launch_bounds__(kLcThreads) void k_lc_pairs(LcPairArgs P) {
+template <int MODE, bool SHAPES, bool WEIGHTED>
+__global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
     extern __shared__ __align__(16) char lds[];
+    __shared__ unsigned int s_nre, s_left;
     const int lane = threadIdx.x & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     double *T = (double *)lds;
@@ -848,16 +885,26 @@ __global__ __launch_bounds__(kLcThreads) void k_lc_pairs(LcPairArgs P) {
     const size_t thr_bytes = ((size_t)(P.n_r + 1 + nx) * 8 + 15) & ~(size_t)15;
     char *hist = lds + thr_bytes + (size_t)wv * P.hist_stride;
     for (int i = lane * 4; i < P.hist_stride; i += kWave * 4) *(uint32_t *)(hist + i) = 0u;
+    if (threadIdx.x == 0) {
+        s_nre = 0;
+        s_left = blockDim.x / kWave;
+    }
     __syncthreads();
+    const uint32_t hist_at = (uint32_t)(uintptr_t)(MIA_LDS char *)hist;
+    const uint32_t row = (uint32_t)(P.n_2 * sizeof(LcSlot<SHAPES, WEIGHTED>));
+    // an empty run adds its zeros to some bin, another one for every lane
+    const uint32_t none = hist_at + (uint32_t)((lane < P.nbins ? lane : 0) * sizeof(LcSlot<SHAPES, WEIGHTED>));
 
     // runs of neighbouring items of the patch-sorted list (which read the
     // same position blocks) stay on one XCD
     const int w = xcd_run_block() * (blockDim.x / kWave) + wv;
-    if (w >= P.n_waves || P.n_items == 0) return;
+    if (P.n_items == 0) return;
+    const bool idle = w >= P.n_waves;
     // a contiguous share of the patch-sorted items, then tail chunks from the counter
     const WaveSchedule sch = make_schedule(P.bounds, P.n_waves);
     int64_t it0, it1;
-    sch.first(w, it0, it1);
+    sch.first(idle ? 0 : w, it0, it1);
+    if (idle) it1 = it0;
     CPtrI items = (CPtrI)P.items;
     CPtrI blocks = (CPtrI)P.blocks;
     CPtrI ranges = (CPtrI)P.ranges;
@@ -869,7 +916,10 @@ __global__ __launch_bounds__(kLcThreads) void k_lc_pairs(LcPairArgs P) {
     asm volatile("v_mov_b32 %0, %1" : "=v"(vlgc) : "s"(P.lgc));
     asm volatile("v_mov_b32 %0, %1" : "=v"(vxc) : "s"(P.xc));
     do {
-        for (int64_t i = it0; i < it1; ++i) {
+        for (int64_t j0 = it0; j0 < it1; ++j0) {
+            // (the compiler does not see that the item is wave-uniform; vector
+            // loads of the position records made the kernel twice as slow)
+            const int64_t i = uniform64(j0);
             CPtrI ip = items + 4 * i;
             const int blk = ip[0], r0 = ip[1], nr = ip[2], ns = ip[3];
             CPtrI bp = blocks + 8 * (int64_t)blk;
@@ -877,12 +927,12 @@ __global__ __launch_bounds__(kLcThreads) void k_lc_pairs(LcPairArgs P) {
             const int ps = ranges[4 * (int64_t)r0 + 2];
             if (pn != cur_pn || ps != cur_ps) {
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                if (cur_pn >= 0) lc_flush<SHAPES>(P, hist, cur_pn, cur_ps, lane);
+                if (cur_pn >= 0) lc_flush<SHAPES, WEIGHTED>(P, hist, cur_pn, cur_ps, lane);
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 cur_pn = pn;
                 cur_ps = ps;
             }
-            LcPend pd{-1, 0, 0.0, 0.0, 0.0};
+            LcPend pd{none, 0, 0.0, 0.0, 0.0};
             int j = r0, o = 0;
             const int jend = r0 + nr;
             for (int done = 0; done < ns; done += kWave) {
@@ -922,8 +972,8 @@ __global__ __launch_bounds__(kLcThreads) void k_lc_pairs(LcPairArgs P) {
                         const double *rn = P.prec + 8 * ((int64_t)p0 + (vn ? kn : 0));
                         const double b0 = rn[0], b1 = rn[1], b2 = rn[2], b3 = rn[3], b4 = rn[4], b5 = rn[5],
                                      b6 = rn[6];
-                        lc_pair<MODE, SHAPES>(P, v, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5, a6,
-                                              hist, T, X, nre, pd, vlgc, vxc);
+                        lc_pair<MODE, SHAPES, WEIGHTED>(P, v, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5, a6,
+                                              hist_at, row, T, X, nre, pd, vlgc, vxc);
                         a0 = b0;
                         a1 = b1;
                         a2 = b2;
@@ -955,13 +1005,13 @@ __global__ __launch_bounds__(kLcThreads) void k_lc_pairs(LcPairArgs P) {
                     CPtrD r1 = (CPtrD)((CPtrC)pr + (ob + 64u));
                     const double b0 = r1[0], b1 = r1[1], b2 = r1[2], b3 = r1[3], b4 = r1[4], b5 = r1[5],
                                  b6 = r1[6];
-                    lc_pair<MODE, SHAPES>(P, valid, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5,
-                                          a6, hist, T, X, nre, pd, vlgc, vxc);
+                    lc_pair<MODE, SHAPES, WEIGHTED>(P, valid, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5,
+                                          a6, hist_at, row, T, X, nre, pd, vlgc, vxc);
                     CPtrD r2 = (CPtrD)((CPtrC)pr + (ob + 128u < olast ? ob + 128u : olast));
                     const double c0 = r2[0], c1 = r2[1], c2 = r2[2], c3 = r2[3], c4 = r2[4], c5 = r2[5],
                                  c6 = r2[6];
-                    lc_pair<MODE, SHAPES>(P, valid, qra, qdec, qchi, qc2, qs2, qw, b0, b1, b2, b3, b4, b5,
-                                          b6, hist, T, X, nre, pd, vlgc, vxc);
+                    lc_pair<MODE, SHAPES, WEIGHTED>(P, valid, qra, qdec, qchi, qc2, qs2, qw, b0, b1, b2, b3, b4, b5,
+                                          b6, hist_at, row, T, X, nre, pd, vlgc, vxc);
                     a0 = c0;
                     a1 = c1;
                     a2 = c2;
@@ -971,23 +1021,29 @@ __global__ __launch_bounds__(kLcThreads) void k_lc_pairs(LcPairArgs P) {
                     a6 = c6;
                 }
                 if (k < np)
-                    lc_pair<MODE, SHAPES>(P, valid, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5,
-                                          a6, hist, T, X, nre, pd, vlgc, vxc);
+                    lc_pair<MODE, SHAPES, WEIGHTED>(P, valid, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5,
+                                          a6, hist_at, row, T, X, nre, pd, vlgc, vxc);
             }
-            if (pd.b >= 0) lc_hist_add<SHAPES>(P, hist, pd);
+            lc_hist_add<SHAPES, WEIGHTED>(pd);
         }
-    } while (sch.next(P.queue, lane, it0, it1));
+    } while (!idle && sch.next(P.queue, lane, it0, it1));
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    if (cur_pn >= 0) lc_flush<SHAPES>(P, hist, cur_pn, cur_ps, lane);
-    if (nre) atomicAdd(P.rechecks, (unsigned long long)nre);
+    if (cur_pn >= 0) lc_flush<SHAPES, WEIGHTED>(P, hist, cur_pn, cur_ps, lane);
+    // the last wave of the workgroup adds its statistics: one atomic each on a
+    // word that all workgroups share
+    if (nre) atomicAdd(&s_nre, nre);
+    if (lane == 0 && __hip_atomic_fetch_add(&s_left, -1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 1u && s_nre)
+        atomicAdd(P.rechecks, (unsigned long long)s_nre);
 }
 
-template <int MODE, bool SHAPES>
-void lc_launch(const LcPairArgs &A, unsigned grid, int wpb, size_t lds, hipStream_t st) {
-    MIA_HIP(hipFuncSetAttribute((const void *)k_lc_pairs<MODE, SHAPES>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_lc_pairs<MODE, SHAPES>), dim3(grid), dim3(kWave * wpb), lds, st, A);
-    MIA_HIP(hipGetLastError());
+// The pair kernel of a count.
+template <int M>
+const void *lc_kernel(bool shapes, bool weighted) {
+    return shapes ? (weighted ? (const void *)k_lc_pairs<M, true, true> : (const void *)k_lc_pairs<M, true, false>)
+                  : (weighted ? (const void *)k_lc_pairs<M, false, true> : (const void *)k_lc_pairs<M, false, false>);
+}
+const void *lc_kernel(int mode, bool shapes, bool weighted) {
+    return mode == MIA_RPPI ? lc_kernel<MIA_RPPI>(shapes, weighted) : lc_kernel<MIA_RMU>(shapes, weighted);
 }
 
 inline unsigned nblk_(int64_t n, int t) {
@@ -1051,10 +1107,9 @@ void lc_segments(Ctx &ctx, const uint64_t *key, int64_t n, const std::string &ta
     *flags_scan = id;
 }
 
-size_t lc_hist_bytes(int B, bool shapes) {
-    size_t off = ((size_t)4 * B + 15) & ~(size_t)15;
-    off += (size_t)8 * B * (shapes ? 3 : 1);
-    return (off + 15) & ~(size_t)15;
+// A histogram of B bins.
+size_t lc_hist_bytes(int B, bool shapes, bool weighted) {
+    return ((size_t)B * lc_slot_bytes(shapes, weighted) + 15) & ~(size_t)15;
 }
 
 }  // namespace
@@ -1063,12 +1118,12 @@ size_t lc_hist_bytes(int B, bool shapes) {
 // histogram (with every threshold) has to fit.
 bool lightcone_fits(const mia_bins &bins) {
     size_t thr = ((size_t)(bins.n_r + 1 + bins.n_2 + 1) * 8 + 15) & ~(size_t)15;
-    return thr + lc_hist_bytes(bins.n_2, true) <= kLcLds;
+    return thr + lc_hist_bytes(bins.n_2, true, true) <= kLcLds;
 }
 
 void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, const mia_counts &out,
                      const mia_tuning *tuning, hipStream_t st, mia_stats *stats) {
-    const bool shapes = s.c2 != nullptr;
+    const bool shapes = s.c2 != nullptr, weighted = s.w != nullptr || s.w_s != nullptr;
     const int n_r = bins.n_r, n_2 = bins.n_2, B = n_r * n_2;
     const int P = s.n_patches;
     const int P1 = P > 0 ? P : 1;
@@ -1417,26 +1472,28 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     A.lgs = (float)lgs;
     // (4u n_r: a pass's constant -l0 lgs - r0 is rounded to FP32 once more)
     double err_r = (4 * u * std::fmax(std::fabs(l0), std::fabs(ln)) + 4 * u) * lgs + 4 * u * n_r;
-    double err_2;
+    double err_2, xc = 0.0;
     if (bins.mode == MIA_RPPI) {
         A.X0 = bins.x2_edges[0];
         A.Xn = bins.x2_edges[n_2];
         double xs = n_2 / (bins.x2_edges[n_2] - bins.x2_edges[0]);
         A.xs = (float)xs;
-        A.xc = (float)(-bins.x2_edges[0] * xs);
+        xc = -bins.x2_edges[0] * xs;
         double mx = std::fmax(std::fabs(bins.x2_edges[0]), std::fabs(bins.x2_edges[n_2]));
         err_2 = 4 * u * mx * xs + 2 * u * n_2;
     } else {
         A.X0 = 0;
         A.Xn = 0;
         A.xs = (float)(n_2 / 2.0);
-        A.xc = 0.0f;
         err_2 = 6 * u * n_2;
     }
     double dr = std::fmax(1e-4, 20 * err_r), d2 = std::fmax(1e-4, 20 * err_2);
     bool exact_only = dr > 0.05 || d2 > 0.05;
-    A.dr = exact_only ? 1.0f : (float)dr;
-    A.d2 = exact_only ? 1.0f : (float)d2;
+    // (the guesses' constants are raised by the half widths)
+    A.dr = exact_only ? 2.0f : (float)(2.0 * dr);
+    A.d2 = exact_only ? 2.0f : (float)(2.0 * d2);
+    const double shift_r = exact_only ? 0.0 : dr, shift_2 = exact_only ? 0.0 : d2;
+    A.xc = (float)(xc + shift_2);
     A.scan = exact_only ? 1 : 0;
     // Passes over r-bin ranges, as in the box counter: pass [r0, r1) bins the
     // pairs with T[r0] <= r^2 < T[r1] (the exact path decides at the pass's
@@ -1447,12 +1504,12 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     const size_t thr_bytes = ((size_t)(n_r + 1 + n_2 + 1) * 8 + 15) & ~(size_t)15;
     auto wpb_for = [&](int nr_) {
         int w = kLcWavesPerBlock;
-        while (w > 1 && thr_bytes + lc_hist_bytes(nr_ * n_2, shapes) * w > kLcLds) w /= 2;
+        while (w > 1 && thr_bytes + lc_hist_bytes(nr_ * n_2, shapes, weighted) * w > kLcLds) w /= 2;
         return w;
     };
     auto waves_per_cu = [&](int nr_) {
         const int w = wpb_for(nr_);
-        const size_t l = thr_bytes + lc_hist_bytes(nr_ * n_2, shapes) * w;
+        const size_t l = thr_bytes + lc_hist_bytes(nr_ * n_2, shapes, weighted) * w;
         if (l > kLcLds) return 0;
         return (int)std::min<size_t>(32 / w, kLcLds / l) * w;
     };
@@ -1480,14 +1537,7 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     }
     const int npass = (n_r + nrp - 1) / nrp;
     const int Bp = nrp * n_2;  // bins of the largest pass
-    int off = ((4 * Bp) + 15) & ~15;
-    A.off_dd = off;
-    off += 8 * Bp;
-    A.off_sp = off;
-    if (shapes) off += 8 * Bp;
-    A.off_sx = off;
-    if (shapes) off += 8 * Bp;
-    A.hist_stride = (off + 15) & ~15;
+    A.hist_stride = (int)lc_hist_bytes(Bp, shapes, weighted);
     A.npairs = (unsigned long long *)out.npairs;
     A.dd = out.dd;
     A.sp = out.splus;
@@ -1496,7 +1546,12 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     const int wpb = wpb_for(nrp);
     const size_t lds = thr_bytes + (size_t)A.hist_stride * wpb;
     MIA_REQUIRE(lds <= kLcLds, "binning too large for the lightcone kernel's LDS histogram");
-    int blocks_per_cu = (int)std::max<size_t>(1, std::min<size_t>(32 / wpb, kLcLds / lds));
+    // as many workgroups as registers and LDS hold at once
+    int blocks_per_cu = 0;
+    const void *kernel = lc_kernel(bins.mode, shapes, weighted);
+    MIA_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    MIA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks_per_cu, kernel, kWave * wpb, lds));
+    blocks_per_cu = std::max(1, blocks_per_cu);
     int waves = tuning && tuning->waves > 0 ? std::min(tuning->waves, kMaxWaves) : ctx.cu_count * blocks_per_cu * wpb;
     if (nitems < waves) waves = std::max(1, nitems);
     A.n_waves = waves;
@@ -1512,19 +1567,10 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
         A.T = Td + r0;
         A.T0lo = bins.r2_edges[r0] * (1.0 - kDomainSlack);
         A.Tnhi = bins.r2_edges[r1] * (1.0 + kDomainSlack);
-        A.lgc = (float)(-l0 * lgs - r0);
+        A.lgc = (float)(-l0 * lgs - r0 + shift_r);
         A.queue = queue + pass;
-        if (bins.mode == MIA_RPPI) {
-            if (shapes)
-                lc_launch<MIA_RPPI, true>(A, grid, wpb, lds, st);
-            else
-                lc_launch<MIA_RPPI, false>(A, grid, wpb, lds, st);
-        } else {
-            if (shapes)
-                lc_launch<MIA_RMU, true>(A, grid, wpb, lds, st);
-            else
-                lc_launch<MIA_RMU, false>(A, grid, wpb, lds, st);
-        }
+        void *args[] = {&A};
+        MIA_HIP(hipLaunchKernel(kernel, dim3(grid), dim3(kWave * wpb), args, lds, st));
     }
     MIA_HIP(hipEventRecord(ev[3], st));
     MIA_HIP(hipEventRecord(ev[4], st));
