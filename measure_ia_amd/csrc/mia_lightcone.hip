@@ -60,6 +60,7 @@ constexpr int kLcThreads = kWave * kLcWavesPerBlock;
 constexpr size_t kLcLds = 160 * 1024 - 64;  // LDS per CU (gfx950) less the pair kernel's own words
 constexpr double kPiC = 3.141592653589793;  // numpy's np.pi
 constexpr double kDeg = kPiC / 180.0;
+constexpr int64_t kLcCountedPairs = 4096;     // patch pairs up to which items are counting-sorted (16 KiB of LDS)
 constexpr int kLcMaxPatches = 4096;           // patch pairs stay below 2^24 keys
 constexpr double kDomainSlack = 1e-9;         // relative widening of the approximate domain test
 
@@ -385,8 +386,7 @@ __global__ void k_lc_blocks_count(const int32_t *__restrict__ seg_start, int nse
 
 __global__ void k_lc_blocks_emit(const int32_t *__restrict__ seg_start,
                                  const uint64_t *__restrict__ seg_key, int nseg, int bsz,
-                                 const int32_t *__restrict__ off, const double *__restrict__ prec,
-                                 int P1, int nslab, LcBlock *__restrict__ blocks) {
+                                 const int32_t *__restrict__ off, int P1, int nslab, LcBlock *__restrict__ blocks) {
     int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= nseg) return;
     int s0 = seg_start[q], n = seg_start[q + 1] - s0;
@@ -399,17 +399,28 @@ __global__ void k_lc_blocks_emit(const int32_t *__restrict__ seg_start,
         B.np = n - b * bsz < bsz ? n - b * bsz : bsz;
         B.cell = cell;
         B.patch = patch;
-        // the positions run along chi only to the quantisation of the sort:
-        // the block's bounds are its true extremes
-        double lo = prec[8 * (int64_t)B.p0 + 2], hi = lo;
-        for (int j = 1; j < B.np; ++j) {
-            const double c = prec[8 * (int64_t)(B.p0 + j) + 2];
-            lo = c < lo ? c : lo;
-            hi = c > hi ? c : hi;
-        }
-        B.chi_lo = lo;
-        B.chi_hi = hi;
+        B.chi_lo = B.chi_hi = 0.0;  // k_lc_block_chi
         blocks[o + b] = B;
+    }
+}
+
+// One wave per block: the chi bounds of its positions.  (They run along chi only
+// to the quantisation of the sort: the bounds are the true extremes.)
+constexpr int kGroupWaves = 4;
+__global__ __launch_bounds__(kGroupWaves * kWave) void k_lc_block_chi(const double *__restrict__ prec, int nblocks,
+                                                                      LcBlock *__restrict__ blocks) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int b = blockIdx.x * kGroupWaves + threadIdx.x / kWave;
+    if (b >= nblocks) return;
+    const int p0 = blocks[b].p0, np = blocks[b].np;
+    double lo = prec[8 * (int64_t)(p0 + (lane < np ? lane : 0)) + 2], hi = lo;
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, d));
+        hi = fmax(hi, __shfl_xor(hi, d));
+    }
+    if (lane == 0) {
+        blocks[b].chi_lo = lo;
+        blocks[b].chi_hi = hi;
     }
 }
 
@@ -482,6 +493,7 @@ struct LcPlan {
     ChiQ scq;
     int item_shapes;          // ranges are split at this many shapes
     int32_t *rcount;          // count pass: ranges per stencil cell
+    int2 *window;             // the shapes [x, y) found in a cell of one segment (kept for the emit pass)
     const int64_t *roff;      // emit pass: range offsets, total + 1
     LcRange *ranges;
     int emit;
@@ -517,6 +529,7 @@ __device__ __forceinline__ int upper_chi(const uint32_t *x, int lo, int hi, uint
 __global__ void k_lc_ranges(LcPlan P) {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= P.total) return;
+    if (P.emit && P.roff[t + 1] == P.roff[t]) return;  // nothing to emit
     int lo = 0, hi = P.nblocks;  // last b with soff[b] <= t
     while (hi - lo > 1) {
         int mid = (lo + hi) >> 1;
@@ -538,14 +551,24 @@ __global__ void k_lc_ranges(LcPlan P) {
     double ddec = fmax(0.0, fmax(tdl - r.dh, r.dl - tdh));
     double dra = fmax(0.0, fmax(tcl - r.ch, r.cl - tch));
     double y = ddec * r.ky, x = dra * r.kx;
-    bool reach = x * x + y * y < g.R * g.R;
+    // (the emit pass has left the cells out of reach)
+    bool reach = P.emit || x * x + y * y < g.R * g.R;
     if (reach) {
         int cell = tr * g.ncols + tc;
         double clo = B.chi_lo + g.wlo, chi_hi = B.chi_hi + g.whi;
         int64_t o = P.emit ? P.roff[t] : 0;
-        for (int s = P.cfs[cell]; s < P.cfs[cell + 1]; ++s) {
-            int a = lower_chi(P.sq, P.sseg[s], P.sseg[s + 1], chi_q(P.scq, clo));
-            int e = upper_chi(P.sq, a, P.sseg[s + 1], chi_q(P.scq, chi_hi));
+        const int s0 = P.cfs[cell], s1 = P.cfs[cell + 1];
+        for (int s = s0; s < s1; ++s) {
+            int a, e;
+            if (P.emit && s1 == s0 + 1) {
+                const int2 w = P.window[t];
+                a = w.x;
+                e = w.y;
+            } else {
+                a = lower_chi(P.sq, P.sseg[s], P.sseg[s + 1], chi_q(P.scq, clo));
+                e = upper_chi(P.sq, a, P.sseg[s + 1], chi_q(P.scq, chi_hi));
+                if (!P.emit && s1 == s0 + 1) P.window[t] = make_int2(a, e);
+            }
             int patch = (int)(P.sseg_key[s] % (uint64_t)g.P1);
             for (int k = a; k < e; k += P.item_shapes) {
                 if (P.emit) {
@@ -563,71 +586,132 @@ __global__ void k_lc_ranges(LcPlan P) {
     if (!P.emit) P.rcount[t] = nout;
 }
 
-// Keys (block, patch) of the ranges, and the gather of the sorted order.
-__global__ void k_lc_range_keys(const LcRange *__restrict__ r, int64_t n, int pstride, uint64_t *__restrict__ key,
-                                int32_t *__restrict__ idx) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    key[i] = (uint64_t)r[i].blk * (uint64_t)pstride + (uint64_t)r[i].patch;
-    idx[i] = (int32_t)i;
-}
-
-__global__ void k_lc_gather_ranges(const int32_t *__restrict__ idx, int64_t n, const LcRange *__restrict__ in,
-                                   LcRange *__restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = in[idx[i]];
+// One wave per block: its ranges grouped by patch, in their order within a
+// patch.  A block's ranges come in stencil-cell order, so a stencil over a patch
+// border alternates patches row by row, and the items (one patch pair each)
+// would break at every change.  A block has a few dozen ranges: a range's place
+// is the number of ranges before it in (patch, index) order, counted directly
+// (a radix sort of all ranges by (block, patch) took 0.13 ms in 16 launches for
+// 1,000,000 positions, this one 0.02 ms).
+__global__ __launch_bounds__(kGroupWaves * kWave) void k_lc_group(const LcRange *__restrict__ in,
+                                                                  const int64_t *__restrict__ roff,
+                                                                  const int64_t *__restrict__ soff, int nblocks,
+                                                                  LcRange *__restrict__ out) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x * kGroupWaves + threadIdx.x / kWave);
+    if (b >= nblocks) return;
+    const int64_t r0 = roff[soff[b]];
+    const int n = (int)(roff[soff[b + 1]] - r0);
+    for (int i0 = 0; i0 < n; i0 += kWave) {
+        const int i = i0 + lane;
+        LcRange mine{};
+        if (i < n) mine = in[r0 + i];
+        int at = 0;
+        for (int j0 = 0; j0 < n; j0 += kWave) {
+            const int m = n - j0 < kWave ? n - j0 : kWave;
+            const int theirs = lane < m ? in[r0 + j0 + lane].patch : 0;
+            for (int k = 0; k < m; ++k) {
+                const int p = __builtin_amdgcn_readlane(theirs, k);
+                at += (p < mine.patch || (p == mine.patch && j0 + k < i)) ? 1 : 0;
+            }
+        }
+        if (i < n) out[r0 + at] = mine;
+    }
 }
 
 // One thread per block: consecutive ranges of one shape patch form an item of
-// at most item_shapes shapes.
-__global__ void k_lc_items(const LcRange *__restrict__ ranges, const int64_t *__restrict__ roff,
-                           const int64_t *__restrict__ soff, int nblocks, int item_shapes,
-                           int32_t *__restrict__ nitem, const int32_t *__restrict__ ioff,
-                           LcItem *__restrict__ items, const LcBlock *__restrict__ blocks,
-                           int P1, int32_t *__restrict__ ikey, int64_t *__restrict__ cost,
-                           unsigned long long *__restrict__ cand) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nblocks) return;
-    int64_t r_begin = roff[soff[b]], r_end = roff[soff[b + 1]];
-    const bool emit = items != nullptr;
-    int n = 0;
-    int o = emit ? ioff[b] : 0;
-    const int np = emit ? blocks[b].np : 0;
-    const int pn = emit ? blocks[b].patch : 0;
-    unsigned long long c = 0;
-    int64_t r0 = r_begin;
-    int acc = 0, patch = -1;
-    auto close = [&](int64_t rend) {
-        if (acc > 0) {
-            if (emit) {
-                LcItem it;
-                it.blk = b;
-                it.r0 = (int32_t)r0;
-                it.nr = (int32_t)(rend - r0);
-                it.ns = acc;
-                items[o + n] = it;
-                ikey[o + n] = pn * P1 + patch;
-                // one 64-lane batch per 64 shapes, each a pass over the block's positions
-                int64_t nbt = (acc + kWave - 1) / kWave;
-                cost[o + n] = nbt * ((int64_t)kWave * np + 32) + 128;
-                c += (unsigned long long)acc * np;
-            }
-            ++n;
-        }
-    };
-    for (int64_t r = r_begin; r < r_end; ++r) {
-        LcRange R = ranges[r];
-        if (R.patch != patch || acc + R.n > item_shapes) {
-            close(r);
-            r0 = r;
-            acc = 0;
-            patch = R.patch;
-        }
-        acc += R.n;
+// at most item_shapes shapes.  With kcount the count pass also counts the items
+// of every patch pair, and with kcursor (their scan) the emit pass places them
+// pair by pair; both add up a workgroup's items per pair in LDS first, since
+// most items belong to a few pairs (a patch with itself), whose counters would
+// otherwise queue (0.6 ms for 600,000 items).  Without them items are placed
+// block by block, with their keys.
+struct LcItemArgs {
+    const LcRange *ranges;
+    const int64_t *roff, *soff;
+    const LcBlock *blocks;
+    int nblocks, item_shapes, P1;
+    int32_t *nitem;        // count pass, without kcount: items per block
+    int32_t *kcount;       // count pass: items per patch pair
+    const int32_t *ioff;   // emit pass: first item of every block
+    int32_t *kcursor;      // emit pass: next place of every pair
+    LcItem *items;         // emit pass (else null)
+    int32_t *ikey;
+    int64_t *cost;
+    unsigned long long *cand;
+};
+
+__global__ __launch_bounds__(256) void k_lc_items(LcItemArgs A) {
+    extern __shared__ int32_t lpair[];  // items per pair of the workgroup, then their base
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool emit = A.items != nullptr, active = b < A.nblocks, counted = A.kcount || A.kcursor;
+    const int nk = A.P1 * A.P1;
+    int64_t r_begin = 0, r_end = 0;
+    int np = 0, pn = 0;
+    if (active) {
+        r_begin = A.roff[A.soff[b]];
+        r_end = A.roff[A.soff[b + 1]];
+        np = A.blocks[b].np;
+        pn = A.blocks[b].patch;
     }
-    close(r_end);
-    if (!emit) nitem[b] = n;
-    if (emit && c) atomicAdd(cand, c);
+    // f(first range, ranges, shapes, patch) of every item of the block
+    auto walk = [&](auto &&f) {
+        int64_t r0 = r_begin;
+        int acc = 0, patch = -1;
+        for (int64_t r = r_begin; r < r_end; ++r) {
+            const LcRange R = A.ranges[r];
+            if (R.patch != patch || acc + R.n > A.item_shapes) {
+                if (acc > 0) f(r0, (int)(r - r0), acc, patch);
+                r0 = r;
+                acc = 0;
+                patch = R.patch;
+            }
+            acc += R.n;
+        }
+        if (acc > 0) f(r0, (int)(r_end - r0), acc, patch);
+    };
+    if (counted) {
+        for (int k = threadIdx.x; k < nk; k += blockDim.x) lpair[k] = 0;
+        __syncthreads();
+        walk([&](int64_t, int, int, int patch) { atomicAdd(&lpair[pn * A.P1 + patch], 1); });
+        __syncthreads();
+        for (int k = threadIdx.x; k < nk; k += blockDim.x) {
+            const int c = lpair[k];
+            if (!c) continue;
+            if (emit)
+                lpair[k] = atomicAdd(&A.kcursor[k], c);
+            else
+                atomicAdd(&A.kcount[k], c);
+        }
+        __syncthreads();
+    }
+    if (!active) return;
+    if (!emit) {
+        if (!counted) {
+            int n = 0;
+            walk([&](int64_t, int, int, int) { ++n; });
+            A.nitem[b] = n;
+        }
+        return;
+    }
+    int o = counted ? 0 : A.ioff[b];
+    unsigned long long c = 0;
+    walk([&](int64_t r0, int nr, int acc, int patch) {
+        const int key = pn * A.P1 + patch;
+        const int at = counted ? atomicAdd(&lpair[key], 1) : o++;
+        LcItem it;
+        it.blk = b;
+        it.r0 = (int32_t)r0;
+        it.nr = nr;
+        it.ns = acc;
+        A.items[at] = it;
+        if (A.ikey) A.ikey[at] = key;
+        // one 64-lane batch per 64 shapes, each a pass over the block's positions
+        const int64_t nbt = (acc + kWave - 1) / kWave;
+        A.cost[at] = nbt * ((int64_t)kWave * np + 32) + 128;
+        c += (unsigned long long)acc * np;
+    });
+    if (c) atomicAdd(A.cand, c);
 }
 
 __global__ void k_lc_widen(const int32_t *__restrict__ a, int64_t *__restrict__ b, int64_t n) {
@@ -1315,7 +1399,10 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     MIA_HIP(hipStreamSynchronize(st));
     LcBlock *blocks = ctx.arena.get<LcBlock>("lc/blocks", std::max(nblocks, 1));
     hipLaunchKernelGGL(k_lc_blocks_emit, dim3(nblk_(npseg, 256)), dim3(256), 0, st, pseg, pseg_key, npseg,
-                       bsz, nbo, prec, P1, g.nslab, blocks);
+                       bsz, nbo, P1, g.nslab, blocks);
+    MIA_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_lc_block_chi, dim3(nblk_(nblocks, kGroupWaves)), dim3(kGroupWaves * kWave), 0, st, prec,
+                       nblocks, blocks);
     MIA_HIP(hipGetLastError());
     LcRect *rect = ctx.arena.get<LcRect>("lc/rect", std::max(nblocks, 1));
     int64_t *ssz = ctx.arena.get<int64_t>("lc/ssz", nblocks + 1);
@@ -1351,6 +1438,7 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     int64_t *rc64 = ctx.arena.get<int64_t>("lc/rc64", total + 1);
     int64_t *roff = ctx.arena.get<int64_t>("lc/roff", total + 1);
     L.rcount = rc;
+    L.window = ctx.arena.get<int2>("lc/window", total + 1);
     L.emit = 0;
     if (total > 0) {
         hipLaunchKernelGGL(k_lc_ranges, dim3(nblk_(total, 256)), dim3(256), 0, st, L);
@@ -1373,46 +1461,50 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
         MIA_HIP(hipGetLastError());
     }
     if (P > 0 && nranges > 1) {
-        // A block's ranges come in stencil-cell order, so a stencil over a
-        // patch border alternates patches row by row and the items (one
-        // patch pair each) break at every change.  A stable sort by (block,
-        // patch) keeps each block's ranges in place and groups its patches:
-        // lightcone1M went from 6.2 items per block to about one per patch.
-        uint64_t *rk = ctx.arena.get<uint64_t>("lc/rk", nranges);
-        uint64_t *rk2 = ctx.arena.get<uint64_t>("lc/rk2", nranges);
-        int32_t *ri = ctx.arena.get<int32_t>("lc/ri", nranges);
-        int32_t *ri2 = ctx.arena.get<int32_t>("lc/ri2", nranges);
         LcRange *ranges2 = ctx.arena.get<LcRange>("lc/ranges2", nranges);
-        hipLaunchKernelGGL(k_lc_range_keys, dim3(nblk_(nranges, 256)), dim3(256), 0, st,
-                           (const LcRange *)ranges, nranges, P1 + 1, rk, ri);
-        MIA_HIP(hipGetLastError());
-        radix_sort<uint64_t>(ctx, rk, rk2, ri, ri2, nranges, bits_for((uint64_t)nblocks * (P1 + 1)), st,
-                             "lc/rsort");
-        hipLaunchKernelGGL(k_lc_gather_ranges, dim3(nblk_(nranges, 256)), dim3(256), 0, st,
-                           (const int32_t *)ri2, nranges, (const LcRange *)ranges, ranges2);
+        hipLaunchKernelGGL(k_lc_group, dim3(nblk_(nblocks, kGroupWaves)), dim3(kGroupWaves * kWave), 0, st,
+                           (const LcRange *)ranges, roff, soff, nblocks, ranges2);
         MIA_HIP(hipGetLastError());
         ranges = ranges2;
     }
 
-    // ---- plan: items (count, scan, emit), sorted by patch pair
+    // ---- plan: items (count, scan, emit), sorted by patch pair: a counting sort
+    // while the pairs' counters stay small (at 27 patches and 100,000 items two
+    // scans instead of a 16-launch radix sort of 0.11 ms), else a radix sort
     int32_t *nit = ctx.arena.get<int32_t>("lc/nit", nblocks + 1);
     int32_t *ioff = ctx.arena.get<int32_t>("lc/ioff", nblocks + 1);
-    hipLaunchKernelGGL(k_lc_items, dim3(nblk_(nblocks, 256)), dim3(256), 0, st, ranges, roff, soff,
-                       nblocks, item_shapes, nit, (const int32_t *)nullptr, (LcItem *)nullptr,
-                       (const LcBlock *)nullptr, P1, (int32_t *)nullptr, (int64_t *)nullptr,
-                       (unsigned long long *)nullptr);
+    const int64_t pairs = (int64_t)P1 * P1;
+    const bool counting = pairs <= kLcCountedPairs;
+    int32_t *kcount = nullptr, *koff = nullptr;
+    if (counting) {
+        kcount = ctx.arena.get<int32_t>("lc/kcount", pairs + 1);
+        koff = ctx.arena.get<int32_t>("lc/koff", pairs + 1);
+        fill<int32_t>(kcount, 0, pairs, st);
+    }
+    LcItemArgs I{};
+    I.ranges = ranges;
+    I.roff = roff;
+    I.soff = soff;
+    I.blocks = blocks;
+    I.nblocks = nblocks;
+    I.item_shapes = item_shapes;
+    I.P1 = P1;
+    I.nitem = nit;
+    I.kcount = kcount;
+    const unsigned igrid = nblk_(nblocks, 256);
+    const size_t ilds = counting ? sizeof(int32_t) * (size_t)pairs : 0;
+    hipLaunchKernelGGL(k_lc_items, dim3(igrid), dim3(256), ilds, st, I);
     MIA_HIP(hipGetLastError());
-    exclusive_scan<int32_t>(ctx, nit, ioff, nblocks, st, "lc/its", 0);
     int32_t nitems = 0;
-    MIA_HIP(hipMemcpyAsync(&nitems, ioff + nblocks, 4, hipMemcpyDeviceToHost, st));
+    if (counting) {
+        exclusive_scan<int32_t>(ctx, kcount, koff, pairs, st, "lc/its", 0);
+        MIA_HIP(hipMemcpyAsync(&nitems, koff + pairs, 4, hipMemcpyDeviceToHost, st));
+    } else {
+        exclusive_scan<int32_t>(ctx, nit, ioff, nblocks, st, "lc/its", 0);
+        MIA_HIP(hipMemcpyAsync(&nitems, ioff + nblocks, 4, hipMemcpyDeviceToHost, st));
+    }
     MIA_HIP(hipStreamSynchronize(st));
-    LcItem *items0 = ctx.arena.get<LcItem>("lc/items0", std::max(nitems, 1));
     LcItem *items = ctx.arena.get<LcItem>("lc/items", std::max(nitems, 1));
-    int32_t *ikey = ctx.arena.get<int32_t>("lc/ikey", std::max(nitems, 1));
-    int32_t *ikey2 = ctx.arena.get<int32_t>("lc/ikey2", std::max(nitems, 1));
-    int32_t *iidx = ctx.arena.get<int32_t>("lc/iidx", std::max(nitems, 1));
-    int32_t *iord = ctx.arena.get<int32_t>("lc/iord", std::max(nitems, 1));
-    int64_t *cost0 = ctx.arena.get<int64_t>("lc/cost0", nitems + 1);
     int64_t *cost = ctx.arena.get<int64_t>("lc/cost", nitems + 1);
     int64_t *cpre = ctx.arena.get<int64_t>("lc/cpre", nitems + 1);
     unsigned long long *counters = ctx.arena.get<unsigned long long>("lc/counters", 2);
@@ -1420,17 +1512,36 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     // one tail-chunk counter per r-bin pass (n_r <= kMaxBinsR)
     int32_t *queue = ctx.arena.get<int32_t>("lc/queue", kMaxBinsR);
     fill<int32_t>(queue, 0, kMaxBinsR, st);
-    hipLaunchKernelGGL(k_lc_items, dim3(nblk_(nblocks, 256)), dim3(256), 0, st, ranges, roff, soff,
-                       nblocks, item_shapes, nit, ioff, items0, blocks, P1, ikey, cost0, counters + 1);
-    MIA_HIP(hipGetLastError());
-    if (nitems > 0) {
-        hipLaunchKernelGGL(k_lc_iota, dim3(nblk_(nitems, 256)), dim3(256), 0, st, iidx, (int64_t)nitems);
+    I.kcount = nullptr;
+    I.cand = counters + 1;
+    if (counting) {
+        I.kcursor = koff;
+        I.items = items;
+        I.cost = cost;
+        hipLaunchKernelGGL(k_lc_items, dim3(igrid), dim3(256), ilds, st, I);
         MIA_HIP(hipGetLastError());
-        radix_sort<int32_t>(ctx, ikey, ikey2, iidx, iord, nitems,
-                            bits_for((uint64_t)P1 * (uint64_t)P1), st, "lc/isort");
-        hipLaunchKernelGGL(k_lc_gather_items, dim3(nblk_(nitems, 256)), dim3(256), 0, st, iord,
-                           (int64_t)nitems, items0, cost0, items, cost);
+    } else {
+        LcItem *items0 = ctx.arena.get<LcItem>("lc/items0", std::max(nitems, 1));
+        int32_t *ikey = ctx.arena.get<int32_t>("lc/ikey", std::max(nitems, 1));
+        int32_t *ikey2 = ctx.arena.get<int32_t>("lc/ikey2", std::max(nitems, 1));
+        int32_t *iidx = ctx.arena.get<int32_t>("lc/iidx", std::max(nitems, 1));
+        int32_t *iord = ctx.arena.get<int32_t>("lc/iord", std::max(nitems, 1));
+        int64_t *cost0 = ctx.arena.get<int64_t>("lc/cost0", nitems + 1);
+        I.ioff = ioff;
+        I.items = items0;
+        I.ikey = ikey;
+        I.cost = cost0;
+        hipLaunchKernelGGL(k_lc_items, dim3(igrid), dim3(256), 0, st, I);
         MIA_HIP(hipGetLastError());
+        if (nitems > 0) {
+            hipLaunchKernelGGL(k_lc_iota, dim3(nblk_(nitems, 256)), dim3(256), 0, st, iidx, (int64_t)nitems);
+            MIA_HIP(hipGetLastError());
+            radix_sort<int32_t>(ctx, ikey, ikey2, iidx, iord, nitems,
+                                bits_for((uint64_t)P1 * (uint64_t)P1), st, "lc/isort");
+            hipLaunchKernelGGL(k_lc_gather_items, dim3(nblk_(nitems, 256)), dim3(256), 0, st, iord,
+                               (int64_t)nitems, items0, cost0, items, cost);
+            MIA_HIP(hipGetLastError());
+        }
     }
     exclusive_scan<int64_t>(ctx, cost, cpre, nitems, st, "lc/cs", 0);
     MIA_HIP(hipEventRecord(ev[2], st));
