@@ -1680,12 +1680,17 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     // private, 7 shared; 3,000,000 positions to 100 Mpc/h 317 against 201 ms),
     // but a group of four waits for its slowest wave wherever the key or the
     // chunk changes (200 bins, 28 private waves per CU, 1,000,000 positions: 8.5
-    // against 11.7 ms).  So it is taken below kSharedBelow private waves per CU,
-    // and where the registers allow more waves than LDS while the launch is too
-    // small for tail chunks (317,811 weighted positions with variances, 20
-    // private waves: 2.65 against 1.9 ms) or so large that its chunks hold many
-    // items (2,000,000 positions, 300 bins: 205 against 200 ms; but twelve
-    // samples of 10,000 to 800,000, 24 private waves: 21 against 31 ms).  Never where the reduction is
+    // against 11.7 ms).  So it is taken
+    //   - below kSharedBelow private waves per CU;
+    //   - in launches too small for tail chunks, where the four waves even out
+    //     each other's items (60,000 shapes in 300,000 positions 1.82 against
+    //     1.55 ms, 75,025 in 317,811 weighted with variances 2.65 against 1.9,
+    //     10,000 in 50,000 0.43 against 0.39, 30,000 in 150,000 equal);
+    //   - where registers allow more waves than LDS and the launch is so large
+    //     that its chunks hold many items (2,000,000 positions, 300 bins: 205
+    //     against 200 ms; but twelve samples of 10,000 to 800,000, 24 private
+    //     waves: 21 against 31 ms).
+    // Never where the reduction is
     // deterministic, since a shared histogram's sums depend on timing.
     // mia_tuning.hist_copies is ignored.
     int wpb = kMaxWavesPerBlock;
@@ -1693,7 +1698,7 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     const int pw = private_waves(thr_bytes, hs), most = std::min(4 * kPairWavesPerSimd, shared_waves(thr_bytes, hs));
     const bool small = candidates < kTailMinCost * pw * cu_count;
     const bool large = candidates > 10 * kTailMinCost * pw * cu_count;
-    A.shared = !det && pw < most && (pw < kSharedBelow || small || large);
+    A.shared = !det && most > 0 && (small || (pw < most && (pw < kSharedBelow || large)));
     if (A.shared) {
         const size_t share = kLdsBytes / kPairWavesPerSimd - kPairStaticLds;
         A.copies = share > thr_bytes + hs ? (int)std::min<size_t>(4, (share - thr_bytes) / hs) : 1;
