@@ -103,7 +103,7 @@ struct PlanSample {
     int ng, G;           // slab groups per column, slabs per group
     int ncp, cpi;        // position columns per side (g.nc * g.m), columns per item
     int pbits, pad;      // positions' fine key = (cell << pbits) + line-of-sight part of the slab
-    double fw, hq;       // position column width, height of a line-of-sight part
+    double fw, hq_inv;   // position column width, line-of-sight parts per length
     double reach_r, reach_z;
     double x_lo, x_hi;   // line-of-sight domain, for cutting slab runs to a block's window
     const int32_t *sstart;
@@ -200,7 +200,7 @@ __device__ __forceinline__ bool slab_in(const PlanSample &P, double zlo, double 
 // to the block's line-of-sight window, or (k0 == nz) the column's tail.
 struct ColumnView {
     const int32_t *pfine;
-    double L, half, margin, fw, hq, reach_r, x_lo, x_hi;
+    double L, half, margin, fw, hq_inv, reach_r, x_lo, x_hi;
     int ncp, nz, pbits, mode, periodic;
 };
 
@@ -212,7 +212,7 @@ __device__ __forceinline__ ColumnView column_view(const PS *p) {
     v.half = p->g.half;
     v.margin = p->g.margin;
     v.fw = p->fw;
-    v.hq = p->hq;
+    v.hq_inv = p->hq_inv;
     v.reach_r = p->reach_r;
     v.x_lo = p->x_lo;
     v.x_hi = p->x_hi;
@@ -225,13 +225,22 @@ __device__ __forceinline__ ColumnView column_view(const PS *p) {
 }
 
 __device__ __forceinline__ void column_positions(const ColumnView &v, double b0, double b1, double b2, double b3,
-                                                 double zlo, double zhi, int ja, int jb, int k0, int k1, int cz,
-                                                 int &pb, int &n) {
+                                                 double zlo, double zhi, int ja, int jb, int k0, int k1, int shifts,
+                                                 int cz, int &pb, int &n) {
     const double m = v.margin;
     double da, db;
-    int ca, cb;
-    axis_class(b0 - (ja + 1) * v.fw - 2 * m, b1 - ja * v.fw + 2 * m, v.L, v.half, v.periodic, da, ca);
-    axis_class(b2 - (jb + 1) * v.fw - 2 * m, b3 - jb * v.fw + 2 * m, v.L, v.half, v.periodic, db, cb);
+    const double alo = b0 - (ja + 1) * v.fw - 2 * m, ahi = b1 - ja * v.fw + 2 * m;
+    const double blo = b2 - (jb + 1) * v.fw - 2 * m, bhi = b3 - jb * v.fw + 2 * m;
+    if (shifts & 64) {
+        int ca, cb;
+        axis_class(alo, ahi, v.L, v.half, v.periodic, da, ca);
+        axis_class(blo, bhi, v.L, v.half, v.periodic, db, cb);
+    } else {
+        // one shift for the whole rectangle: the distance of the shifted ranges from zero
+        const double sa = shift_val(shifts & 3, v.L), sb = shift_val((shifts >> 2) & 3, v.L);
+        da = fmax(fmax(alo + sa, -(ahi + sa)), 0.0);
+        db = fmax(fmax(blo + sb, -(bhi + sb)), 0.0);
+    }
     const double rr = v.reach_r + 4 * m;
     const double dxy2 = da * da + db * db;
     pb = 0;
@@ -253,7 +262,7 @@ __device__ __forceinline__ void column_positions(const ColumnView &v, double b0,
             whi = zhi + sh + rz + 4 * m;
         }
         const double q0 = (double)(k0 << v.pbits), q1 = (double)(k1 << v.pbits);
-        const double lo = fmin(fmax(floor(wlo / v.hq), q0), q1), hi = fmin(fmax(floor(whi / v.hq) + 1.0, q0), q1);
+        const double lo = fmin(fmax(floor(wlo * v.hq_inv), q0), q1), hi = fmin(fmax(floor(whi * v.hq_inv) + 1.0, q0), q1);
         f0 = (base << v.pbits) + (int64_t)lo;
         f1 = (base << v.pbits) + (int64_t)hi;
         if (f1 <= f0) return;
@@ -482,12 +491,16 @@ __global__ __launch_bounds__(kPlanThreads) void k_emit_items(PlanLaunch A) {
 
 // The lane's column of an item, and its positions.
 __device__ __forceinline__ void item_column(const ColumnView &v, const double *bb, int ja, int jb, int wb, int nc,
-                                            int c0, int k0, int k1, int cz, int lane, int &pb, int &n) {
+                                            int c0, int k0, int k1, int w, int lane, int &pb, int &n) {
     pb = 0;
     n = 0;
     if (lane < nc) {
-        const int c = c0 + lane, row = c / wb;
-        column_positions(v, bb[0], bb[1], bb[2], bb[3], bb[4], bb[5], ja + row, jb + (c - row * wb), k0, k1, cz, pb, n);
+        // the first column's row and place in it are the wave's; the lane's
+        // quotient is of numbers below 2^13, exact in FP32 from half a unit up
+        const int row0 = c0 / wb, x = c0 - row0 * wb + lane;
+        const int row = (int)(((float)x + 0.5f) * __frcp_rn((float)wb));
+        column_positions(v, bb[0], bb[1], bb[2], bb[3], bb[4], bb[5], ja + row0 + row, jb + (x - row * wb), k0, k1,
+                         (w >> 16) & 0xff, (w >> 24) & 3, pb, n);
     }
 }
 
@@ -512,8 +525,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_item_cost(const PlanSample *ps
         const int ns = bp[1];
         int pb, np;
         item_column(column_view((const MIA_CONST PlanSample *)ps + bp[4]), bb, jj & 0xffff, (jj >> 16) & 0xffff,
-                    wn & 0xffff, (wn >> 16) & 0xffff, c0, kk & 0xffff, (kk >> 16) & 0xffff, (w >> 24) & 3, lane, pb,
-                    np);
+                    wn & 0xffff, (wn >> 16) & 0xffff, c0, kk & 0xffff, (kk >> 16) & 0xffff, w, lane, pb, np);
         for (int d = kWave / 2; d > 0; d >>= 1) np += __shfl_xor(np, d);
         if (lane == 0) {
             items[i].np = np;
@@ -1440,7 +1452,7 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
                     const double bb[6] = {bc[0], bc[1], bc[2], bc[3], bc[4], bc[5]};
                     item_column(column_view((const MIA_CONST PlanSample *)P.ps + sample), bb, jj & 0xffff,
                                 (jj >> 16) & 0xffff, wn & 0xffff, (wn >> 16) & 0xffff, c0, kk & 0xffff,
-                                (kk >> 16) & 0xffff, (w >> 24) & 3, lane, cpb, cn);
+                                (kk >> 16) & 0xffff, w, lane, cpb, cn);
                 }
                 // (r, mu) sums r^2 in an order fixed by the line of sight: one
                 // loop per order, so the pair loop holds no branch on it
@@ -1903,7 +1915,7 @@ CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_b
         Q.ncp = g.nc * g.m;
         Q.pbits = x.pbits;
         Q.fw = g.cw / g.m;
-        Q.hq = g.hz / (double)(1 << x.pbits);
+        Q.hq_inv = (double)(1 << x.pbits) / g.hz;
         // columns per item: about kItemPositions positions at the mean density
         // (mia_tuning.item_positions), at most one column per lane
         const double per_col = (double)x.n_pos / ((double)Q.ncp * Q.ncp) *
