@@ -35,6 +35,8 @@ constexpr int kBlockShapes = 64;
 constexpr int kItemPositions = 8192;
 constexpr int kMaxPosColumns = 4096;     // position columns per side (12-bit indices)
 
+constexpr int kSearchSteps = 24;         // column and slab counts tried per axis, about
+
 struct Choice {
     int ncj, nzj, G, m;
 };
@@ -112,8 +114,20 @@ Choice search(double L, int jk, double R, double Z, bool rmu, int64_t ns, int64_
     int z1 = std::max(z0, std::min(512 / jk, (int)std::ceil(span / (zr / 12.0))));
     Choice best{c0, z0, 1, 1};
     double best_t = -1.0;
-    for (int ncj = c0; ncj <= c1; ++ncj)
-        for (int nzj = z0; nzj <= z1; ++nzj)
+    // at most kSearchSteps counts per axis, evenly spaced in the logarithm (a
+    // search over all of them took 0.1 s for a large box without jackknife)
+    auto counts = [](int lo, int hi) {
+        std::vector<int> v;
+        for (int k = 0; k <= kSearchSteps; ++k) {
+            const int x = hi - lo < kSearchSteps ? lo + k
+                                                 : (int)std::lround(lo * std::pow((double)hi / lo, k / (double)kSearchSteps));
+            if (x <= hi && (v.empty() || x > v.back())) v.push_back(x);
+        }
+        return v;
+    };
+    const std::vector<int> cs = counts(c0, c1), zs = counts(z0, z1);
+    for (int ncj : cs)
+        for (int nzj : zs)
             for (int G = 1; G <= 4 && G <= nzj; ++G) {
                 if (nzj % G) continue;
                 Choice c{ncj, nzj, G, 1};

@@ -771,10 +771,16 @@ typedef const __attribute__((address_space(4))) int32_t *CPtrI;
 // One bin of a wave's histogram: the pair count, with shapes S+D and SxD, with
 // weights DD (unit weights: DD is the count itself, so random-random counts
 // touch four bytes per bin).  A pending run keeps its slot's address and the
-// fields lie at constant offsets from it.
+// fields lie at constant offsets from it.  With weights the counts are an array
+// of their own behind the slots (28 instead of 32 bytes per bin with shapes:
+// fine binnings run few waves per CU, each histogram byte counting).
 template <bool SHAPES, bool WEIGHTED>
 struct LcSlot {
-    double v[(SHAPES ? 2 : 0) + (WEIGHTED ? 1 : 0)];  // [S+D, SxD], [DD]
+    double v[(SHAPES ? 2 : 0) + 1];  // [S+D, SxD], DD
+};
+template <>
+struct LcSlot<true, false> {
+    double v[2];
     uint32_t c, pad;
 };
 template <>
@@ -782,14 +788,16 @@ struct LcSlot<false, false> {
     uint32_t c;
 };
 static_assert(sizeof(LcSlot<false, false>) == 4 && sizeof(LcSlot<true, false>) == 24 &&
-                  sizeof(LcSlot<true, true>) == 32 && sizeof(LcSlot<false, true>) == 16,
+                  sizeof(LcSlot<true, true>) == 24 && sizeof(LcSlot<false, true>) == 8,
               "LcSlot layout");
+// bytes per bin, the count among them
 constexpr size_t lc_slot_bytes(bool shapes, bool weighted) {
-    return shapes || weighted ? 8 + (shapes ? 16 : 0) + (weighted ? 8 : 0) : 4;
+    return weighted ? (shapes ? 28 : 12) : (shapes ? 24 : 4);
 }
 
 struct LcPend {
     uint32_t at;  // LDS address of the slot
+    uint32_t ac;  // with weights: LDS address of the count
     uint32_t c;
     double dd, sp, sx;
 };
@@ -803,7 +811,10 @@ template <bool SHAPES, bool WEIGHTED>
 __device__ __forceinline__ void lc_hist_add(const LcPend &p) {
     typedef MIA_LDS LcSlot<SHAPES, WEIGHTED> S;
     S *s = (S *)p.at;
-    lds_add(&s->c, p.c);
+    if constexpr (WEIGHTED)
+        lds_add((MIA_LDS uint32_t *)p.ac, p.c);
+    else
+        lds_add(&s->c, p.c);
     if constexpr (SHAPES) {
         lds_add(&s->v[0], p.sp);
         lds_add(&s->v[1], p.sx);
@@ -818,7 +829,14 @@ __device__ void lc_flush(const LcPairArgs &P, char *hist, int pn, int ps, int la
     const int B = P.nbins, BO = P.nbins_out;
     for (int b = lane; b < B; b += kWave) {
         const Slot t = slots[b];
-        const uint32_t c = t.c;
+        uint32_t c;
+        if constexpr (WEIGHTED) {
+            uint32_t *cnt = (uint32_t *)(slots + B);
+            c = cnt[b];
+            cnt[b] = 0;
+        } else {
+            c = t.c;
+        }
         if (c == 0) continue;
         slots[b] = Slot{};
         double vsp = 0.0, vsx = 0.0, vdd = (double)c;
@@ -867,7 +885,7 @@ template <int MODE, bool SHAPES, bool WEIGHTED>
 __device__ __forceinline__ void lc_pair(const LcPairArgs &P, bool valid, double qra, double qdec,
                                         double qchi, double qc2, double qs2, double qw, double pra,
                                         double pdec, double pchi, double pax, double pay, double pw,
-                                        double pcos, uint32_t hist, uint32_t row, const double *T, const double *X,
+                                        double pcos, uint32_t hist, uint32_t hist_c, uint32_t row, const double *T, const double *X,
                                         uint32_t &nre, LcPend &pd, float vlgc, float vxc) {
     const int n_r = P.n_r, n_2 = P.n_2;
     const double dra = qra - pra, ddec = qdec - pdec;
@@ -944,6 +962,7 @@ __device__ __forceinline__ void lc_pair(const LcPairArgs &P, bool valid, double 
     const bool nw = at != pd.at;
     if (nw) lc_hist_add<SHAPES, WEIGHTED>(pd);
     pd.at = at;
+    if (WEIGHTED) pd.ac = __umul24(ir, 4u * (uint32_t)n_2) + (4u * (uint32_t)i2 + hist_c);
     pd.c = (nw ? 0u : pd.c) + 1u;
     if (SHAPES || WEIGHTED) {
         const double keep = nw ? 0.0 : 1.0;
@@ -977,7 +996,9 @@ __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
     const uint32_t hist_at = (uint32_t)(uintptr_t)(MIA_LDS char *)hist;
     const uint32_t row = (uint32_t)(P.n_2 * sizeof(LcSlot<SHAPES, WEIGHTED>));
     // an empty run adds its zeros to some bin, another one for every lane
-    const uint32_t none = hist_at + (uint32_t)((lane < P.nbins ? lane : 0) * sizeof(LcSlot<SHAPES, WEIGHTED>));
+    const uint32_t first = lane < P.nbins ? lane : 0;
+    const uint32_t hist_c = hist_at + (uint32_t)(P.nbins * sizeof(LcSlot<SHAPES, WEIGHTED>));
+    const uint32_t none = hist_at + first * (uint32_t)sizeof(LcSlot<SHAPES, WEIGHTED>), none_c = hist_c + 4u * first;
 
     // runs of neighbouring items of the patch-sorted list (which read the
     // same position blocks) stay on one XCD
@@ -1016,7 +1037,7 @@ __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
                 cur_pn = pn;
                 cur_ps = ps;
             }
-            LcPend pd{none, 0, 0.0, 0.0, 0.0};
+            LcPend pd{none, none_c, 0, 0.0, 0.0, 0.0};
             int j = r0, o = 0;
             const int jend = r0 + nr;
             for (int done = 0; done < ns; done += kWave) {
@@ -1057,7 +1078,7 @@ __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
                         const double b0 = rn[0], b1 = rn[1], b2 = rn[2], b3 = rn[3], b4 = rn[4], b5 = rn[5],
                                      b6 = rn[6];
                         lc_pair<MODE, SHAPES, WEIGHTED>(P, v, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5, a6,
-                                              hist_at, row, T, X, nre, pd, vlgc, vxc);
+                                              hist_at, hist_c, row, T, X, nre, pd, vlgc, vxc);
                         a0 = b0;
                         a1 = b1;
                         a2 = b2;
@@ -1090,12 +1111,12 @@ __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
                     const double b0 = r1[0], b1 = r1[1], b2 = r1[2], b3 = r1[3], b4 = r1[4], b5 = r1[5],
                                  b6 = r1[6];
                     lc_pair<MODE, SHAPES, WEIGHTED>(P, valid, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5,
-                                          a6, hist_at, row, T, X, nre, pd, vlgc, vxc);
+                                          a6, hist_at, hist_c, row, T, X, nre, pd, vlgc, vxc);
                     CPtrD r2 = (CPtrD)((CPtrC)pr + (ob + 128u < olast ? ob + 128u : olast));
                     const double c0 = r2[0], c1 = r2[1], c2 = r2[2], c3 = r2[3], c4 = r2[4], c5 = r2[5],
                                  c6 = r2[6];
                     lc_pair<MODE, SHAPES, WEIGHTED>(P, valid, qra, qdec, qchi, qc2, qs2, qw, b0, b1, b2, b3, b4, b5,
-                                          b6, hist_at, row, T, X, nre, pd, vlgc, vxc);
+                                          b6, hist_at, hist_c, row, T, X, nre, pd, vlgc, vxc);
                     a0 = c0;
                     a1 = c1;
                     a2 = c2;
@@ -1106,7 +1127,7 @@ __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
                 }
                 if (k < np)
                     lc_pair<MODE, SHAPES, WEIGHTED>(P, valid, qra, qdec, qchi, qc2, qs2, qw, a0, a1, a2, a3, a4, a5,
-                                          a6, hist_at, row, T, X, nre, pd, vlgc, vxc);
+                                          a6, hist_at, hist_c, row, T, X, nre, pd, vlgc, vxc);
             }
             lc_hist_add<SHAPES, WEIGHTED>(pd);
         }
