@@ -52,9 +52,11 @@ __device__ __forceinline__ int xcd_run_block() {
 // Contiguous static ranges keep the histogram flushes few and neighbouring
 // items on one XCD.  Measured on the benchmark workloads: pair kernels
 // 20-27 % faster than a static split of the whole cost; with claims, a
-// 0.8 ms launch (lightcone1M) was 40 % slower, hence the static case.
+// 0.8 ms launch (lightcone1M) was 40 % slower, hence the static case.  Claims
+// from 2.5e5 instead of 4e5 units on: 140,000 shapes in 700,000 positions 6.33 ->
+// 5.54 ms, 200,000 in 400,000 5.27 -> 4.45 ms, 1,200,000 multipoles 8.7 -> 7.5 ms.
 constexpr int kScheduleUnits = 32;
-constexpr double kTailMinCost = 4.0e5;   // item-cost units per wave (about 5 ms of pair work)
+constexpr double kTailMinCost = 2.5e5;   // item-cost units per wave (about 3 ms of pair work)
 constexpr double kTailFineCost = 8.0e5;  // (about 10 ms)
 constexpr int64_t kTailItems = 16;       // items per unit below which groups of several waves take no chunks
 constexpr int kMaxWaves = 1 << 20;       // persistent waves per launch (tail counter stays in int)

@@ -1743,8 +1743,8 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     int wpb = kMaxWavesPerBlock;
     const size_t hs = A.hist_stride;
     const int pw = private_waves(thr_bytes, hs), most = std::min(4 * kPairWavesPerSimd, shared_waves(thr_bytes, hs));
-    const bool small = candidates < kTailMinCost * pw * cu_count;
-    const bool large = candidates > 10 * kTailMinCost * pw * cu_count;
+    const bool small = candidates < 0.8 * kTailMinCost * pw * cu_count;
+    const bool large = candidates > 16 * kTailMinCost * pw * cu_count;
     A.shared = !det && most > 0 && (small || (pw < most && (pw < kSharedBelow || large)));
     if (A.shared) {
         const size_t share = kLdsBytes / kPairWavesPerSimd - kPairStaticLds;
