@@ -35,7 +35,7 @@ constexpr int kBlockShapes = 64;
 constexpr int kItemPositions = 8192;
 constexpr int kMaxPosColumns = 4096;     // position columns per side (12-bit indices)
 
-constexpr int kSearchSteps = 24;         // column and slab counts tried per axis, about
+constexpr int kSearchSteps = 40;         // column and slab counts tried per axis, about
 
 struct Choice {
     int ncj, nzj, G, m;
