@@ -932,18 +932,33 @@ struct PairArgs {
     double *slot_sp, *slot_sx, *slot_dd, *slot_var;
 };
 
-// One bin of a wave's histogram.  A pending run keeps its slot's address and
-// the fields lie at constant offsets from it, so a flush computes no
-// addresses.
+// One bin of a histogram: S+D and SxD, then DD (weighted samples) and the sum of
+// e+^2 (variance requested), and the pair count.  Bins lie an odd number of 8-byte
+// words apart, so that those of a wave's lanes spread over all LDS banks (32 bytes
+// apart, three sums with their count, only every fourth pair of banks starts a
+// bin: 300,001 weighted positions, 100,003 shapes, 200 bins 14.6 ms of pair kernel,
+// now 12.0).  Two or four sums are padded to three or five words by the count; of
+// three, the counts lie in front of the sums, bin b's b + 1 words before them,
+// which also leaves LDS for more waves (360 weighted bins: 16 per CU instead of 12,
+// 21.9 -> 17.0 ms in 300,001 positions).
 template <bool WEIGHTED, bool VAR>
 struct Slot {
-    double sp, sx;                       // S+D, SxD
-    double more[WEIGHTED + VAR];         // DD (weighted samples), sum of e+^2 (variance requested)
-    uint32_t c, pad;
+    static constexpr int kSums = 2 + WEIGHTED + VAR;
+    static constexpr bool kApart = kSums == 3;
+    static constexpr uint32_t kBytes = kApart ? 24 : 8 * kSums + 8;
+    uint32_t c;
+    double v[kSums];  // S+D, SxD, [DD], [sum of e+^2]
 };
-static_assert(sizeof(Slot<false, false>) == 24 && sizeof(Slot<true, true>) == 40, "Slot layout");
-constexpr size_t slot_bytes(bool weighted, bool var) {
-    return sizeof(Slot<false, false>) + 8 * (size_t)(weighted + var);
+static_assert(Slot<false, false>::kBytes == 24 && Slot<true, true>::kBytes == 40, "hist_bytes");
+// bytes of a histogram of nbins bins
+constexpr size_t hist_bytes(int nbins, bool weighted, bool var) {
+    const size_t n = (size_t)nbins;
+    return ((weighted == var ? (weighted ? 40 : 24) * n : 24 * n + ((4 * n + 7) & ~(size_t)7)) + 15) & ~(size_t)15;
+}
+// bytes of the counts in front of the sums
+template <bool WEIGHTED, bool VAR>
+__device__ __forceinline__ int front_bytes(int nbins) {
+    return Slot<WEIGHTED, VAR>::kApart ? (4 * nbins + 7) & ~7 : 0;
 }
 
 // Shape record {a, b, l, ax, ay, e*w, w, 2*e*w} read through the scalar cache:
@@ -955,15 +970,18 @@ template <bool WEIGHTED, bool VAR>
 __device__ __forceinline__ Slot<WEIGHTED, VAR> take_bin(const PairArgs &P, char *hist, int copies, int b) {
     typedef Slot<WEIGHTED, VAR> BinSlot;
     BinSlot t{};
+    hist += front_bytes<WEIGHTED, VAR>(P.nbins);
     for (int k = 0; k < copies; ++k, hist += P.hist_stride) {
-        BinSlot *s = (BinSlot *)hist + b;
-        if (s->c == 0) continue;
-        t.c += s->c;
-        t.sp += s->sp;
-        t.sx += s->sx;
-        if constexpr (WEIGHTED) t.more[0] += s->more[0];
-        if constexpr (VAR) t.more[WEIGHTED ? 1 : 0] += s->more[WEIGHTED ? 1 : 0];
-        *s = BinSlot{};
+        double *v = (double *)(hist + (uint32_t)b * BinSlot::kBytes);
+        uint32_t *c = BinSlot::kApart ? (uint32_t *)hist - 1 - b : (uint32_t *)(v + BinSlot::kSums);
+        if (*c == 0) continue;
+        t.c += *c;
+        *c = 0;
+#pragma unroll
+        for (int i = 0; i < BinSlot::kSums; ++i) {
+            t.v[i] += v[i];
+            v[i] = 0.0;
+        }
     }
     return t;
 }
@@ -977,10 +995,10 @@ __device__ void flush_hist(const PairArgs &P, char *hist, int copies, const Samp
     for (int b = tid; b < B; b += nthr) {
         const Slot<WEIGHTED, VAR> t = take_bin<WEIGHTED, VAR>(P, hist, copies, b);
         const uint32_t c = t.c;
-        const double vsp = t.sp, vsx = t.sx;
+        const double vsp = t.v[0], vsx = t.v[1];
         double vdd = 0.0, vvr = 0.0;
-        if constexpr (WEIGHTED) vdd = t.more[0];
-        if constexpr (VAR) vvr = t.more[WEIGHTED ? 1 : 0];
+        if constexpr (WEIGHTED) vdd = t.v[2];
+        if constexpr (VAR) vvr = t.v[WEIGHTED ? 3 : 2];
         if (c == 0) continue;
         const int gb = b + P.bin_off;  // the pass's local bin in the output grid
         atomicAdd(&S.npairs[gb], (unsigned long long)c);
@@ -1018,10 +1036,10 @@ __device__ void flush_slot(const PairArgs &P, char *hist, int copies, int64_t sl
         const Slot<WEIGHTED, VAR> t = take_bin<WEIGHTED, VAR>(P, hist, copies, b);
         const int64_t o = slot * P.nbins_out + P.bin_off + b;
         P.slot_np[o] = t.c;
-        P.slot_sp[o] = t.sp;
-        P.slot_sx[o] = t.sx;
-        if constexpr (WEIGHTED) P.slot_dd[o] = t.more[0];
-        if constexpr (VAR) P.slot_var[o] = t.more[WEIGHTED ? 1 : 0];
+        P.slot_sp[o] = t.v[0];
+        P.slot_sx[o] = t.v[1];
+        if constexpr (WEIGHTED) P.slot_dd[o] = t.v[2];
+        if constexpr (VAR) P.slot_var[o] = t.v[WEIGHTED ? 3 : 2];
     }
     if (tid == 0) P.slot_key[slot] = key;
 }
@@ -1089,23 +1107,41 @@ enum { SH_NONE = 0, SH_CONST = 1, SH_WRAP = 2 };
 // summed in registers and reach the LDS histogram as one atomic per run,
 // which cuts the same-address collisions of the hot (outer r) bins.
 struct Pend {
-    uint32_t at;  // LDS address of the slot
+    uint32_t at;  // LDS address of the bin; counts in front of the sums: the bin's number
     uint32_t c;
     double sp, sx, dd, vr;
 };
 
 #define MIA_LDS __attribute__((address_space(3)))
 
+template <class T>
+__device__ __forceinline__ void lds_add(uint32_t at, T v) {
+    __hip_atomic_fetch_add((MIA_LDS T *)at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// hist: LDS address of the histogram's sums; with counts in front of them 4 bytes
+// less, so that no offset is negative.  The other kind of pending run holds its
+// bin's address, and a flush computes none.
 template <bool WEIGHTED, bool VAR>
-__device__ __forceinline__ void hist_add(const Pend &p) {
-    typedef MIA_LDS Slot<WEIGHTED, VAR> LdsSlot;
-    LdsSlot *s = (LdsSlot *)p.at;
-    __hip_atomic_fetch_add(&s->c, p.c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_add(&s->sp, p.sp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_add(&s->sx, p.sx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if constexpr (WEIGHTED)
-        __hip_atomic_fetch_add(&s->more[0], p.dd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if constexpr (VAR) __hip_atomic_fetch_add(&s->more[WEIGHTED ? 1 : 0], p.vr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+__device__ __forceinline__ uint32_t pend_at(uint32_t hist, int b) {
+    typedef Slot<WEIGHTED, VAR> BinSlot;
+    return BinSlot::kApart ? (uint32_t)b : __umul24(b, BinSlot::kBytes) + hist;
+}
+
+template <bool WEIGHTED, bool VAR>
+__device__ __forceinline__ void hist_add(uint32_t hist, const Pend &p) {
+    typedef Slot<WEIGHTED, VAR> BinSlot;
+    uint32_t at = p.at;
+    if constexpr (BinSlot::kApart) {
+        lds_add<uint32_t>((uint32_t)(__mul24((int)p.at, -4) + (int)hist), p.c);
+        at = __umul24(p.at, BinSlot::kBytes) + hist + 4;
+    } else {
+        lds_add<uint32_t>(at + 8 * BinSlot::kSums, p.c);
+    }
+    lds_add<double>(at, p.sp);
+    lds_add<double>(at + 8, p.sx);
+    if constexpr (WEIGHTED) lds_add<double>(at + 16, p.dd);
+    if constexpr (VAR) lds_add<double>(at + (WEIGHTED ? 24 : 16), p.vr);
 }
 
 template <int MODE, int SH, bool WEIGHTED, bool VAR, bool LZ>
@@ -1213,14 +1249,16 @@ __device__ __forceinline__ void one_pair(const PairArgs &P, const SampleView &S,
             ep = pw * ep;
             ex = pw * ex;
         }
-        const uint32_t at = __umul24(ir, row) + (__umul24(i2, (uint32_t)sizeof(Slot<WEIGHTED, VAR>)) + hist);
+        const uint32_t at = Slot<WEIGHTED, VAR>::kApart
+                                ? (uint32_t)(__mul24(ir, n_2) + i2)
+                                : __umul24(ir, row) + (__umul24(i2, Slot<WEIGHTED, VAR>::kBytes) + hist);
         double dd = WEIGHTED ? pw * qw : 0.0;
         double vr = VAR ? ep * ep : 0.0;
         // a new slot flushes the pending run; the run then restarts from this
         // pair: keep = 0 drops the old sums (fma(0, sum, x) = x, fma(1, sum, x)
         // = sum + x, both exactly as the plain assignment and addition)
         const bool nw = at != pd.at;
-        if (nw) hist_add<WEIGHTED, VAR>(pd);
+        if (nw) hist_add<WEIGHTED, VAR>(hist, pd);
         const double keep = nw ? 0.0 : 1.0;
         pd.at = at;
         pd.c = (nw ? 0u : pd.c) + 1u;
@@ -1301,8 +1339,8 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
     const int nb = walk.nb;
     iterations += (uint64_t)nb * ns;
     // an empty run adds its zeros to some bin, another one for every lane
-    const uint32_t row = (uint32_t)(P.n_2 * sizeof(Slot<WEIGHTED, VAR>));
-    Pend pd{hist + (uint32_t)((lane < P.nbins ? lane : 0) * sizeof(Slot<WEIGHTED, VAR>)), 0, 0, 0, 0, 0};
+    const uint32_t row = (uint32_t)P.n_2 * Slot<WEIGHTED, VAR>::kBytes;
+    Pend pd{pend_at<WEIGHTED, VAR>(hist, lane < P.nbins ? lane : 0), 0, 0, 0, 0, 0};
     // positions are loaded one batch ahead
     bool vn;
     const double2 *prn = (const double2 *)(S.prec + 4 * (int64_t)walk.position(0, lane, vn));
@@ -1350,7 +1388,7 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
             one_pair<MODE, SH, WEIGHTED, VAR, LZ>(P, S, v0, pa0, pb0, pl0, pw0, qa, qb, ql, qax, qay, qew, qw,
                                          q2ew, sha, shb, shl, hist, row, T, X, nre, pd, vlgc, vlg2, vxs, vxc);
     }
-    hist_add<WEIGHTED, VAR>(pd);
+    hist_add<WEIGHTED, VAR>(hist, pd);
 }
 
 // An item's pair loop for its periodic-shift variant.
@@ -1392,7 +1430,6 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     for (int i = threadIdx.x; i < P.n_r + 1; i += blockDim.x) T[i] = P.T[i];
     for (int i = threadIdx.x; i < nx; i += blockDim.x) X[i] = P.X[i];
     size_t thr_bytes = ((size_t)(P.n_r + 1 + nx) * 8 + 15) & ~(size_t)15;
-    typedef Slot<WEIGHTED, VAR> BinSlot;
     char *hist0 = lds + thr_bytes;
     const int nhist = shared ? P.copies : (int)(blockDim.x / kWave);
     for (int i = threadIdx.x * 4; i < nhist * P.hist_stride; i += blockDim.x * 4) *(uint32_t *)(hist0 + i) = 0u;
@@ -1416,7 +1453,8 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     const int tid = shared ? threadIdx.x : lane, nthr = shared ? blockDim.x : kWave;
     char *hist = hist0 + (shared ? 0 : wv * P.hist_stride);
     const int place = ((lane & 7) << 3) | (lane >> 3);
-    const uint32_t hist_at = (uint32_t)(uintptr_t)(MIA_LDS char *)(hist + (shared ? place % P.copies : 0) * P.hist_stride);
+    const uint32_t hist_at = (uint32_t)(uintptr_t)(MIA_LDS char *)(hist + (shared ? place % P.copies : 0) * P.hist_stride) +
+                             front_bytes<WEIGHTED, VAR>(P.nbins) - (Slot<WEIGHTED, VAR>::kApart ? 4 : 0);
     // a contiguous share of the cost-sorted items, then tail chunks from the counter
     const WaveSchedule sch = make_schedule(P.bounds, shared ? (int)gridDim.x : P.n_waves);
     int64_t it0, it1;
@@ -1558,7 +1596,7 @@ void launch_pairs_mode(const PairArgs &A, unsigned grid, int wpb, size_t lds, hi
 
 // LDS bytes of one wave's histogram (one copy) and of the block's thresholds.
 size_t wave_hist_bytes(const mia_bins &bins, bool weighted) {
-    return ((size_t)bins.n_r * bins.n_2 * slot_bytes(weighted, bins.accumulate_variance) + 15) & ~(size_t)15;
+    return hist_bytes(bins.n_r * bins.n_2, weighted, bins.accumulate_variance);
 }
 
 size_t threshold_bytes(const mia_bins &bins) {
@@ -1718,7 +1756,7 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     // one histogram copy per wave: the pending-slot registers already absorb
     // most same-address collisions, and one copy leaves LDS for 8 waves per
     // SIMD (2 copies measured 20 % slower); mia_tuning.hist_copies is ignored
-    A.hist_stride = (int)(((size_t)Bp * slot_bytes(A.weighted, A.var) + 15) & ~(size_t)15);
+    A.hist_stride = (int)hist_bytes(Bp, A.weighted, A.var);
     // A private histogram per wave (one copy: the pending-slot registers already
     // absorb most same-address collisions), or one per workgroup, shared by its
     // four waves, in as many copies (at most 4) as leave room for
