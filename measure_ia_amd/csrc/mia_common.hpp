@@ -101,11 +101,21 @@ __device__ __forceinline__ WaveSchedule make_schedule(const int64_t *bounds, int
 
 // bounds[0..waves * kScheduleUnits + 2] of the schedule above, on stream st.
 void schedule_bounds(const int64_t *cost_prefix, int64_t n, int waves, int64_t *bounds, hipStream_t st);
-// the same with the item count read on the device; all_static: every wave
-// takes only its static range (no tail claims), so the item -> wave map is
-// fixed by the costs
-void schedule_bounds(const int64_t *cost_prefix, const int64_t *n_dev, int waves, int64_t *bounds,
-                     hipStream_t st, bool all_static = false, int waves_per_unit = 1);
+// The same with the item count read on the device and bounds inside items: an
+// item costs kItemOverhead and as much for each of its batches (64 of its
+// positions, np[np_stride * i] in all), and bounds[u] = i << kBatchBits | b is the
+// first batch, b of item i, that starts at cost u C / U or later.  `waves` units
+// of kScheduleUnits, each worked on by waves_per_unit waves.  all_static: no tail
+// claims, so the batch -> wave map is fixed by the costs.
+// A unit costs at least kMinUnitCost, and the last groups of a tiny count take
+// nothing: every busy one adds its histogram to the same few hundred sums (2,000
+// galaxies, 160 bins: pair kernel 45 us without the bound, now 21).
+constexpr double kMinUnitCost = 160.0;
+constexpr int kBatchBits = 26;           // batches of an item: below 2^31 / 64
+constexpr int64_t kItemOverhead = 1024;  // per-item cost, in pair evaluations (256: a batch of eight uneven samples
+                                         // 4.8 ms of pair kernel, 512 4.1, 1024 3.6; 317,811 galaxies equal)
+void schedule_batches(const int64_t *cost_prefix, const int64_t *n_dev, const int32_t *np, int np_stride, int waves,
+                      int64_t *bounds, hipStream_t st, bool all_static, int waves_per_unit);
 
 constexpr int kMaxBins2 = 256;      // max n_2 (pi or mu bins)
 constexpr int kMaxBinsR = 256;      // max n_r

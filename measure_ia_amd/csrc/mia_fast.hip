@@ -12,16 +12,16 @@
 //               make a work item.  Items are counting-sorted by
 //               (sample, R_s, R_p).
 //   2. pairs  : a persistent grid takes contiguous runs of the sorted list,
-//               balanced by estimated cost, then claims tail chunks from a
-//               counter.  Each lane looks up the positions of one column of an
-//               item; the wave then reads its shape block through the scalar
-//               cache (one 64-byte record per shape, wave-uniform) and streams
-//               the positions through registers, 64 at a time.  Separations
-//               are the reference's own FP64 differences, so r_p^2 (or r^2)
-//               and pi are compared exactly with the host-bisected thresholds
-//               (an FP32 log2 only guesses the bin); e+ and ex are FP64 (CDNA4
-//               runs FP64 FMA at the rate of non-packed FP32) and go into an
-//               LDS histogram (a wave's own, or shared by a workgroup) with
+//               balanced by estimated cost to a batch of 64 positions, then
+//               claims tail chunks from a counter.  Each lane looks up the
+//               positions of one column of an item; the wave then reads its
+//               shape block through the scalar cache (one 64-byte record per
+//               shape, wave-uniform) and streams the positions through
+//               registers, 64 at a time.  Separations are the reference's own
+//               FP64 differences, so r_p^2 (or r^2) and pi are compared exactly
+//               with the host-bisected thresholds (an FP32 log2 only guesses
+//               the bin); e+ and ex are FP64 (CDNA4 runs FP64 FMA at the rate
+//               of non-packed FP32) and go into an LDS histogram (a wave's own, or shared by a workgroup) with
 //               LDS atomics.  mu = pi/r is screened in FP32 and recomputed in
 //               FP64 when it lies within a guard band of a bin edge; the
 //               arccos NaN rule is likewise checked in FP64 for nearly
@@ -52,6 +52,7 @@ constexpr size_t kLdsBytes = 160 * 1024;         // LDS per CU (gfx950)
 constexpr size_t kPairStaticLds = 64;            // the pair kernel's own LDS words, at most
 constexpr int kStatCopies = 32, kStatStride = 16;  // copies of the pair kernel's statistics, words apart
 constexpr int kSharedBelow = 16;                 // private waves per CU below which histograms are shared
+constexpr int kSplitItems = 32;                  // items per group of four waves below which a claim is a quarter of an item
 constexpr int kPairWavesPerSimd = 6;             // waves per SIMD the pair kernel's registers allow
 constexpr int64_t kMaxKeysPerSample = 1 << 24;   // K^2 planner keys per sample (K regions)
 constexpr double kSinExact = 1e-5;  // FP64 arccos-domain check when |sin phi| < 1e-5 |cos phi|
@@ -275,7 +276,6 @@ constexpr int kPlanThreads = 256;
 constexpr int kPlanWaves = kPlanThreads / kWave;
 constexpr int kPlanGridPerCu = 8;        // workgroups per CU of the planner's persistent grids
 constexpr int kItemPositions = 8192;    // positions of an item, about
-constexpr int64_t kItemOverhead = 256;  // per-item cost, in pair evaluations
 // Segments a block's reach falls into along one axis: the sub-boxes it meets
 // (at most one of them twice, where the periodic image closes on itself) plus
 // the changes of shift class (-L, mixed, none, mixed, +L).
@@ -696,10 +696,9 @@ __global__ void k_finalize(const FinSample *fs, const int64_t *fin0, int S, cons
 
 // Deterministic reduction, step 1: the histogram flushes of every wave of an
 // all-static schedule (bounds from schedule_bounds(all_static)), which are the
-// distinct planner keys among its items: the non-empty keys from key(i0) to
-// key(i1 - 1) over its range [i0, i1) of the key-sorted items (key_off:
-// nkeys + 1 item offsets), 0 for an empty range.  Their exclusive scan
-// numbers the slots.
+// distinct planner keys among its items: the non-empty keys from the first to
+// the last item that its range of batches touches (key_off: nkeys + 1 item
+// offsets), 0 for an empty range.  Their exclusive scan numbers the slots.
 __device__ __forceinline__ int64_t key_of_item(const int64_t *key_off, int64_t nkeys, int64_t i) {
     int64_t lo = 0, hi = nkeys - 1;  // largest k with key_off[k] <= i
     while (lo < hi) {
@@ -719,12 +718,18 @@ __global__ void k_key_nonempty(const int64_t *key_off, int64_t nkeys, int64_t *n
     if (k < nkeys) ne[k] = key_off[k + 1] > key_off[k] ? 1 : 0;
 }
 
+// The item after the last one of which a range of batches that ends at b takes some.
+__device__ __forceinline__ int64_t items_end(int64_t b) {
+    return (b >> kBatchBits) + ((b & ((1ll << kBatchBits) - 1)) != 0 ? 1 : 0);
+}
+
 __global__ void k_slot_runs(const int64_t *bounds, int W, const int64_t *key_off, int64_t nkeys,
                             const int64_t *ne_pre, int64_t *runs) {
     const int w = blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= W) return;
-    const int64_t i0 = bounds[(int64_t)w * kScheduleUnits], i1 = bounds[(int64_t)(w + 1) * kScheduleUnits];
-    runs[w] = i1 > i0 ? ne_pre[key_of_item(key_off, nkeys, i1 - 1) + 1] - ne_pre[key_of_item(key_off, nkeys, i0)]
+    const int64_t b0 = bounds[(int64_t)w * kScheduleUnits], b1 = bounds[(int64_t)(w + 1) * kScheduleUnits];
+    const int64_t i0 = b0 >> kBatchBits, i1 = items_end(b1);
+    runs[w] = b1 > b0 ? ne_pre[key_of_item(key_off, nkeys, i1 - 1) + 1] - ne_pre[key_of_item(key_off, nkeys, i0)]
                       : 0;
 }
 
@@ -1281,7 +1286,8 @@ struct ColumnWalk {
     int c, base, ce;    // the column the lane reads from
     int np, nb;
 
-    __device__ __forceinline__ void begin(int lane, int pb_, int n) {
+    // batches are read from bt0 on, in ascending order
+    __device__ __forceinline__ void begin(int lane, int pb_, int n, int bt0) {
         end = n;
 #pragma unroll
         for (int d = 1; d < kWave; d <<= 1) {
@@ -1292,7 +1298,7 @@ struct ColumnWalk {
         np = __builtin_amdgcn_readlane(end, kWave - 1);
         nb = (np + kWave - 1) / kWave;
         // the first column that ends past the lane's first coordinate
-        const int k = lane * nb < np ? lane * nb : np - 1;
+        const int k = lane * nb + bt0 < np ? lane * nb + bt0 : np - 1;
         c = 0;
 #pragma unroll
         for (int d = kWave / 2; d > 0; d >>= 1) c += __shfl(end, c + d - 1) <= k ? d : 0;
@@ -1314,7 +1320,7 @@ struct ColumnWalk {
 };
 
 template <int MODE, int SH, bool WEIGHTED, bool VAR, bool LZ>
-__device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S, int cpb, int cn,
+__device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S, int cpb, int cn, int bt0, int bt1,
                                          int shifts, ShapePtr shp, int ns, uint32_t hist,
                                          const double *T, const double *X, int lane,
                                          uint32_t &nre, uint64_t &iterations) {
@@ -1335,20 +1341,19 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
         asm volatile("v_mov_b32 %0, %1" : "=v"(vlg2) : "s"(P.xc));
     }
     ColumnWalk walk;
-    walk.begin(lane, cpb, cn);
-    const int nb = walk.nb;
-    iterations += (uint64_t)nb * ns;
+    walk.begin(lane, cpb, cn, bt0);
+    iterations += (uint64_t)(bt1 - bt0) * ns;
     // an empty run adds its zeros to some bin, another one for every lane
     const uint32_t row = (uint32_t)P.n_2 * Slot<WEIGHTED, VAR>::kBytes;
     Pend pd{pend_at<WEIGHTED, VAR>(hist, lane < P.nbins ? lane : 0), 0, 0, 0, 0, 0};
     // positions are loaded one batch ahead
     bool vn;
-    const double2 *prn = (const double2 *)(S.prec + 4 * (int64_t)walk.position(0, lane, vn));
+    const double2 *prn = (const double2 *)(S.prec + 4 * (int64_t)walk.position(bt0, lane, vn));
     double2 abn = prn[0], lwn = prn[1];
-    for (int bt = 0; bt < nb; ++bt) {
+    for (int bt = bt0; bt < bt1; ++bt) {
         const bool v0 = vn;
         const double2 ab = abn, lw = lwn;
-        if (bt + 1 < nb) {
+        if (bt + 1 < bt1) {
             prn = (const double2 *)(S.prec + 4 * (int64_t)walk.position(bt + 1, lane, vn));
             abn = prn[0];
             lwn = prn[1];
@@ -1391,34 +1396,41 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
     hist_add<WEIGHTED, VAR>(hist, pd);
 }
 
-// An item's pair loop for its periodic-shift variant.
+// The batches [bt0, bt1) of an item, in the pair loop for its periodic-shift variant.
 template <int MODE, bool WEIGHTED, bool VAR, bool LZ>
-__device__ __forceinline__ void run_shifted(const PairArgs &P, const SampleView &S, int cpb, int cn,
+__device__ __forceinline__ void run_shifted(const PairArgs &P, const SampleView &S, int cpb, int cn, int bt0, int bt1,
                                             int shifts, ShapePtr shp, int ns, uint32_t hist, const double *T,
                                             const double *X, int lane, uint32_t &nre, uint64_t &iterations) {
     if (shifts & 64)
-        run_item<MODE, SH_WRAP, WEIGHTED, VAR, LZ>(P, S, cpb, cn, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_WRAP, WEIGHTED, VAR, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
                                                    iterations);
     else if (shifts & 63)
-        run_item<MODE, SH_CONST, WEIGHTED, VAR, LZ>(P, S, cpb, cn, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_CONST, WEIGHTED, VAR, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
                                                     iterations);
     else
-        run_item<MODE, SH_NONE, WEIGHTED, VAR, LZ>(P, S, cpb, cn, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_NONE, WEIGHTED, VAR, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
                                                    iterations);
 }
 
-// Persistent groups of waves over the cost-balanced, key-sorted items.  A group
-// works on the items of one key at a time and adds into its histogram, which
-// goes to the key's sums when the key changes.  A group is one wave; or, where
-// private histograms would leave too few waves per CU (P.shared), the four
-// waves of a workgroup, which take a key's items from a counter in LDS and
-// share P.copies copies of one histogram, a lane adding into the copy of its
-// place (so neighbouring lanes, which often hit one bin, hit different
-// addresses).
+// Persistent groups of waves over the cost-balanced batches of the key-sorted
+// items (a share may begin and end inside an item, so its length does not hang on
+// the largest item: 20,000 weighted clustered galaxies and 5,000 shapes in a box
+// of 75, 1,500 items for 6,144 waves, 0.83 ms of pair kernel with whole items, now
+// 0.13).  A group works on the items of one key at a time and adds into its
+// histogram, which goes to the key's sums when the key changes.  A group is one
+// wave; or, where private histograms would leave too few waves per CU (P.shared),
+// the four waves of a workgroup, which claim the items of a key from a counter in
+// LDS and share P.copies copies of one histogram, a lane adding into the copy of
+// its place (so neighbouring lanes, which often hit one bin, hit different
+// addresses).  With few items per group a claim is a quarter of an item's batches;
+// with many whole items even the waves out, and the empty claims of small items
+// cost more (a batch of samples with 91 items per group, 1.5 against 2.1 ms;
+// 2,000,000 multipoles 196 against 204).
 template <int MODE, bool WEIGHTED, bool VAR>
 __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs P) {
     extern __shared__ __align__(16) char lds[];
-    __shared__ int s_next[2], s_chunk, s_left;
+    __shared__ unsigned s_next[2];
+    __shared__ int s_chunk, s_left;
     __shared__ unsigned long long s_stat[3];
     const int lane = threadIdx.x & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -1455,15 +1467,15 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     const int place = ((lane & 7) << 3) | (lane >> 3);
     const uint32_t hist_at = (uint32_t)(uintptr_t)(MIA_LDS char *)(hist + (shared ? place % P.copies : 0) * P.hist_stride) +
                              front_bytes<WEIGHTED, VAR>(P.nbins) - (Slot<WEIGHTED, VAR>::kApart ? 4 : 0);
-    // a contiguous share of the cost-sorted items, then tail chunks from the counter
+    // a contiguous share of the cost, then tail chunks from the counter
     const WaveSchedule sch = make_schedule(P.bounds, shared ? (int)gridDim.x : P.n_waves);
-    int64_t it0, it1;
+    int64_t it0, it1;  // item << kBatchBits | batch
     sch.first(shared ? wg : (wave < P.n_waves ? wave : 0), it0, it1);
-    if (!shared && wave >= P.n_waves) it1 = it0;
+    const bool idle = wave >= P.n_waves;
+    const bool split = n_items < (int64_t)kSplitItems * gridDim.x;  // (shared)
+    if (!shared && idle) it1 = it0;
     it0 = uniform64(it0);
     it1 = uniform64(it1);
-    const MIA_CONST int32_t *items = (const MIA_CONST int32_t *)P.items;
-    const MIA_CONST int32_t *blocks = (const MIA_CONST int32_t *)P.blocks;
     int cur_key = -1, flushes = 0, par = 0;
     uint32_t nre = 0;
     uint64_t iterations = 0;  // wave-uniform
@@ -1474,11 +1486,20 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
         else
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     };
+    // The arguments that only the code around the pair loop needs, read again
+    // where they are needed: held in scalar registers across the pair loop they
+    // push its own out into vector lanes
+    auto args = [] {
+        const MIA_CONST PairArgs *q = (const MIA_CONST PairArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(q));
+        return q;
+    };
     // the histogram goes to its key's sums, the next adds are for `key` (every
     // thread of the group, with no adds in flight)
     auto turn_to = [&](int key) {
         if (cur_key >= 0) {
             sync();
+            const PairArgs &P = *(const PairArgs *)args();
             const int kk = P.K1 * P.K1;
             const int sample = cur_key / kk, in = cur_key - sample * kk;
             const int rs = in / P.K1, rp = in - rs * P.K1;
@@ -1493,48 +1514,72 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     };
 
     while (true) {
-        for (int64_t it = it0; it < it1;) {
+        it0 = uniform64(it0);
+        it1 = uniform64(it1);
+        const int i0 = (int)(it0 >> kBatchBits), i1 = (int)(it1 >> kBatchBits);
+        const int b0 = (int)(it0 & ((1 << kBatchBits) - 1)), b1 = (int)(it1 & ((1 << kBatchBits) - 1));
+        const int end = it1 > it0 ? i1 + (b1 > 0 ? 1 : 0) : i0;
+        for (int it = i0; it < end;) {
             // the items [it, se) of one key
-            const int key = __builtin_amdgcn_readfirstlane(items[8 * it + 7]);
-            const int64_t ke = ((const MIA_CONST int64_t *)P.key_off)[key + 1];
-            const int64_t se = uniform64(ke < it1 ? ke : it1);
+            const MIA_CONST PairArgs *Q = args();
+            const int key = __builtin_amdgcn_readfirstlane(((const MIA_CONST int32_t *)Q->items)[8 * (int64_t)it + 7]);
+            const int ke = (int)((const MIA_CONST int64_t *)Q->key_off)[key + 1];
+            const int se = __builtin_amdgcn_readfirstlane(ke < end ? ke : end);
             if (key != cur_key) turn_to(key);
-            int64_t i = it;
-            while (true) {
+            for (int j = it;; ++j) {
+                // shared: an item is one claim, or four, its quarters (all of it and
+                // three empty ones where it is a single batch)
+                int quarter = 0;
                 if (shared) {
-                    int t = 0;
-                    if (lane == 0) t = wave < P.n_waves ? atomicAdd(&s_next[par], 1) : 0x7fffffff;
-                    i = it + __builtin_amdgcn_readfirstlane(t);
+                    if (idle) break;
+                    unsigned t = 0;
+                    if (lane == 0) t = atomicAdd(&s_next[par], 1u);
+                    t = __builtin_amdgcn_readfirstlane(t);
+                    j = it + (int)(split ? t >> 2 : t);
+                    quarter = split ? t & 3 : 0;
                 }
-                // (the compiler does not see that i is wave-uniform; vector
+                // (the compiler does not see that the item is wave-uniform; vector
                 // loads of the shape records would cost 70 registers)
-                i = uniform64(i);
+                const int i = __builtin_amdgcn_readfirstlane(j);
                 if (i >= se) break;
-                const MIA_CONST int32_t *ip = items + 8 * i;
-                ++i;
-                if (ip[6] == 0) continue;  // no column of the item is in reach
+                const MIA_CONST PairArgs *Q = args();
+                const MIA_CONST int32_t *ip = (const MIA_CONST int32_t *)Q->items + 8 * (int64_t)i;
+                int bt0 = i == i0 ? b0 : 0;
+                int bt1 = i == i1 ? b1 : (ip[6] + kWave - 1) / kWave;
+                if (shared) {
+                    const int n = bt1 - bt0;
+                    if (split && n > 1) {
+                        bt1 = bt0 + (n * (quarter + 1) >> 2);
+                        bt0 += n * quarter >> 2;
+                    } else if (quarter) {
+                        continue;
+                    }
+                }
+                bt0 = __builtin_amdgcn_readfirstlane(bt0);
+                bt1 = __builtin_amdgcn_readfirstlane(bt1);
+                if (bt0 >= bt1) continue;  // (no batch: no column of the item is in reach)
                 const int blk = ip[0], w = ip[1], jj = ip[2], wn = ip[3], c0 = ip[4], kk = ip[5];
                 const int shifts = (w >> 16) & 0xff;
-                const MIA_CONST int32_t *bp = blocks + 6 * (int64_t)blk;
+                const MIA_CONST int32_t *bp = (const MIA_CONST int32_t *)Q->blocks + 6 * (int64_t)blk;
                 const int s0 = bp[0], ns = bp[1], sample = bp[4];
-                const SampleView S = load_view(P.samples + sample);
+                const SampleView S = load_view(Q->samples + sample);
                 ShapePtr shp = (ShapePtr)(S.srec + 8 * (int64_t)s0);
                 int cpb, cn;
                 {
-                    const MIA_CONST double *bc = (const MIA_CONST double *)P.bbox + 6 * (int64_t)blk;
+                    const MIA_CONST double *bc = (const MIA_CONST double *)Q->bbox + 6 * (int64_t)blk;
                     const double bb[6] = {bc[0], bc[1], bc[2], bc[3], bc[4], bc[5]};
-                    item_column(column_view((const MIA_CONST PlanSample *)P.ps + sample), bb, jj & 0xffff,
+                    item_column(column_view((const MIA_CONST PlanSample *)Q->ps + sample), bb, jj & 0xffff,
                                 (jj >> 16) & 0xffff, wn & 0xffff, (wn >> 16) & 0xffff, c0, kk & 0xffff,
                                 (kk >> 16) & 0xffff, w, lane, cpb, cn);
                 }
                 // (r, mu) sums r^2 in an order fixed by the line of sight: one
                 // loop per order, so the pair loop holds no branch on it
                 if (MODE == MIA_RMU && S.los != 2)
-                    run_shifted<MODE, WEIGHTED, VAR, false>(P, S, cpb, cn, shifts, shp, ns, hist_at, T, X, lane, nre,
-                                                            iterations);
+                    run_shifted<MODE, WEIGHTED, VAR, false>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist_at, T, X,
+                                                            lane, nre, iterations);
                 else
-                    run_shifted<MODE, WEIGHTED, VAR, true>(P, S, cpb, cn, shifts, shp, ns, hist_at, T, X, lane, nre,
-                                                           iterations);
+                    run_shifted<MODE, WEIGHTED, VAR, true>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist_at, T, X,
+                                                           lane, nre, iterations);
             }
             if (shared) {
                 __syncthreads();
@@ -1546,10 +1591,10 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
             it = se;
         }
         if (!shared) {
-            if (wave >= P.n_waves || !sch.next(P.queue, lane, it0, it1)) break;
+            if (idle || !sch.next(args()->queue, lane, it0, it1)) break;
         } else {
             if (sch.tail == 0) break;
-            if (threadIdx.x == 0) s_chunk = atomicAdd(P.queue, 1);
+            if (threadIdx.x == 0) s_chunk = atomicAdd(args()->queue, 1);
             __syncthreads();
             const int k = __builtin_amdgcn_readfirstlane(s_chunk);
             __syncthreads();
@@ -1564,7 +1609,7 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     if (lane == 0) {
         if (iterations) atomicAdd(&s_stat[1], (unsigned long long)iterations);
         if (__hip_atomic_fetch_add(&s_left, -1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 1 && s_stat[1]) {
-            unsigned long long *st = P.stat + (wg % kStatCopies) * kStatStride;
+            unsigned long long *st = args()->stat + (wg % kStatCopies) * kStatStride;
             atomicAdd(&st[0], s_stat[0]);
             atomicAdd(&st[1], s_stat[1]);
             atomicMax(&st[2], ~s_stat[2]);
@@ -2256,7 +2301,8 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
         cost = p.cost2;
     }
     scan_ws<int64_t>(cost, p.cpre, p.item_cap, p.n_items, p.scan_cost, st);
-    schedule_bounds(p.cpre, p.n_items, p.pc.groups, p.bounds, st, p.det, p.pc.A.shared ? p.pc.wpb : 1);
+    schedule_batches(p.cpre, p.n_items, &items->np, sizeof(Item) / sizeof(int32_t), p.pc.groups, p.bounds, st, p.det,
+                     p.pc.A.shared ? p.pc.wpb : 1);
     if (p.det) {
         // slot numbers of every wave's flushes (slot0[W] = slots in all)
         hipLaunchKernelGGL(k_key_nonempty, dim3(nblk(p.nkeys, 256)), dim3(256), 0, st, (const int64_t *)p.ko,

@@ -29,13 +29,14 @@ __global__ void k_fill(T *p, T v, int64_t n) {
 
 // bounds[u] = first i in [0, n] with cost_prefix[i] * U >= u * C, for u in
 // [0, U]; bounds[U + 1], bounds[U + 2] = static units per wave and units per
-// tail chunk.
-__global__ void k_schedule_bounds(const int64_t *cpre, int64_t n_host, const int64_t *n_dev, int64_t U,
-                                  int waves_per_unit, int all_static, int64_t *bounds) {
+// tail chunk.  With np: the first batch that starts there (schedule_batches).
+__global__ void k_schedule_bounds(const int64_t *cpre, int64_t n_host, const int64_t *n_dev, const int32_t *np,
+                                  int np_stride, int64_t U, int waves_per_unit, int all_static, int64_t *bounds) {
     const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (u > U + 2) return;
     const int64_t n = n_dev ? *n_dev : n_host;
-    const double C = (double)cpre[n], Ud = (double)U, t = (double)u * C;
+    const double C = (double)cpre[n];
+    const double Ud = np ? fmin((double)U, fmax(1.0, C / kMinUnitCost)) : (double)U, t = fmin((double)u, Ud) * C;
     if (u > U) {
         // a group of several waves waits for its slowest at the end of every
         // chunk: its chunks hold at least kTailItems items or it takes none
@@ -55,6 +56,21 @@ __global__ void k_schedule_bounds(const int64_t *cpre, int64_t n_host, const int
             hi = mid;
         else
             lo = mid + 1;
+    }
+    if (np) {
+        int64_t b = 0;
+        // item lo - 1 may hold the boundary
+        if (lo > 0) {
+            const int64_t i = lo - 1, nb = (np[np_stride * i] + kWave - 1) / kWave;
+            const double at = t / Ud - (double)cpre[i] - (double)kItemOverhead;
+            const double per = (double)(cpre[lo] - cpre[i] - kItemOverhead) / (double)(nb > 0 ? nb : 1);
+            b = at > 0.0 ? (int64_t)fmin(ceil(at / per), (double)nb) : 0;
+            if (b < nb)
+                lo = i;
+            else
+                b = 0;
+        }
+        lo = lo << kBatchBits | b;
     }
     bounds[u] = lo;
 }
@@ -342,14 +358,14 @@ void fill(T *p, T v, int64_t n, hipStream_t st) {
 void schedule_bounds(const int64_t *cost_prefix, int64_t n, int waves, int64_t *bounds, hipStream_t st) {
     const int64_t U = (int64_t)waves * kScheduleUnits;
     hipLaunchKernelGGL(k_schedule_bounds, dim3((unsigned)((U + 3 + 255) / 256)), dim3(256), 0, st, cost_prefix,
-                       n, (const int64_t *)nullptr, U, 1, 0, bounds);
+                       n, (const int64_t *)nullptr, (const int32_t *)nullptr, 0, U, 1, 0, bounds);
     MIA_HIP(hipGetLastError());
 }
-void schedule_bounds(const int64_t *cost_prefix, const int64_t *n_dev, int waves, int64_t *bounds,
-                     hipStream_t st, bool all_static, int waves_per_unit) {
+void schedule_batches(const int64_t *cost_prefix, const int64_t *n_dev, const int32_t *np, int np_stride, int waves,
+                      int64_t *bounds, hipStream_t st, bool all_static, int waves_per_unit) {
     const int64_t U = (int64_t)waves * kScheduleUnits;
     hipLaunchKernelGGL(k_schedule_bounds, dim3((unsigned)((U + 3 + 255) / 256)), dim3(256), 0, st, cost_prefix,
-                       (int64_t)0, n_dev, U, waves_per_unit, all_static ? 1 : 0, bounds);
+                       (int64_t)0, n_dev, np, np_stride, U, waves_per_unit, all_static ? 1 : 0, bounds);
     MIA_HIP(hipGetLastError());
 }
 
