@@ -741,9 +741,32 @@ __device__ __forceinline__ void neumaier(double &s, double &c, double v) {
     s = t;
 }
 
-// Deterministic reduction, step 2: the slots of one key are consecutive; the
-// first one (its head) takes their sum, and the second, where there is one, the
-// sum's compensation, bin by bin.
+// Deterministic reduction, step 2: the slots of one key are consecutive and are
+// cut into pieces of kPieceSlots from the key's first; the first slot of a piece
+// (its head) takes the piece's sum, and the second, where there is one, the sum's
+// compensation, bin by bin.  One workgroup per piece and 256 bins: a count
+// without regions has all its waves' slots in one key (200,000 positions, 6,144
+// slots of 200 bins: 4.3 ms of finalisation in one workgroup, now 0.15).
+constexpr int kPieceSlots = 32;
+
+// The key's first slot.
+__device__ __forceinline__ int64_t first_slot(const int64_t *slot_key, int64_t n, int64_t key) {
+    int64_t lo = 0, hi = n;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (slot_key[mid] < key)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// Whether slot q is a head.
+__device__ __forceinline__ bool head_slot(const int64_t *slot_key, int64_t n, int64_t q) {
+    return (q - first_slot(slot_key, n, slot_key[q])) % kPieceSlots == 0;
+}
+
 __device__ __forceinline__ void sum_run(double *slot, int64_t o, int64_t step, int n) {
     double s = slot[o], c = 0.0;
     for (int k = 1; k < n; ++k) neumaier(s, c, slot[o + k * step]);
@@ -756,12 +779,12 @@ __global__ __launch_bounds__(256) void k_sum_slots(const int64_t *slot_total, co
                                                    double *slot_dd, double *slot_var, int BO) {
     const int64_t n = *slot_total;
     for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
+        if (!head_slot(slot_key, n, q)) continue;
         const int64_t key = slot_key[q];
-        if (q > 0 && slot_key[q - 1] == key) continue;
         int run = 1;
-        while (q + run < n && slot_key[q + run] == key) ++run;
+        while (run < kPieceSlots && q + run < n && slot_key[q + run] == key) ++run;
         if (run == 1) continue;
-        for (int b = threadIdx.x; b < BO; b += blockDim.x) {
+        for (int b = blockIdx.y * blockDim.x + threadIdx.x; b < BO; b += gridDim.y * blockDim.x) {
             const int64_t o = q * BO + b;
             unsigned long long c = slot_np[o];
             for (int k = 1; k < run; ++k) c += slot_np[o + (int64_t)k * BO];
@@ -784,7 +807,7 @@ __global__ __launch_bounds__(1024) void k_slot_heads(const int64_t *slot_total, 
     int64_t base = 0;
     for (int64_t q0 = 0; q0 < n; q0 += blockDim.x) {
         const int64_t q = q0 + threadIdx.x;
-        const bool head = q < n && (q == 0 || slot_key[q - 1] != slot_key[q]);
+        const bool head = q < n && head_slot(slot_key, n, q);
         const uint64_t m = __ballot(head);
         if (lane == 0) s_cnt[wv] = __popcll(m);
         __syncthreads();
@@ -803,7 +826,7 @@ __global__ __launch_bounds__(1024) void k_slot_heads(const int64_t *slot_total, 
     if (threadIdx.x == 0) *n_heads = base;
 }
 
-// Step 3: caller outputs from the keys' sums, one wave per output.  Output
+// Step 3: caller outputs from the pieces' sums, one wave per output.  Output
 // element (tally t, bin b) of a sample sums the heads of that sample whose key
 // (R_s, R_p) includes region t - 1 (every head for t = 0): lane l every 64th
 // from the l-th, then the lanes pairwise, all with compensated FP64 sums, in an
@@ -2359,7 +2382,7 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
     if (p.det) {
         const int64_t *slots = p.slot0 + p.pc.waves;  // their number
         const unsigned sgrid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(p.slot_cap, 8192));
-        hipLaunchKernelGGL(k_sum_slots, dim3(sgrid), dim3(256), 0, st, slots, (const int64_t *)p.slot_key, p.slot_np,
+        hipLaunchKernelGGL(k_sum_slots, dim3(sgrid, nblk(n_r * n_2, 256)), dim3(256), 0, st, slots, (const int64_t *)p.slot_key, p.slot_np,
                            p.slot_sp, p.slot_sx, p.slot_dd, p.slot_var, n_r * n_2);
         MIA_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_slot_heads, dim3(1), dim3(1024), 0, st, slots, (const int64_t *)p.slot_key, p.heads,
