@@ -8,14 +8,23 @@
 //   runs  : once per block and position, the lane's pending histogram run ends;
 //   bodies: the pairs whose column touches the domain of their shape (bins,
 //           e+ and ex, the histogram);
-//   items : the column lookup and the planner's work per item.
+//   wraps : tests whose separation takes the minimum image pair by pair, where a
+//           block and a slab or column straddle half the box;
+//   items : the column lookup and the planner's work per item;
+//   blocks: the planner's and the scalar loads' work per shape block.
 // Thin position columns cut tests and bodies near the edge of the domain and
 // add items (at most 64 columns each); small blocks cut tests and add runs and
 // items.  The areas that columns of width f cover around a block or a shape are
 // those of the Minkowski sums (for a convex outline of area A and perimeter p
 // on a square grid, on average A + (2/pi) p f + f^2).  The constants are a fit
 // to eight grids of a million clustered positions (200,000 shapes, reach 20 by
-// 60), 8.7 to 9.8 ms: within 3 %, the best grid 2 % from the one it picks.
+// 60), 8.7 to 9.8 ms: within 3 %, the best grid 2 % from the one it picks.  Wraps
+// and blocks are from 590 grids of sixteen counts in boxes of 75 to 500: without
+// wraps, blocks as tall as the box won wherever pi_max is half of it (300,001
+// positions, 100,003 weighted shapes in a box of 75 16.8 ms, now 14.7; 208,875
+// and 59,553 6.9, now 6.0), without blocks, three shapes per block in thin samples
+// (562,663 positions, 40,378 shapes in a box of 300 1.86 ms, now 1.61).  Against
+// the best of the grids tried for each count the pick is 1 % behind in the median.
 #include "mia_common.hpp"
 
 #include <algorithm>
@@ -30,7 +39,9 @@ namespace {
 constexpr double kTestCost = 1.15e-12;   // s per tested (shape, position) pair
 constexpr double kRunCost = 1.1e-12;     // s per tested (block, position) pair
 constexpr double kBodyCost = 1.0e-12;    // s per pair of the columns that touch a shape's domain
+constexpr double kWrapCost = 0.5e-12;    // s per tested pair with a wrap
 constexpr double kItemCost = 1.5e-9;     // s per work item
+constexpr double kBlockCost = 4.0e-9;    // s per shape block
 constexpr int kBlockShapes = 64;
 constexpr int kItemPositions = 8192;
 constexpr int kMaxPosColumns = 4096;     // position columns per side (12-bit indices)
@@ -73,8 +84,12 @@ double grid_cost(double L, int jk, const Choice &c, double R, double Z, bool rmu
     const double items = nblocks * std::max(rects, 1.27 * columns * sz / cpi + 0.5 * rects);
     if (items_out) *items_out = items;
     const double idle = items * 32.0 * per_block;
-    return kTestCost * (tests + idle) + kRunCost * tests / std::max(per_block, 1.0) +
-           kBodyCost * Ns * rho * area(0.0, f) * win + kItemCost * items;
+    // the part of an axis's windows that straddles half the box: the block's and a
+    // cell's extent (w) on either side, where the reach comes as far
+    auto mixed = [&](double reach, double w) { return reach + w > L / 2.0 ? std::min(1.0, 2.0 * w / L) : 0.0; };
+    const double straight = 1.0 - mixed(R, bw + f), wraps = 1.0 - (1.0 - mixed(rmu ? R : Z, bh + L / nz)) * straight * straight;
+    return (kTestCost + kWrapCost * wraps) * (tests + idle) + kRunCost * (tests + idle) / std::max(per_block, 1.0) +
+           kBodyCost * Ns * rho * area(0.0, f) * win + kItemCost * items + kBlockCost * nblocks;
 }
 
 std::mutex g_mu;
