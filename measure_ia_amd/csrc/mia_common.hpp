@@ -117,6 +117,16 @@ constexpr int64_t kItemOverhead = 1024;  // per-item cost, in pair evaluations (
 void schedule_batches(const int64_t *cost_prefix, const int64_t *n_dev, const int32_t *np, int np_stride, int waves,
                       int64_t *bounds, hipStream_t st, bool all_static, int waves_per_unit);
 
+// Workgroups of `bytes` of LDS each that a CU (gfx950: 160 KiB) holds at once.  LDS
+// is allocated in granules of 1,280 bytes, which hipOccupancyMaxActiveBlocks-
+// PerMultiprocessor does not round up to: of workgroups of 54,096 bytes it says
+// three, and the third ran behind the other two.
+constexpr size_t kLdsBytes = 160 * 1024, kLdsGranule = 1280;
+inline int workgroups_by_lds(size_t bytes) {
+    const size_t a = (bytes + kLdsGranule - 1) / kLdsGranule * kLdsGranule;
+    return a > kLdsBytes ? 0 : (int)(kLdsBytes / (a > 0 ? a : kLdsGranule));
+}
+
 constexpr int kMaxBins2 = 256;      // max n_2 (pi or mu bins)
 constexpr int kMaxBinsR = 256;      // max n_r
 constexpr int kMaxBlockShapes = 64;

@@ -48,7 +48,6 @@ namespace {
 
 constexpr int kMaxWavesPerBlock = 4;
 constexpr int kThreads = kWave * kMaxWavesPerBlock;
-constexpr size_t kLdsBytes = 160 * 1024;         // LDS per CU (gfx950)
 constexpr size_t kPairStaticLds = 64;            // the pair kernel's own LDS words, at most
 constexpr int kStatCopies = 32, kStatStride = 16;  // copies of the pair kernel's statistics, words apart
 constexpr int kSharedBelow = 16;                 // private waves per CU below which histograms are shared
@@ -1696,7 +1695,7 @@ const void *pair_kernel(int mode, bool weighted, bool var) {
 int resident_workgroups(int mode, bool weighted, bool var, int wpb, size_t lds) {
     int n = 0;
     MIA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pair_kernel(mode, weighted, var), kWave * wpb, lds));
-    return std::max(1, n);
+    return std::max(1, std::min(n, workgroups_by_lds(lds + kPairStaticLds)));
 }
 
 // Waves per CU whose histograms (hs bytes) and thresholds LDS holds, with a
@@ -1704,12 +1703,10 @@ int resident_workgroups(int mode, bool weighted, bool var, int wpb, size_t lds) 
 int private_waves(size_t thr_bytes, size_t hs) {
     int w = kMaxWavesPerBlock;
     while (w > 1 && thr_bytes + hs * w + kPairStaticLds > kLdsBytes) w /= 2;
-    const size_t l = thr_bytes + hs * w + kPairStaticLds;
-    return l > kLdsBytes ? 0 : (int)std::min<size_t>(32 / w, kLdsBytes / l) * w;
+    return std::min(32 / w, workgroups_by_lds(thr_bytes + hs * w + kPairStaticLds)) * w;
 }
 int shared_waves(size_t thr_bytes, size_t hs) {
-    const size_t l = thr_bytes + hs + kPairStaticLds;
-    return l > kLdsBytes ? 0 : (int)std::min<size_t>(32 / kMaxWavesPerBlock, kLdsBytes / l) * kMaxWavesPerBlock;
+    return std::min(32 / kMaxWavesPerBlock, workgroups_by_lds(thr_bytes + hs + kPairStaticLds)) * kMaxWavesPerBlock;
 }
 
 // candidates: expected (shape, position) pairs of the count.
@@ -1853,7 +1850,7 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     const bool large = candidates > 16 * kTailMinCost * pw * cu_count;
     A.shared = !det && most > 0 && (small || (pw < most && (pw < kSharedBelow || large)));
     if (A.shared) {
-        const size_t share = kLdsBytes / kPairWavesPerSimd - kPairStaticLds;
+        const size_t share = kLdsBytes / kPairWavesPerSimd / kLdsGranule * kLdsGranule - kPairStaticLds;
         A.copies = share > thr_bytes + hs ? (int)std::min<size_t>(4, (share - thr_bytes) / hs) : 1;
         C.lds = thr_bytes + hs * A.copies;
     } else {

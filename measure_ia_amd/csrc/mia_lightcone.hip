@@ -57,7 +57,8 @@ namespace {
 
 constexpr int kLcWavesPerBlock = 4;
 constexpr int kLcThreads = kWave * kLcWavesPerBlock;
-constexpr size_t kLcLds = 160 * 1024 - 64;  // LDS per CU (gfx950) less the pair kernel's own words
+constexpr size_t kLcStaticLds = 64;         // the pair kernel's own LDS words, at most
+constexpr size_t kLcLds = kLdsBytes - kLcStaticLds;
 constexpr double kPiC = 3.141592653589793;  // numpy's np.pi
 constexpr double kDeg = kPiC / 180.0;
 constexpr int64_t kLcCountedPairs = 4096;     // patch pairs up to which items are counting-sorted (16 KiB of LDS)
@@ -1642,8 +1643,7 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     auto waves_per_cu = [&](int nr_) {
         const int w = wpb_for(nr_);
         const size_t l = thr_bytes + lc_hist_bytes(nr_ * n_2, shapes, weighted) * w;
-        if (l > kLcLds) return 0;
-        return (int)std::min<size_t>(32 / w, kLcLds / l) * w;
+        return std::min(32 / w, workgroups_by_lds(l + kLcStaticLds)) * w;
     };
     int nrp = n_r;
     if (tuning && tuning->r_bins_per_pass > 0) {
@@ -1683,7 +1683,7 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     const void *kernel = lc_kernel(bins.mode, shapes, weighted);
     MIA_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     MIA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks_per_cu, kernel, kWave * wpb, lds));
-    blocks_per_cu = std::max(1, blocks_per_cu);
+    blocks_per_cu = std::max(1, std::min(blocks_per_cu, workgroups_by_lds(lds + kLcStaticLds)));
     int waves = tuning && tuning->waves > 0 ? std::min(tuning->waves, kMaxWaves) : ctx.cu_count * blocks_per_cu * wpb;
     if (nitems < waves) waves = std::max(1, nitems);
     A.n_waves = waves;
