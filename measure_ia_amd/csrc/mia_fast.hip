@@ -1773,12 +1773,16 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     // Passes over r-bin ranges.  Pass [r0, r0 + nrp) takes the pairs with
     // T[r0] <= r^2 < T[r0 + nrp] (exact FP64 comparisons, so every pair lands
     // in one pass), bins them locally and flushes to output bins
-    // r0 * n_2 + local.  A pass's time goes as 1 / min(1, w / 16), w the
-    // waves per CU its histogram leaves room for (latency-bound below 16
-    // waves, VALU-bound above; measured on 60 x 60 and 100 x 100 bins), so nrp
-    // minimises passes / min(1, w / 16) (ties: fewer passes), with at least
-    // 4 waves per CU where any split allows it (at 2 a pass runs slower than
-    // that model says).  Ordinary binnings run in one pass.
+    // r0 * n_2 + local.  A pass's time goes about as 1 / min(1, w / W), w the
+    // waves per CU its histogram leaves room for, so nrp minimises
+    // passes / min(1, w / W) (ties: fewer passes), with at least 4 waves per
+    // CU where any split allows it (at 2 a pass runs slower than that model
+    // says).  W is 7 with histograms per wave (deterministic) and 10 with
+    // histograms per workgroup, whose waves wait for each other.  Pair kernels
+    // with W = 16 and now, 1,000,000 positions and 200,000 shapes: deterministic
+    // 100 x 100 bins 25 passes of 16 waves 181 ms, 7 of 4 121; 60 x 60 8 of 12 70 ms,
+    // 5 of 8 54; shared, 200,000 and 50,000: 100 x 100 5 of 12 6.1 ms, 2 of 4
+    // 4.1.  Ordinary binnings run in one pass.
     const size_t thr_bytes = threshold_bytes(bins);
     int nrp = n_r;
     {
@@ -1802,7 +1806,7 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
                     const int w = waves_per_cu(c);
                     if (w < pass_min_waves) continue;
                     const int passes = (n_r + c - 1) / c;
-                    const double cost = (double)passes / std::min(1.0, w / 16.0);
+                    const double cost = (double)passes / std::min(1.0, w / (det ? 7.0 : 10.0));
                     if (cost < best * (1 - 1e-9) || (cost <= best * (1 + 1e-9) && passes < best_p)) {
                         best = cost;
                         best_p = passes;
