@@ -51,6 +51,10 @@ constexpr int kThreads = kWave * kMaxWavesPerBlock;
 constexpr size_t kPairStaticLds = 64;            // the pair kernel's own LDS words, at most
 constexpr int kStatCopies = 32, kStatStride = 16;  // copies of the pair kernel's statistics, words apart
 constexpr int kSharedBelow = 16;                 // private waves per CU below which histograms are shared
+// A wave spills the 32-bit counts every 2^kSpillBits wave-iterations of 64 pairs at
+// most, and looks after kRunBatches batches against 64 shapes: the four waves of a
+// group add at most 4 * 64 * (2^23 + 2^22) < 2^32 pairs to a count in between.
+constexpr int kSpillBits = 23, kRunBatches = 1 << 16;
 constexpr int kSplitItems = 32;                  // items per group of four waves below which a claim is a quarter of an item
 constexpr int kPairWavesPerSimd = 6;             // waves per SIMD the pair kernel's registers allow
 constexpr int64_t kMaxKeysPerSample = 1 << 24;   // K^2 planner keys per sample (K regions)
@@ -908,6 +912,7 @@ __global__ __launch_bounds__(256) void k_finalize_det(const FinSample *fs, const
     sx.reduce();
     vr.reduce();
     if (lane) return;
+    c += F.np[j];  // spilled counts
     F.out.npairs[j] = c;
     if (F.out.dd) F.out.dd[j] = F.weighted ? dd.s + dd.c : (double)c;
     F.out.splus[j] = sp.s + sp.c;
@@ -992,6 +997,14 @@ __device__ __forceinline__ int front_bytes(int nbins) {
 // the inner loop is uniform over shapes, so every field lands in SGPRs.
 typedef const __attribute__((address_space(4))) double *ShapePtr;
 
+// The place of bin b's count in a histogram.
+template <bool WEIGHTED, bool VAR>
+__device__ __forceinline__ uint32_t *bin_count(char *sums, int b) {
+    typedef Slot<WEIGHTED, VAR> BinSlot;
+    return BinSlot::kApart ? (uint32_t *)sums - 1 - b
+                           : (uint32_t *)(sums + (uint32_t)b * BinSlot::kBytes + 8 * BinSlot::kSums);
+}
+
 // One bin of a histogram, summed over its copies and cleared.
 template <bool WEIGHTED, bool VAR>
 __device__ __forceinline__ Slot<WEIGHTED, VAR> take_bin(const PairArgs &P, char *hist, int copies, int b) {
@@ -1000,7 +1013,7 @@ __device__ __forceinline__ Slot<WEIGHTED, VAR> take_bin(const PairArgs &P, char 
     hist += front_bytes<WEIGHTED, VAR>(P.nbins);
     for (int k = 0; k < copies; ++k, hist += P.hist_stride) {
         double *v = (double *)(hist + (uint32_t)b * BinSlot::kBytes);
-        uint32_t *c = BinSlot::kApart ? (uint32_t *)hist - 1 - b : (uint32_t *)(v + BinSlot::kSums);
+        uint32_t *c = bin_count<WEIGHTED, VAR>(hist, b);
         if (*c == 0) continue;
         t.c += *c;
         *c = 0;
@@ -1011,6 +1024,35 @@ __device__ __forceinline__ Slot<WEIGHTED, VAR> take_bin(const PairArgs &P, char 
         }
     }
     return t;
+}
+
+// c pairs of the pass's bin b for the total and the tallies of both regions.
+__device__ __forceinline__ void add_pairs(const PairArgs &P, const SampleDev &S, int rs, int rp, int b,
+                                          unsigned long long c) {
+    const int gb = b + P.bin_off;  // the pass's local bin in the output grid
+    atomicAdd(&S.npairs[gb], c);
+    if (S.K > 0) {
+        atomicAdd(&S.npairs[(int64_t)(1 + rs) * P.nbins_out + gb], c);
+        if (rp != rs) atomicAdd(&S.npairs[(int64_t)(1 + rp) * P.nbins_out + gb], c);
+    }
+}
+
+// A wave takes all but one pair of every count to the 64-bit sums, with adds of
+// other waves in flight: the histogram's 32-bit counts then stay below 2^32 whatever
+// its waves test before the next flush (a bin without a pair would not be flushed).
+template <bool WEIGHTED, bool VAR>
+__device__ void spill_counts(const PairArgs &P, char *hist, int copies, const SampleDev &S, int rs, int rp, int lane) {
+    for (int b = lane; b < P.nbins; b += kWave) {
+        char *sums = hist + front_bytes<WEIGHTED, VAR>(P.nbins);
+        unsigned long long c = 0;
+        for (int k = 0; k < copies; ++k, sums += P.hist_stride) {
+            uint32_t *at = bin_count<WEIGHTED, VAR>(sums, b);
+            // (a count of one or more never falls below one before the flush)
+            if (__hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > 1)
+                c += __hip_atomic_exchange(at, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) - 1;
+        }
+        if (c) add_pairs(P, S, rs, rp, b, c);
+    }
 }
 
 template <bool WEIGHTED, bool VAR>
@@ -1027,20 +1069,18 @@ __device__ void flush_hist(const PairArgs &P, char *hist, int copies, const Samp
         if constexpr (WEIGHTED) vdd = t.v[2];
         if constexpr (VAR) vvr = t.v[WEIGHTED ? 3 : 2];
         if (c == 0) continue;
-        const int gb = b + P.bin_off;  // the pass's local bin in the output grid
-        atomicAdd(&S.npairs[gb], (unsigned long long)c);
+        const int gb = b + P.bin_off;
+        add_pairs(P, S, rs, rp, b, c);
         atomicAdd(&S.sp[gb], vsp);
         atomicAdd(&S.sx[gb], vsx);
         if (dd && S.dd) atomicAdd(&S.dd[gb], vdd);
         if (vr && S.var) atomicAdd(&S.var[gb], vvr);
         if (S.K > 0) {
             int64_t o = (int64_t)(1 + rs) * BO + gb;
-            atomicAdd(&S.npairs[o], (unsigned long long)c);
             atomicAdd(&S.sp[o], vsp);
             if (dd && S.dd) atomicAdd(&S.dd[o], vdd);
             if (rp != rs) {
                 o = (int64_t)(1 + rp) * BO + gb;
-                atomicAdd(&S.npairs[o], (unsigned long long)c);
                 atomicAdd(&S.sp[o], vsp);
                 if (dd && S.dd) atomicAdd(&S.dd[o], vdd);
             }
@@ -1501,6 +1541,7 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     int cur_key = -1, flushes = 0, par = 0;
     uint32_t nre = 0;
     uint64_t iterations = 0;  // wave-uniform
+    uint32_t spills = 0;
 
     auto sync = [&]() {
         if (shared)
@@ -1594,14 +1635,23 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
                                 (jj >> 16) & 0xffff, wn & 0xffff, (wn >> 16) & 0xffff, c0, kk & 0xffff,
                                 (kk >> 16) & 0xffff, w, lane, cpb, cn);
                 }
-                // (r, mu) sums r^2 in an order fixed by the line of sight: one
-                // loop per order, so the pair loop holds no branch on it
-                if (MODE == MIA_RMU && S.los != 2)
-                    run_shifted<MODE, WEIGHTED, VAR, false>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist_at, T, X,
-                                                            lane, nre, iterations);
-                else
-                    run_shifted<MODE, WEIGHTED, VAR, true>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist_at, T, X,
-                                                           lane, nre, iterations);
+                for (int b = bt0; b < bt1; b += kRunBatches) {
+                    const int e = bt1 - b < kRunBatches ? bt1 : b + kRunBatches;
+                    // (r, mu) sums r^2 in an order fixed by the line of sight: one
+                    // loop per order, so the pair loop holds no branch on it
+                    if (MODE == MIA_RMU && S.los != 2)
+                        run_shifted<MODE, WEIGHTED, VAR, false>(P, S, cpb, cn, b, e, shifts, shp, ns, hist_at, T, X,
+                                                                lane, nre, iterations);
+                    else
+                        run_shifted<MODE, WEIGHTED, VAR, true>(P, S, cpb, cn, b, e, shifts, shp, ns, hist_at, T, X,
+                                                               lane, nre, iterations);
+                    if ((uint32_t)(iterations >> kSpillBits) == spills) continue;
+                    spills = (uint32_t)(iterations >> kSpillBits);
+                    const PairArgs &A = *(const PairArgs *)args();
+                    const int kk = A.K1 * A.K1, in = cur_key % kk;
+                    spill_counts<WEIGHTED, VAR>(A, hist, shared ? A.copies : 1, A.samples[cur_key / kk], in / A.K1,
+                                                in % A.K1, lane);
+                }
             }
             if (shared) {
                 __syncthreads();
