@@ -590,19 +590,63 @@ __global__ void k_lc_ranges(LcPlan P) {
 // One wave per block: its ranges grouped by patch, in their order within a
 // patch.  A block's ranges come in stencil-cell order, so a stencil over a patch
 // border alternates patches row by row, and the items (one patch pair each)
-// would break at every change.  A block has a few dozen ranges: a range's place
-// is the number of ranges before it in (patch, index) order, counted directly
-// (a radix sort of all ranges by (block, patch) took 0.13 ms in 16 launches for
-// 1,000,000 positions, this one 0.02 ms).
+// would break at every change.  A block at hundreds of Mpc has a few dozen
+// ranges: a range's place is the number of ranges before it in (patch, index)
+// order, counted directly (a radix sort of all ranges by (block, patch) took 0.13
+// ms in 16 launches for 1,000,000 positions, this one 0.02 ms).  A block near the
+// observer reaches the whole sky and may have a hundred thousand: beyond
+// kGroupDirect ranges they are counted per patch in LDS and placed 64 at a time
+// (64 positions at 4 to 8 Mpc, 60,000 shapes at 5 to 25 over the sky: planning 32
+// ms by comparing all, now 2.1).
+constexpr int kGroupDirect = 256;
 __global__ __launch_bounds__(kGroupWaves * kWave) void k_lc_group(const LcRange *__restrict__ in,
                                                                   const int64_t *__restrict__ roff,
                                                                   const int64_t *__restrict__ soff, int nblocks,
-                                                                  LcRange *__restrict__ out) {
+                                                                  int P1, LcRange *__restrict__ out) {
     const int lane = threadIdx.x & (kWave - 1);
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x * kGroupWaves + threadIdx.x / kWave);
     if (b >= nblocks) return;
     const int64_t r0 = roff[soff[b]];
     const int n = (int)(roff[soff[b + 1]] - r0);
+    if (n > kGroupDirect) {
+        extern __shared__ int32_t group_tab[];  // P1 words per wave: the next place of every patch
+        int32_t *tab = group_tab + (threadIdx.x / kWave) * P1;
+        for (int k = lane; k < P1; k += kWave) tab[k] = 0;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        for (int i = lane; i < n; i += kWave) atomicAdd(&tab[in[r0 + i].patch], 1);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        int base = 0;
+        for (int k0 = 0; k0 < P1; k0 += kWave) {
+            const int c = k0 + lane < P1 ? tab[k0 + lane] : 0;
+            int sum = c;
+            for (int d = 1; d < kWave; d <<= 1) {
+                const int o = __shfl_up(sum, d);
+                sum += lane >= d ? o : 0;
+            }
+            if (k0 + lane < P1) tab[k0 + lane] = base + sum - c;
+            base += __shfl(sum, kWave - 1);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        for (int i0 = 0; i0 < n; i0 += kWave) {
+            const int i = i0 + lane;
+            LcRange mine{};
+            mine.patch = -1;
+            if (i < n) mine = in[r0 + i];
+            uint64_t left = __ballot(i < n);
+            while (left) {  // the lanes of one patch at a time, in lane order
+                const int p = __builtin_amdgcn_readlane(mine.patch, __builtin_ctzll(left));
+                const bool same = mine.patch == p;
+                const uint64_t m = __ballot(same);
+                const int at = tab[p];
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                if (same) out[r0 + at + __popcll(m & ((1ull << lane) - 1))] = mine;
+                if (lane == 0) tab[p] = at + __popcll(m);
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                left &= ~m;
+            }
+        }
+        return;
+    }
     for (int i0 = 0; i0 < n; i0 += kWave) {
         const int i = i0 + lane;
         LcRange mine{};
@@ -659,15 +703,22 @@ __global__ __launch_bounds__(256) void k_lc_items(LcItemArgs A) {
     auto walk = [&](auto &&f) {
         int64_t r0 = r_begin;
         int acc = 0, patch = -1;
-        for (int64_t r = r_begin; r < r_end; ++r) {
-            const LcRange R = A.ranges[r];
-            if (R.patch != patch || acc + R.n > A.item_shapes) {
-                if (acc > 0) f(r0, (int)(r - r0), acc, patch);
-                r0 = r;
-                acc = 0;
-                patch = R.patch;
+        // (four loads in flight: a block near the observer has tens of thousands of ranges)
+        for (int64_t rb = r_begin; rb < r_end; rb += 4) {
+            LcRange R[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) R[k] = A.ranges[rb + k < r_end ? rb + k : r_end - 1];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (rb + k >= r_end) break;
+                if (R[k].patch != patch || acc + R[k].n > A.item_shapes) {
+                    if (acc > 0) f(r0, (int)(rb + k - r0), acc, patch);
+                    r0 = rb + k;
+                    acc = 0;
+                    patch = R[k].patch;
+                }
+                acc += R[k].n;
             }
-            acc += R.n;
         }
         if (acc > 0) f(r0, (int)(r_end - r0), acc, patch);
     };
@@ -1484,8 +1535,9 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     }
     if (P > 0 && nranges > 1) {
         LcRange *ranges2 = ctx.arena.get<LcRange>("lc/ranges2", nranges);
-        hipLaunchKernelGGL(k_lc_group, dim3(nblk_(nblocks, kGroupWaves)), dim3(kGroupWaves * kWave), 0, st,
-                           (const LcRange *)ranges, roff, soff, nblocks, ranges2);
+        hipLaunchKernelGGL(k_lc_group, dim3(nblk_(nblocks, kGroupWaves)), dim3(kGroupWaves * kWave),
+                           sizeof(int32_t) * kGroupWaves * (size_t)P1, st, (const LcRange *)ranges, roff, soff,
+                           nblocks, P1, ranges2);
         MIA_HIP(hipGetLastError());
         ranges = ranges2;
     }
