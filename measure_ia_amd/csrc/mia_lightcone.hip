@@ -59,6 +59,10 @@ constexpr int kLcWavesPerBlock = 4;
 constexpr int kLcThreads = kWave * kLcWavesPerBlock;
 constexpr size_t kLcStaticLds = 64;         // the pair kernel's own LDS words, at most
 constexpr size_t kLcLds = kLdsBytes - kLcStaticLds;
+// stencil cells up to which the count pass keeps the windows that it found for the
+// emit pass (128 MiB; beyond, the emit pass looks for them again, as cheap as its
+// share of the memory is dear: 8 bytes a cell were 17 GB at the limit of 2^31)
+constexpr int64_t kLcWindows = 1 << 24;
 constexpr double kPiC = 3.141592653589793;  // numpy's np.pi
 constexpr double kDeg = kPiC / 180.0;
 constexpr int64_t kLcCountedPairs = 4096;     // patch pairs up to which items are counting-sorted (16 KiB of LDS)
@@ -494,7 +498,7 @@ struct LcPlan {
     ChiQ scq;
     int item_shapes;          // ranges are split at this many shapes
     int32_t *rcount;          // count pass: ranges per stencil cell
-    int2 *window;             // the shapes [x, y) found in a cell of one segment (kept for the emit pass)
+    int2 *window;             // the shapes [x, y) found in a cell of one segment, for the emit pass (or null)
     const int64_t *roff;      // emit pass: range offsets, total + 1
     LcRange *ranges;
     int emit;
@@ -561,14 +565,14 @@ __global__ void k_lc_ranges(LcPlan P) {
         const int s0 = P.cfs[cell], s1 = P.cfs[cell + 1];
         for (int s = s0; s < s1; ++s) {
             int a, e;
-            if (P.emit && s1 == s0 + 1) {
+            if (P.emit && P.window && s1 == s0 + 1) {
                 const int2 w = P.window[t];
                 a = w.x;
                 e = w.y;
             } else {
                 a = lower_chi(P.sq, P.sseg[s], P.sseg[s + 1], chi_q(P.scq, clo));
                 e = upper_chi(P.sq, a, P.sseg[s + 1], chi_q(P.scq, chi_hi));
-                if (!P.emit && s1 == s0 + 1) P.window[t] = make_int2(a, e);
+                if (!P.emit && P.window && s1 == s0 + 1) P.window[t] = make_int2(a, e);
             }
             int patch = (int)(P.sseg_key[s] % (uint64_t)g.P1);
             for (int k = a; k < e; k += P.item_shapes) {
@@ -1511,7 +1515,7 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     int64_t *rc64 = ctx.arena.get<int64_t>("lc/rc64", total + 1);
     int64_t *roff = ctx.arena.get<int64_t>("lc/roff", total + 1);
     L.rcount = rc;
-    L.window = ctx.arena.get<int2>("lc/window", total + 1);
+    L.window = total <= kLcWindows ? ctx.arena.get<int2>("lc/window", total + 1) : nullptr;
     L.emit = 0;
     if (total > 0) {
         hipLaunchKernelGGL(k_lc_ranges, dim3(nblk_(total, 256)), dim3(256), 0, st, L);
