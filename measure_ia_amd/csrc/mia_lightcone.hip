@@ -1033,7 +1033,8 @@ __device__ __forceinline__ void lc_pair(const LcPairArgs &P, bool valid, double 
 template <int MODE, bool SHAPES, bool WEIGHTED>
 __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
     extern __shared__ __align__(16) char lds[];
-    __shared__ unsigned int s_nre, s_left;
+    __shared__ unsigned long long s_nre;
+    __shared__ unsigned int s_left;
     const int lane = threadIdx.x & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     double *T = (double *)lds;
@@ -1192,9 +1193,9 @@ __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
     if (cur_pn >= 0) lc_flush<SHAPES, WEIGHTED>(P, hist, cur_pn, cur_ps, lane);
     // the last wave of the workgroup adds its statistics: one atomic each on a
     // word that all workgroups share
-    if (nre) atomicAdd(&s_nre, nre);
+    if (nre) atomicAdd(&s_nre, (unsigned long long)nre);
     if (lane == 0 && __hip_atomic_fetch_add(&s_left, -1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 1u && s_nre)
-        atomicAdd(P.rechecks, (unsigned long long)s_nre);
+        atomicAdd(P.rechecks, s_nre);
 }
 
 // The pair kernel of a count.
