@@ -1071,7 +1071,7 @@ __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
     CPtrI blocks = (CPtrI)P.blocks;
     CPtrI ranges = (CPtrI)P.ranges;
     int cur_pn = -1, cur_ps = -1;
-    uint32_t nre = 0;
+    uint32_t nre = 0, held = 0;  // held: pairs tested since the last flush
     // the additive constants of the FP32 bin guesses, held in VGPRs (a VOP3
     // FMA reads one scalar operand; the other would be copied on every pair)
     float vlgc, vxc;
@@ -1087,13 +1087,16 @@ __global__ __launch_bounds__(kLcThreads, 6) void k_lc_pairs(LcPairArgs P) {
             CPtrI bp = blocks + 8 * (int64_t)blk;
             const int p0 = bp[0], np = bp[1], pn = bp[3];
             const int ps = ranges[4 * (int64_t)r0 + 2];
-            if (pn != cur_pn || ps != cur_ps) {
+            // (a flush at 2^31 pairs keeps the 32-bit counts from wrapping)
+            if (pn != cur_pn || ps != cur_ps || held > 1u << 31) {
+                held = 0;
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 if (cur_pn >= 0) lc_flush<SHAPES, WEIGHTED>(P, hist, cur_pn, cur_ps, lane);
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 cur_pn = pn;
                 cur_ps = ps;
             }
+            held += (uint32_t)(ns * np);
             LcPend pd{none, none_c, 0, 0.0, 0.0, 0.0};
             int j = r0, o = 0;
             const int jend = r0 + nr;
@@ -1410,7 +1413,8 @@ void count_lightcone(Ctx &ctx, const mia_lc_sample &s, const mia_bins &bins, con
     g.nslab = (int)std::max(1.0, std::min(nsl, 1.0e6));
     const int ncells = nrows * ncols;
     const int bsz = tuning && tuning->block_shapes > 0 ? std::min(tuning->block_shapes, kWave) : kWave;
-    const int item_shapes = tuning && tuning->item_positions > 0 ? tuning->item_positions : 1024;
+    // (2^24 shapes against a block of 64: below the 2^31 pairs at which the pair kernel flushes)
+    const int item_shapes = tuning && tuning->item_positions > 0 ? std::min(tuning->item_positions, 1 << 24) : 1024;
 
     // ---- 2. sort both samples
     uint64_t *pkey = nullptr, *skey = nullptr;

@@ -34,3 +34,11 @@ def test_rechecks_beyond_32_bits():
     res = _count(ra, ra_s, np.logspace(np.log10(10.0), np.log10(10.01), 11), 8, 4, flat=True)
     assert int(res.npairs[0].sum()) == N * N
     assert res.stats["rechecks"] == N * N, res.stats
+
+
+def test_counts_beyond_32_bits():
+    """One wave counts 4.3e9 pairs in one bin."""
+    rng = np.random.default_rng(6)
+    res = _count(10.0 + rng.uniform(0.0, 1.0, N), 10.0 + rng.uniform(0.0, 1.0, N), np.array([1e-12, 100.0]), 1, 1)
+    assert int(res.npairs[0].sum()) == N * N
+    np.testing.assert_array_equal(res.dd, res.npairs.astype(float))
