@@ -880,6 +880,23 @@ void stage_count(Ctx &ctx, int n, const mia_sample *samples, const mia_bins &bin
                  const mia_tuning *tuning, mia_stats *stats, hipStream_t st, StageMode mode) {
     // the deterministic sort's radix-sort launches stay out of graphs
     if (mode == STAGE_GRAPH && tuning && tuning->deterministic) mode = STAGE_EAGER;
+    // The static workspace: a count that does not fit on the tuner's grid is planned on
+    // up to kCoarser coarser ones, which need fewer cells and items (1,110,150
+    // positions and shapes in a box of 75: the first coarser grid)
+    constexpr int kCoarser = 4;
+    int coarser = 0;
+    mia_tuning coarse{};
+    if (tuning) coarse = *tuning;
+    const bool own_grid = tuning && (tuning->columns_per_side > 0 || tuning->slabs_per_side > 0);
+    auto try_coarser = [&](const Grid &g) {
+        if (mode != STAGE_STATIC || own_grid || coarser == kCoarser) return false;
+        ++coarser;
+        const int jk = g.jk > 0 ? g.jk : 1;
+        coarse.columns_per_side = std::max(jk, g.nc * 3 / 4);
+        coarse.slabs_per_side = std::max(jk, g.nz / 2);
+        tuning = &coarse;
+        return true;
+    };
     for (int attempt = 0;; ++attempt) {
         PrepPlan prep;
         prep_plan(prep, n, samples, bins, tuning);
@@ -901,6 +918,7 @@ void stage_count(Ctx &ctx, int n, const mia_sample *samples, const mia_bins &bin
                     total = pbytes + count_bytes(*cp);
                 }
             }
+            if (total > room && try_coarser(prep.grids[0])) continue;
             if (total > room)
                 throw Error{MIA_E_UNSUPPORTED, "the count needs " + std::to_string(total) +
                                                    " bytes of workspace; the static workspace holds " +
@@ -921,6 +939,7 @@ void stage_count(Ctx &ctx, int n, const mia_sample *samples, const mia_bins &bin
                 throw Error{MIA_E_RANGE, "coordinates outside [0, boxsize] (or NaN) in sample " + std::to_string(s)};
         if (r.words[2]) {
             // more work items than the capacity: grow it and count again
+            if (try_coarser(prep.grids[0])) continue;
             if (mode == STAGE_STATIC)
                 throw Error{MIA_E_UNSUPPORTED, "the count needs " + std::to_string(r.words[3]) +
                                                    " work items; the static workspace holds " +
