@@ -520,7 +520,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_emit_items(PlanLaunch A) {
                           it.nc = (uint16_t)(cols - it.c0 < P.cpi ? cols - it.c0 : P.cpi);
                           A.items[slot + i] = it;
                           if (A.sort_key)
-                              A.sort_key[slot + i] = ((unsigned long long)(kb + key) << A.sort_shift) |
+                              A.sort_key[slot + i] = (A.sort_shift < 64 ? (unsigned long long)(kb + key) << A.sort_shift : 0ull) |
                                                      ((unsigned long long)blk * (kMaxSegs * kMaxSegs * (kMaxSegs + 1)) + t);
                       }
                   });
@@ -630,10 +630,17 @@ __global__ void k_items_total(const int64_t *key_off, int64_t nkeys, int64_t cap
 }
 
 // Deterministic order of the items: the permutation of a stable sort by
-// (key, plan thread) applied to the items and their costs.
+// (key, block, rectangle) applied to the items and their costs.
 __global__ void k_iota(int32_t *a, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = (int32_t)i;
+}
+
+// The planner keys of the items in a given order.
+__global__ void k_item_keys(const int32_t *order, const int64_t *n_dev, int64_t cap, const Item *items,
+                            unsigned long long *key) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < cap) key[i] = i < *n_dev ? (unsigned long long)items[order[i]].key : ~0ull;
 }
 
 __global__ void k_gather_items(const int32_t *order, const int64_t *n_dev, const Item *items, const int64_t *cost,
@@ -2029,10 +2036,16 @@ int det_low_bits(const CountPlan &p) {
     while (b < 62 && ((int64_t)1 << b) < n) ++b;
     return b;
 }
-int det_key_bits(const CountPlan &p) {
+int det_index_bits(const CountPlan &p) {
     int b = 1;
     while (b < 31 && ((int64_t)1 << b) < p.nkeys + 1) ++b;
-    return det_low_bits(p) + b;
+    return b;
+}
+// A key and a block's rectangle that do not fit one word take two stable sorts,
+// by rectangle and then by key (50,000,000 shape blocks with 4,096 regions).
+bool det_two_sorts(const CountPlan &p) { return det_low_bits(p) + det_index_bits(p) > 64; }
+int det_key_bits(const CountPlan &p) {
+    return det_two_sorts(p) ? std::max(det_low_bits(p), det_index_bits(p)) : det_low_bits(p) + det_index_bits(p);
 }
 
 CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_bins &bins,
@@ -2139,7 +2152,6 @@ CountPlan *plan_count(Ctx &ctx, const std::vector<SortedSample> &ss, const mia_b
     p.nkeys = (int64_t)S * p.K1 * p.K1;
     p.slot_cap = p.det ? (int64_t)p.pc.waves + p.nkeys : 0;
     MIA_REQUIRE(p.nblk_cap < ((int64_t)1 << 31), "too many shape blocks");
-    MIA_REQUIRE(!p.det || det_key_bits(p) <= 64, "plan too large for the deterministic item order");
     // item capacity: the caller's (grown after an overflow), at least twice
     // the uniform-density estimate plus a margin
     p.item_cap = cap_exact ? item_cap : std::max<int64_t>(item_cap, (int64_t)(2.0 * est_items) + 65536);
@@ -2351,7 +2363,7 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
         hipLaunchKernelGGL(k_iota, dim3(nblk(p.item_cap, 256)), dim3(256), 0, st, p.sidx, p.item_cap);
         MIA_HIP(hipGetLastError());
         L.sort_key = p.skey;
-        L.sort_shift = det_low_bits(p);
+        L.sort_shift = det_two_sorts(p) ? 64 : det_low_bits(p);
     }
     hipLaunchKernelGGL(k_emit_items, dim3(bgrid), dim3(kPlanThreads), 0, st, L);
     MIA_HIP(hipGetLastError());
@@ -2361,13 +2373,24 @@ void count_enqueue(const CountPlan &p, hipStream_t st, const hipEvent_t *ev) {
                        (const double *)p.bbox, (const int64_t *)p.n_items, p.items, p.cost, p.words + 1);
     MIA_HIP(hipGetLastError());
     if (p.det) {
-        // items of one key in (plan thread, emission) order: a stable sort of
-        // the whole capacity (unused slots keep the largest key and sort last)
+        // items of one key in (block, rectangle) order: a stable sort of the whole
+        // capacity (unused slots keep the largest key and sort last)
+        const bool two = det_two_sorts(p);
+        const int32_t *order = p.sidx2;
         size_t bytes = p.stmp_bytes;
         MIA_HIP(hipcub::DeviceRadixSort::SortPairs(p.stmp, bytes, (const unsigned long long *)p.skey, p.skey2,
                                                    (const int32_t *)p.sidx, p.sidx2, (int)p.item_cap, 0,
-                                                   det_key_bits(p), st));
-        hipLaunchKernelGGL(k_gather_items, dim3(nblk(p.item_cap, 256)), dim3(256), 0, st, (const int32_t *)p.sidx2,
+                                                   two ? det_low_bits(p) : det_key_bits(p), st));
+        if (two) {
+            hipLaunchKernelGGL(k_item_keys, dim3(nblk(p.item_cap, 256)), dim3(256), 0, st, (const int32_t *)p.sidx2,
+                               (const int64_t *)p.n_items, p.item_cap, (const Item *)p.items, p.skey);
+            MIA_HIP(hipGetLastError());
+            MIA_HIP(hipcub::DeviceRadixSort::SortPairs(p.stmp, bytes, (const unsigned long long *)p.skey, p.skey2,
+                                                       (const int32_t *)p.sidx2, p.sidx, (int)p.item_cap, 0,
+                                                       det_index_bits(p), st));
+            order = p.sidx;
+        }
+        hipLaunchKernelGGL(k_gather_items, dim3(nblk(p.item_cap, 256)), dim3(256), 0, st, order,
                            (const int64_t *)p.n_items, (const Item *)p.items, (const int64_t *)p.cost, p.items2,
                            p.cost2);
         MIA_HIP(hipGetLastError());
