@@ -56,7 +56,7 @@ enum mia_mode { MIA_RPPI = 0, MIA_RMU = 1 };
  *   MIA_PLAIN: one thread per shape, FP64 geometry in the reference's op
  *              order, global-atomic histograms (the straightforward GPU form).
  *   MIA_FAST : cell-pair work items sorted by jackknife region pair, a
- *              persistent cost-balanced grid, per-wavefront LDS histograms
+ *              persistent cost-balanced grid, LDS histograms
  *              (u32 counts, FP64 sums); FP64 separations and e+ in the
  *              reference's rounding, FP32 bin guesses resolved exactly in
  *              FP64 near an edge. */
@@ -136,7 +136,7 @@ typedef struct mia_tuning {
     int32_t item_positions;     /* positions per work item, about (whole position
                                    columns, 1 to 64 of them)                            */
     int32_t waves;              /* persistent waves of the pair kernel (at most 2^20)  */
-    int32_t hist_copies;        /* ignored (one LDS histogram copy per wave)           */
+    int32_t hist_copies;        /* ignored (the library chooses)                       */
     int32_t cell_shapes;        /* > 0: size cells to hold this many shapes on average
                                    instead of the cost-model search                     */
     int32_t r_bins_per_pass;    /* > 0: r bins per pass of the pair kernel, clamped to

@@ -1879,35 +1879,35 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     const int Bp = nrp * n_2;     // bins of the largest pass
     A.nbins_out = B;
     A.bin_off = 0;
-    // one histogram copy per wave: the pending-slot registers already absorb
-    // most same-address collisions, and one copy leaves LDS for 8 waves per
-    // SIMD (2 copies measured 20 % slower); mia_tuning.hist_copies is ignored
     A.hist_stride = (int)hist_bytes(Bp, A.weighted, A.var);
     // A private histogram per wave (one copy: the pending-slot registers already
     // absorb most same-address collisions), or one per workgroup, shared by its
     // four waves, in as many copies (at most 4) as leave room for
     // kPairWavesPerSimd waves per SIMD.  Sharing keeps the SIMDs full where
-    // private histograms leave LDS for few waves (600 bins: 2 waves per SIMD
-    // private, 7 shared; 3,000,000 positions to 100 Mpc/h 317 against 201 ms),
-    // but a group of four waits for its slowest wave wherever the key or the
-    // chunk changes (200 bins, 28 private waves per CU, 1,000,000 positions: 8.5
-    // against 11.7 ms).  So it is taken
-    //   - below kSharedBelow private waves per CU;
-    //   - in launches too small for tail chunks, where the four waves even out
-    //     each other's items (60,000 shapes in 300,000 positions 1.82 against
-    //     1.55 ms, 75,025 in 317,811 weighted with variances 2.65 against 1.9,
-    //     10,000 in 50,000 0.43 against 0.39, 30,000 in 150,000 equal);
+    // private histograms leave LDS for few waves, and a key's histogram is flushed
+    // once for four waves; but a group of four waits for its slowest wave wherever
+    // the key or the chunk changes.  Shared / private, pair kernel in ms:
+    //   - below kSharedBelow private waves per CU shared: 600 bins, 3,000,000
+    //     positions to 100 Mpc/h 188 / 306 (8 waves); 1600 bins, 43,140 weightless
+    //     positions 1.3 / 2.3 (4 waves);
+    //   - the smallest launches shared, where the flushes weigh most: 2,000 galaxies
+    //     0.022 / 0.035, 20,000 with 27 regions 0.094 / 0.187, 20,000 in 100,000
+    //     0.22 / 0.26, 30,000 in 150,000 0.39 / 0.44; from 24,000 in 120,000 (0.28 /
+    //     0.26) on private: 40,000 in 200,000 0.61 / 0.57, 60,000 in 300,000 1.43 /
+    //     1.14, 200,000 in 1,000,000 10.4 / 7.6, a batch of eight uneven samples
+    //     3.7 / 2.7;
+    //   - with weights and variances, whose bins leave 16 private waves for 200 bins,
+    //     shared up to eight times as many: 40,000 in 200,000 0.71 / 0.87, 75,025 in
+    //     317,811 1.89 / 2.08, but 80,000 in 400,000 2.44 / 2.21;
     //   - where registers allow more waves than LDS and the launch is so large
-    //     that its chunks hold many items (2,000,000 positions, 300 bins: 205
-    //     against 200 ms; but twelve samples of 10,000 to 800,000, 24 private
-    //     waves: 21 against 31 ms).
-    // Never where the reduction is
-    // deterministic, since a shared histogram's sums depend on timing.
-    // mia_tuning.hist_copies is ignored.
+    //     that its chunks hold many items shared: 2,000,000 multipoles, 300 bins
+    //     195 / 202.
+    // Never where the reduction is deterministic, since a shared histogram's sums
+    // depend on timing.  mia_tuning.hist_copies is ignored.
     int wpb = kMaxWavesPerBlock;
     const size_t hs = A.hist_stride;
     const int pw = private_waves(thr_bytes, hs), most = std::min(4 * kPairWavesPerSimd, shared_waves(thr_bytes, hs));
-    const bool small = candidates < 0.8 * kTailMinCost * pw * cu_count;
+    const bool small = candidates < (any_w && any_var ? 0.65 : 0.08) * kTailMinCost * pw * cu_count;
     const bool large = candidates > 16 * kTailMinCost * pw * cu_count;
     A.shared = !det && most > 0 && (small || (pw < most && (pw < kSharedBelow || large)));
     if (A.shared) {
