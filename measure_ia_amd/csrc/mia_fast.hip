@@ -1,4 +1,4 @@
-// Fast pair counter: cell-pair work items, per-wavefront LDS histograms.
+// Fast pair counter: cell-pair work items, LDS histograms.
 //
 // Replaces the per-shape KDTree loop and np.add.at scatter of the reference
 // (src/measureia/measure_w_box_jk.py:386-461, measure_m_box_jk.py:403-487)
@@ -64,7 +64,6 @@ constexpr double kSinExact = 1e-5;  // FP64 arccos-domain check when |sin phi| <
 
 struct Block {
     int32_t s0, ns;
-    int32_t col, grp;   // column index, slab group (== ngroups: tail)
     int32_t sample, rs;
 };
 
@@ -85,7 +84,7 @@ struct Item {
     int32_t key;        // planner key over all samples
 };
 static_assert(sizeof(Item) == 32, "Item layout");
-static_assert(sizeof(Block) == 24, "Block layout");
+static_assert(sizeof(Block) == 16, "Block layout");
 
 struct SampleDev {
     // sorted sample
@@ -557,12 +556,12 @@ __global__ __launch_bounds__(kPlanThreads) void k_item_cost(const PlanSample *ps
         // (wave-uniform: read through the scalar cache)
         const MIA_CONST int32_t *ip = (const MIA_CONST int32_t *)items + 8 * i;
         const int blk = ip[0], w = ip[1], jj = ip[2], wn = ip[3], c0 = ip[4], kk = ip[5];
-        const MIA_CONST int32_t *bp = (const MIA_CONST int32_t *)blocks + 6 * (int64_t)blk;
+        const MIA_CONST int32_t *bp = (const MIA_CONST int32_t *)blocks + 4 * (int64_t)blk;
         const MIA_CONST double *bc = (const MIA_CONST double *)bbox + 6 * (int64_t)blk;
         const double bb[6] = {bc[0], bc[1], bc[2], bc[3], bc[4], bc[5]};
         const int ns = bp[1];
         int pb, np;
-        item_column(column_view((const MIA_CONST PlanSample *)ps + bp[4]), bb, jj & 0xffff, (jj >> 16) & 0xffff,
+        item_column(column_view((const MIA_CONST PlanSample *)ps + bp[2]), bb, jj & 0xffff, (jj >> 16) & 0xffff,
                     wn & 0xffff, (wn >> 16) & 0xffff, c0, kk & 0xffff, (kk >> 16) & 0xffff, w, lane, pb, np);
         for (int d = kWave / 2; d > 0; d >>= 1) np += __shfl_xor(np, d);
         if (lane == 0) {
@@ -610,8 +609,6 @@ __global__ void k_blocks(const PlanSample *ps, const int64_t *cell0, int S, int 
         Block B;
         B.s0 = s0 + b * bsz;
         B.ns = n - b * bsz < bsz ? n - b * bsz : bsz;
-        B.col = col;
-        B.grp = grp;
         B.sample = s;
         B.rs = rs;
         blocks[o + b] = B;
@@ -1630,8 +1627,8 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
                 if (bt0 >= bt1) continue;  // (no batch: no column of the item is in reach)
                 const int blk = ip[0], w = ip[1], jj = ip[2], wn = ip[3], c0 = ip[4], kk = ip[5];
                 const int shifts = (w >> 16) & 0xff;
-                const MIA_CONST int32_t *bp = (const MIA_CONST int32_t *)Q->blocks + 6 * (int64_t)blk;
-                const int s0 = bp[0], ns = bp[1], sample = bp[4];
+                const MIA_CONST int32_t *bp = (const MIA_CONST int32_t *)Q->blocks + 4 * (int64_t)blk;
+                const int s0 = bp[0], ns = bp[1], sample = bp[2];
                 const SampleView S = load_view(Q->samples + sample);
                 ShapePtr shp = (ShapePtr)(S.srec + 8 * (int64_t)s0);
                 int cpb, cn;
