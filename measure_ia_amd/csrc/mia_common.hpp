@@ -108,9 +108,12 @@ void schedule_bounds(const int64_t *cost_prefix, int64_t n, int waves, int64_t *
 // of kScheduleUnits, each worked on by waves_per_unit waves.  all_static: no tail
 // claims, so the batch -> wave map is fixed by the costs.
 // A unit costs at least kMinUnitCost, and the last groups of a tiny count take
-// nothing: every busy one adds its histogram to the same few hundred sums (2,000
-// galaxies, 160 bins: pair kernel 45 us without the bound, now 21).
-constexpr double kMinUnitCost = 160.0;
+// nothing: every busy one adds its histogram to the same few hundred sums.  Where
+// there are regions a group flushes once per key instead, one after the other, so
+// the bound is half of what is best without (pair kernel without the bound, at 80
+// and at 160: 2,000 galaxies, 160 bins 45, 29 and 22 us; 27 regions, 500 in 2,000
+// galaxies 24, 29 and 34, 213 in 4,011 with weights and variances 24, 34 and 48).
+constexpr double kMinUnitCost = 80.0;
 constexpr int kBatchBits = 26;           // batches of an item: below 2^31 / 64
 constexpr int64_t kItemOverhead = 1024;  // per-item cost, in pair evaluations (256: a batch of eight uneven samples
                                          // 4.8 ms of pair kernel, 512 4.1, 1024 3.6; 317,811 galaxies equal)
