@@ -1887,10 +1887,10 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     //   - below kSharedBelow private waves per CU shared: 600 bins, 3,000,000
     //     positions to 100 Mpc/h 188 / 306 (8 waves); 1600 bins, 43,140 weightless
     //     positions 1.3 / 2.3 (4 waves);
-    //   - the smallest launches shared, where the flushes weigh most: 2,000 galaxies
-    //     0.022 / 0.035, 20,000 with 27 regions 0.094 / 0.187, 20,000 in 100,000
-    //     0.22 / 0.26, 30,000 in 150,000 0.39 / 0.44; from 24,000 in 120,000 (0.28 /
-    //     0.26) on private: 40,000 in 200,000 0.61 / 0.57, 60,000 in 300,000 1.43 /
+    //   - the smallest launches shared, where the flushes weigh most: 20,000 with 27
+    //     regions 0.096 / 0.175, 20,000 in 100,000 0.21 / 0.26, 30,000 in 150,000 0.41
+    //     / 0.45 (2,000 galaxies equal); from 24,000 in 120,000 (0.285 / 0.26) on
+    //     private: 40,000 in 200,000 0.61 / 0.57, 60,000 in 300,000 1.43 /
     //     1.14, 200,000 in 1,000,000 10.4 / 7.6, a batch of eight uneven samples
     //     3.7 / 2.7;
     //   - with weights and variances, whose bins leave 16 private waves for 200 bins,
