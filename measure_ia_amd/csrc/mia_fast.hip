@@ -951,6 +951,7 @@ struct PairArgs {
     int scan;                    // 1: the exact path scans every threshold (guard band of a whole bin)
     const SampleDev *samples;
     int hist_stride;             // bytes of a histogram
+    int apart;                   // the counts lie in front of the sums
     int shared, copies;          // the waves of a workgroup share `copies` histograms (else one per wave)
     int bin_off, nbins_out;      // this pass's first output bin (r0 * n_2) and the output's B
     // kStatCopies copies of: pairs binned exactly, wave-iterations (a 64-lane
@@ -974,27 +975,28 @@ struct PairArgs {
 // apart, three sums with their count, only every fourth pair of banks starts a
 // bin: 300,001 weighted positions, 100,003 shapes, 200 bins 14.6 ms of pair kernel,
 // now 12.0).  Two or four sums are padded to three or five words by the count; of
-// three, the counts lie in front of the sums, bin b's b + 1 words before them,
-// which also leaves LDS for more waves (360 weighted bins: 16 per CU instead of 12,
-// 21.9 -> 17.0 ms in 300,001 positions).
-template <bool WEIGHTED, bool VAR>
+// three, the counts lie in front of the sums (APART), bin b's b + 1 words before
+// them, which also leaves LDS for more waves (360 weighted bins: 16 per CU instead
+// of 12, 21.9 -> 17.0 ms in 300,001 positions).  Two and four sums have the counts
+// apart in the deterministic mode's larger binnings (pair_config).
+template <bool WEIGHTED, bool VAR, bool APART>
 struct Slot {
     static constexpr int kSums = 2 + WEIGHTED + VAR;
-    static constexpr bool kApart = kSums == 3;
-    static constexpr uint32_t kBytes = kApart ? 24 : 8 * kSums + 8;
+    static constexpr bool kApart = APART;
+    static constexpr uint32_t kBytes = kApart ? 8 * kSums : 8 * kSums + 8;
+    static_assert(APART || kSums != 3, "three sums have their counts apart");
     uint32_t c;
     double v[kSums];  // S+D, SxD, [DD], [sum of e+^2]
 };
-static_assert(Slot<false, false>::kBytes == 24 && Slot<true, true>::kBytes == 40, "hist_bytes");
 // bytes of a histogram of nbins bins
-constexpr size_t hist_bytes(int nbins, bool weighted, bool var) {
-    const size_t n = (size_t)nbins;
-    return ((weighted == var ? (weighted ? 40 : 24) * n : 24 * n + ((4 * n + 7) & ~(size_t)7)) + 15) & ~(size_t)15;
+constexpr size_t hist_bytes(int nbins, bool weighted, bool var, bool apart) {
+    const size_t n = (size_t)nbins, sums = 8 * (2 + weighted + var) * n;
+    return (sums + (apart ? (4 * n + 7) & ~(size_t)7 : 8 * n) + 15) & ~(size_t)15;
 }
 // bytes of the counts in front of the sums
-template <bool WEIGHTED, bool VAR>
+template <bool WEIGHTED, bool VAR, bool APART>
 __device__ __forceinline__ int front_bytes(int nbins) {
-    return Slot<WEIGHTED, VAR>::kApart ? (4 * nbins + 7) & ~7 : 0;
+    return Slot<WEIGHTED, VAR, APART>::kApart ? (4 * nbins + 7) & ~7 : 0;
 }
 
 // Shape record {a, b, l, ax, ay, e*w, w, 2*e*w} read through the scalar cache:
@@ -1002,22 +1004,22 @@ __device__ __forceinline__ int front_bytes(int nbins) {
 typedef const __attribute__((address_space(4))) double *ShapePtr;
 
 // The place of bin b's count in a histogram.
-template <bool WEIGHTED, bool VAR>
+template <bool WEIGHTED, bool VAR, bool APART>
 __device__ __forceinline__ uint32_t *bin_count(char *sums, int b) {
-    typedef Slot<WEIGHTED, VAR> BinSlot;
+    typedef Slot<WEIGHTED, VAR, APART> BinSlot;
     return BinSlot::kApart ? (uint32_t *)sums - 1 - b
                            : (uint32_t *)(sums + (uint32_t)b * BinSlot::kBytes + 8 * BinSlot::kSums);
 }
 
 // One bin of a histogram, summed over its copies and cleared.
-template <bool WEIGHTED, bool VAR>
-__device__ __forceinline__ Slot<WEIGHTED, VAR> take_bin(const PairArgs &P, char *hist, int copies, int b) {
-    typedef Slot<WEIGHTED, VAR> BinSlot;
+template <bool WEIGHTED, bool VAR, bool APART>
+__device__ __forceinline__ Slot<WEIGHTED, VAR, APART> take_bin(const PairArgs &P, char *hist, int copies, int b) {
+    typedef Slot<WEIGHTED, VAR, APART> BinSlot;
     BinSlot t{};
-    hist += front_bytes<WEIGHTED, VAR>(P.nbins);
+    hist += front_bytes<WEIGHTED, VAR, APART>(P.nbins);
     for (int k = 0; k < copies; ++k, hist += P.hist_stride) {
         double *v = (double *)(hist + (uint32_t)b * BinSlot::kBytes);
-        uint32_t *c = bin_count<WEIGHTED, VAR>(hist, b);
+        uint32_t *c = bin_count<WEIGHTED, VAR, APART>(hist, b);
         if (*c == 0) continue;
         t.c += *c;
         *c = 0;
@@ -1044,13 +1046,13 @@ __device__ __forceinline__ void add_pairs(const PairArgs &P, const SampleDev &S,
 // A wave takes all but one pair of every count to the 64-bit sums, with adds of
 // other waves in flight: the histogram's 32-bit counts then stay below 2^32 whatever
 // its waves test before the next flush (a bin without a pair would not be flushed).
-template <bool WEIGHTED, bool VAR>
+template <bool WEIGHTED, bool VAR, bool APART>
 __device__ void spill_counts(const PairArgs &P, char *hist, int copies, const SampleDev &S, int rs, int rp, int lane) {
     for (int b = lane; b < P.nbins; b += kWave) {
-        char *sums = hist + front_bytes<WEIGHTED, VAR>(P.nbins);
+        char *sums = hist + front_bytes<WEIGHTED, VAR, APART>(P.nbins);
         unsigned long long c = 0;
         for (int k = 0; k < copies; ++k, sums += P.hist_stride) {
-            uint32_t *at = bin_count<WEIGHTED, VAR>(sums, b);
+            uint32_t *at = bin_count<WEIGHTED, VAR, APART>(sums, b);
             // (a count of one or more never falls below one before the flush)
             if (__hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > 1)
                 c += __hip_atomic_exchange(at, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) - 1;
@@ -1059,14 +1061,14 @@ __device__ void spill_counts(const PairArgs &P, char *hist, int copies, const Sa
     }
 }
 
-template <bool WEIGHTED, bool VAR>
+template <bool WEIGHTED, bool VAR, bool APART>
 __device__ void flush_hist(const PairArgs &P, char *hist, int copies, const SampleDev &S, int rs, int rp, int tid,
                            int nthr) {
     const bool dd = WEIGHTED, vr = VAR;
     const int B = P.nbins;
     const int BO = P.nbins_out;
     for (int b = tid; b < B; b += nthr) {
-        const Slot<WEIGHTED, VAR> t = take_bin<WEIGHTED, VAR>(P, hist, copies, b);
+        const Slot<WEIGHTED, VAR, APART> t = take_bin<WEIGHTED, VAR, APART>(P, hist, copies, b);
         const uint32_t c = t.c;
         const double vsp = t.v[0], vsx = t.v[1];
         double vdd = 0.0, vvr = 0.0;
@@ -1100,11 +1102,11 @@ __device__ __forceinline__ int64_t slot_key_of(int sample, int rs, int rp) {
 
 // The deterministic flush: the wave's histogram (every bin of the pass, the
 // empty ones too) is stored into its slot instead of added by atomics.
-template <bool WEIGHTED, bool VAR>
+template <bool WEIGHTED, bool VAR, bool APART>
 __device__ void flush_slot(const PairArgs &P, char *hist, int copies, int64_t slot, int64_t key, int tid, int nthr) {
     if (slot >= P.slot_cap) return;  // cannot happen: the slot plan counts every flush
     for (int b = tid; b < P.nbins; b += nthr) {
-        const Slot<WEIGHTED, VAR> t = take_bin<WEIGHTED, VAR>(P, hist, copies, b);
+        const Slot<WEIGHTED, VAR, APART> t = take_bin<WEIGHTED, VAR, APART>(P, hist, copies, b);
         const int64_t o = slot * P.nbins_out + P.bin_off + b;
         P.slot_np[o] = t.c;
         P.slot_sp[o] = t.v[0];
@@ -1193,15 +1195,15 @@ __device__ __forceinline__ void lds_add(uint32_t at, T v) {
 // hist: LDS address of the histogram's sums; with counts in front of them 4 bytes
 // less, so that no offset is negative.  The other kind of pending run holds its
 // bin's address, and a flush computes none.
-template <bool WEIGHTED, bool VAR>
+template <bool WEIGHTED, bool VAR, bool APART>
 __device__ __forceinline__ uint32_t pend_at(uint32_t hist, int b) {
-    typedef Slot<WEIGHTED, VAR> BinSlot;
+    typedef Slot<WEIGHTED, VAR, APART> BinSlot;
     return BinSlot::kApart ? (uint32_t)b : __umul24(b, BinSlot::kBytes) + hist;
 }
 
-template <bool WEIGHTED, bool VAR>
+template <bool WEIGHTED, bool VAR, bool APART>
 __device__ __forceinline__ void hist_add(uint32_t hist, const Pend &p) {
-    typedef Slot<WEIGHTED, VAR> BinSlot;
+    typedef Slot<WEIGHTED, VAR, APART> BinSlot;
     uint32_t at = p.at;
     if constexpr (BinSlot::kApart) {
         lds_add<uint32_t>((uint32_t)(__mul24((int)p.at, -4) + (int)hist), p.c);
@@ -1215,7 +1217,7 @@ __device__ __forceinline__ void hist_add(uint32_t hist, const Pend &p) {
     if constexpr (VAR) lds_add<double>(at + (WEIGHTED ? 24 : 16), p.vr);
 }
 
-template <int MODE, int SH, bool WEIGHTED, bool VAR, bool LZ>
+template <int MODE, int SH, bool WEIGHTED, bool VAR, bool APART, bool LZ>
 __device__ __forceinline__ void one_pair(const PairArgs &P, const SampleView &S, bool valid,
                                          double pa, double pb, double pl, double pw, double qa,
                                          double qb, double ql, double qax, double qay, double qew,
@@ -1320,16 +1322,16 @@ __device__ __forceinline__ void one_pair(const PairArgs &P, const SampleView &S,
             ep = pw * ep;
             ex = pw * ex;
         }
-        const uint32_t at = Slot<WEIGHTED, VAR>::kApart
+        const uint32_t at = Slot<WEIGHTED, VAR, APART>::kApart
                                 ? (uint32_t)(__mul24(ir, n_2) + i2)
-                                : __umul24(ir, row) + (__umul24(i2, Slot<WEIGHTED, VAR>::kBytes) + hist);
+                                : __umul24(ir, row) + (__umul24(i2, Slot<WEIGHTED, VAR, APART>::kBytes) + hist);
         double dd = WEIGHTED ? pw * qw : 0.0;
         double vr = VAR ? ep * ep : 0.0;
         // a new slot flushes the pending run; the run then restarts from this
         // pair: keep = 0 drops the old sums (fma(0, sum, x) = x, fma(1, sum, x)
         // = sum + x, both exactly as the plain assignment and addition)
         const bool nw = at != pd.at;
-        if (nw) hist_add<WEIGHTED, VAR>(hist, pd);
+        if (nw) hist_add<WEIGHTED, VAR, APART>(hist, pd);
         const double keep = nw ? 0.0 : 1.0;
         pd.at = at;
         pd.c = (nw ? 0u : pd.c) + 1u;
@@ -1385,7 +1387,7 @@ struct ColumnWalk {
     }
 };
 
-template <int MODE, int SH, bool WEIGHTED, bool VAR, bool LZ>
+template <int MODE, int SH, bool WEIGHTED, bool VAR, bool APART, bool LZ>
 __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S, int cpb, int cn, int bt0, int bt1,
                                          int shifts, ShapePtr shp, int ns, uint32_t hist,
                                          const double *T, const double *X, int lane,
@@ -1410,8 +1412,8 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
     walk.begin(lane, cpb, cn, bt0);
     iterations += (uint64_t)(bt1 - bt0) * ns;
     // an empty run adds its zeros to some bin, another one for every lane
-    const uint32_t row = (uint32_t)P.n_2 * Slot<WEIGHTED, VAR>::kBytes;
-    Pend pd{pend_at<WEIGHTED, VAR>(hist, lane < P.nbins ? lane : 0), 0, 0, 0, 0, 0};
+    const uint32_t row = (uint32_t)P.n_2 * Slot<WEIGHTED, VAR, APART>::kBytes;
+    Pend pd{pend_at<WEIGHTED, VAR, APART>(hist, lane < P.nbins ? lane : 0), 0, 0, 0, 0, 0};
     // positions are loaded one batch ahead
     bool vn;
     const double2 *prn = (const double2 *)(S.prec + 4 * (int64_t)walk.position(bt0, lane, vn));
@@ -1439,12 +1441,12 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
             ShapePtr r1 = (ShapePtr)((const MIA_CONST char *)shp + (o + 64u));
             const double b0 = r1[0], b1 = r1[1], b2 = r1[2], b3 = r1[3], b4 = r1[4], b5 = r1[5],
                          b6 = r1[6], b7 = r1[7];
-            one_pair<MODE, SH, WEIGHTED, VAR, LZ>(P, S, v0, pa0, pb0, pl0, pw0, qa, qb, ql, qax, qay, qew, qw,
+            one_pair<MODE, SH, WEIGHTED, VAR, APART, LZ>(P, S, v0, pa0, pb0, pl0, pw0, qa, qb, ql, qax, qay, qew, qw,
                                          q2ew, sha, shb, shl, hist, row, T, X, nre, pd, vlgc, vlg2, vxs, vxc);
             ShapePtr r2 = (ShapePtr)((const MIA_CONST char *)shp + (o + 128u < olast ? o + 128u : olast));
             const double c0 = r2[0], c1 = r2[1], c2 = r2[2], c3 = r2[3], c4 = r2[4], c5 = r2[5],
                          c6 = r2[6], c7 = r2[7];
-            one_pair<MODE, SH, WEIGHTED, VAR, LZ>(P, S, v0, pa0, pb0, pl0, pw0, b0, b1, b2, b3, b4, b5, b6,
+            one_pair<MODE, SH, WEIGHTED, VAR, APART, LZ>(P, S, v0, pa0, pb0, pl0, pw0, b0, b1, b2, b3, b4, b5, b6,
                                          b7, sha, shb, shl, hist, row, T, X, nre, pd, vlgc, vlg2, vxs, vxc);
             qa = c0;
             qb = c1;
@@ -1456,25 +1458,25 @@ __device__ __forceinline__ void run_item(const PairArgs &P, const SampleView &S,
             q2ew = c7;
         }
         if (j < ns)
-            one_pair<MODE, SH, WEIGHTED, VAR, LZ>(P, S, v0, pa0, pb0, pl0, pw0, qa, qb, ql, qax, qay, qew, qw,
+            one_pair<MODE, SH, WEIGHTED, VAR, APART, LZ>(P, S, v0, pa0, pb0, pl0, pw0, qa, qb, ql, qax, qay, qew, qw,
                                          q2ew, sha, shb, shl, hist, row, T, X, nre, pd, vlgc, vlg2, vxs, vxc);
     }
-    hist_add<WEIGHTED, VAR>(hist, pd);
+    hist_add<WEIGHTED, VAR, APART>(hist, pd);
 }
 
 // The batches [bt0, bt1) of an item, in the pair loop for its periodic-shift variant.
-template <int MODE, bool WEIGHTED, bool VAR, bool LZ>
+template <int MODE, bool WEIGHTED, bool VAR, bool APART, bool LZ>
 __device__ __forceinline__ void run_shifted(const PairArgs &P, const SampleView &S, int cpb, int cn, int bt0, int bt1,
                                             int shifts, ShapePtr shp, int ns, uint32_t hist, const double *T,
                                             const double *X, int lane, uint32_t &nre, uint64_t &iterations) {
     if (shifts & 64)
-        run_item<MODE, SH_WRAP, WEIGHTED, VAR, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_WRAP, WEIGHTED, VAR, APART, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
                                                    iterations);
     else if (shifts & 63)
-        run_item<MODE, SH_CONST, WEIGHTED, VAR, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_CONST, WEIGHTED, VAR, APART, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
                                                     iterations);
     else
-        run_item<MODE, SH_NONE, WEIGHTED, VAR, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
+        run_item<MODE, SH_NONE, WEIGHTED, VAR, APART, LZ>(P, S, cpb, cn, bt0, bt1, shifts, shp, ns, hist, T, X, lane, nre,
                                                    iterations);
 }
 
@@ -1492,7 +1494,7 @@ __device__ __forceinline__ void run_shifted(const PairArgs &P, const SampleView 
 // with many whole items even the waves out, and the empty claims of small items
 // cost more (a batch of samples with 91 items per group, 1.5 against 2.1 ms;
 // 2,000,000 multipoles 196 against 204).
-template <int MODE, bool WEIGHTED, bool VAR>
+template <int MODE, bool WEIGHTED, bool VAR, bool APART>
 __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs P) {
     extern __shared__ __align__(16) char lds[];
     __shared__ unsigned s_next[2];
@@ -1532,7 +1534,7 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     char *hist = hist0 + (shared ? 0 : wv * P.hist_stride);
     const int place = ((lane & 7) << 3) | (lane >> 3);
     const uint32_t hist_at = (uint32_t)(uintptr_t)(MIA_LDS char *)(hist + (shared ? place % P.copies : 0) * P.hist_stride) +
-                             front_bytes<WEIGHTED, VAR>(P.nbins) - (Slot<WEIGHTED, VAR>::kApart ? 4 : 0);
+                             front_bytes<WEIGHTED, VAR, APART>(P.nbins) - (Slot<WEIGHTED, VAR, APART>::kApart ? 4 : 0);
     // a contiguous share of the cost, then tail chunks from the counter
     const WaveSchedule sch = make_schedule(P.bounds, shared ? (int)gridDim.x : P.n_waves);
     int64_t it0, it1;  // item << kBatchBits | batch
@@ -1572,9 +1574,9 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
             const int rs = in / P.K1, rp = in - rs * P.K1;
             const int n = shared ? P.copies : 1;
             if (P.det)
-                flush_slot<WEIGHTED, VAR>(P, hist, n, P.slot0[wave] + flushes++, slot_key_of(sample, rs, rp), tid, nthr);
+                flush_slot<WEIGHTED, VAR, APART>(P, hist, n, P.slot0[wave] + flushes++, slot_key_of(sample, rs, rp), tid, nthr);
             else
-                flush_hist<WEIGHTED, VAR>(P, hist, n, P.samples[sample], rs, rp, tid, nthr);
+                flush_hist<WEIGHTED, VAR, APART>(P, hist, n, P.samples[sample], rs, rp, tid, nthr);
             sync();
         }
         cur_key = key;
@@ -1644,16 +1646,16 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
                     // (r, mu) sums r^2 in an order fixed by the line of sight: one
                     // loop per order, so the pair loop holds no branch on it
                     if (MODE == MIA_RMU && S.los != 2)
-                        run_shifted<MODE, WEIGHTED, VAR, false>(P, S, cpb, cn, b, e, shifts, shp, ns, hist_at, T, X,
+                        run_shifted<MODE, WEIGHTED, VAR, APART, false>(P, S, cpb, cn, b, e, shifts, shp, ns, hist_at, T, X,
                                                                 lane, nre, iterations);
                     else
-                        run_shifted<MODE, WEIGHTED, VAR, true>(P, S, cpb, cn, b, e, shifts, shp, ns, hist_at, T, X,
+                        run_shifted<MODE, WEIGHTED, VAR, APART, true>(P, S, cpb, cn, b, e, shifts, shp, ns, hist_at, T, X,
                                                                lane, nre, iterations);
                     if ((uint32_t)(iterations >> kSpillBits) == spills) continue;
                     spills = (uint32_t)(iterations >> kSpillBits);
                     const PairArgs &A = *(const PairArgs *)args();
                     const int kk = A.K1 * A.K1, in = cur_key % kk;
-                    spill_counts<WEIGHTED, VAR>(A, hist, shared ? A.copies : 1, A.samples[cur_key / kk], in / A.K1,
+                    spill_counts<WEIGHTED, VAR, APART>(A, hist, shared ? A.copies : 1, A.samples[cur_key / kk], in / A.K1,
                                                 in % A.K1, lane);
                 }
             }
@@ -1694,32 +1696,27 @@ __global__ __launch_bounds__(kThreads, kPairWavesPerSimd) void k_pairs(PairArgs 
     }
 }
 
-template <int MODE, bool WEIGHTED, bool VAR>
+template <int MODE, bool WEIGHTED, bool VAR, bool APART>
 void launch_pairs(const PairArgs &A, unsigned grid, int wpb, size_t lds, hipStream_t st) {
-    hipLaunchKernelGGL((k_pairs<MODE, WEIGHTED, VAR>), dim3(grid), dim3(kWave * wpb), lds, st, A);
+    hipLaunchKernelGGL((k_pairs<MODE, WEIGHTED, VAR, APART>), dim3(grid), dim3(kWave * wpb), lds, st, A);
     MIA_HIP(hipGetLastError());
 }
 
 template <int MODE>
 void launch_pairs_mode(const PairArgs &A, unsigned grid, int wpb, size_t lds, hipStream_t st) {
-    if (A.weighted) {
-        if (A.var)
-            launch_pairs<MODE, true, true>(A, grid, wpb, lds, st);
-        else
-            launch_pairs<MODE, true, false>(A, grid, wpb, lds, st);
-    } else {
-        if (A.var)
-            launch_pairs<MODE, false, true>(A, grid, wpb, lds, st);
-        else
-            launch_pairs<MODE, false, false>(A, grid, wpb, lds, st);
-    }
+    if (A.weighted && A.var)
+        A.apart ? launch_pairs<MODE, true, true, true>(A, grid, wpb, lds, st)
+                : launch_pairs<MODE, true, true, false>(A, grid, wpb, lds, st);
+    else if (A.weighted)
+        launch_pairs<MODE, true, false, true>(A, grid, wpb, lds, st);
+    else if (A.var)
+        launch_pairs<MODE, false, true, true>(A, grid, wpb, lds, st);
+    else
+        A.apart ? launch_pairs<MODE, false, false, true>(A, grid, wpb, lds, st)
+                : launch_pairs<MODE, false, false, false>(A, grid, wpb, lds, st);
 }
 
-// LDS bytes of one wave's histogram (one copy) and of the block's thresholds.
-size_t wave_hist_bytes(const mia_bins &bins, bool weighted) {
-    return hist_bytes(bins.n_r * bins.n_2, weighted, bins.accumulate_variance);
-}
-
+// LDS bytes of the thresholds of a workgroup.
 size_t threshold_bytes(const mia_bins &bins) {
     return ((size_t)(bins.n_r + 1 + bins.n_2 + 1) * 8 + 15) & ~(size_t)15;
 }
@@ -1737,18 +1734,23 @@ struct PairConfig {
 };
 
 // The pair kernel of a count.
-const void *pair_kernel(int mode, bool weighted, bool var) {
-#define MIA_PICK(M) \
-    (weighted ? (var ? (const void *)k_pairs<M, true, true> : (const void *)k_pairs<M, true, false>) \
-              : (var ? (const void *)k_pairs<M, false, true> : (const void *)k_pairs<M, false, false>))
-    return mode == MIA_RPPI ? MIA_PICK(MIA_RPPI) : MIA_PICK(MIA_RMU);
-#undef MIA_PICK
+template <int M>
+const void *pair_kernel(bool weighted, bool var, bool apart) {
+    if (weighted != var)
+        return weighted ? (const void *)k_pairs<M, true, false, true> : (const void *)k_pairs<M, false, true, true>;
+    if (apart)
+        return weighted ? (const void *)k_pairs<M, true, true, true> : (const void *)k_pairs<M, false, false, true>;
+    return weighted ? (const void *)k_pairs<M, true, true, false> : (const void *)k_pairs<M, false, false, false>;
+}
+const void *pair_kernel(int mode, bool weighted, bool var, bool apart) {
+    return mode == MIA_RPPI ? pair_kernel<MIA_RPPI>(weighted, var, apart) : pair_kernel<MIA_RMU>(weighted, var, apart);
 }
 
 // Workgroups of that kernel a CU holds at once (registers and LDS).
-int resident_workgroups(int mode, bool weighted, bool var, int wpb, size_t lds) {
+int resident_workgroups(const PairArgs &A, int wpb, size_t lds) {
     int n = 0;
-    MIA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pair_kernel(mode, weighted, var), kWave * wpb, lds));
+    MIA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pair_kernel(A.mode, A.weighted, A.var, A.apart),
+                                                         kWave * wpb, lds));
     return std::max(1, std::min(n, workgroups_by_lds(lds + kPairStaticLds)));
 }
 
@@ -1835,40 +1837,53 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     // histograms per workgroup, whose waves wait for each other.  Pair kernels
     // with W = 16 and now, 1,000,000 positions and 200,000 shapes: deterministic
     // 100 x 100 bins 25 passes of 16 waves 181 ms, 7 of 4 121; 60 x 60 8 of 12 70 ms,
-    // 5 of 8 54; shared, 200,000 and 50,000: 100 x 100 5 of 12 6.1 ms, 2 of 4
+    // 5 of 8 54 (counts inside the bins); shared, 200,000 and 50,000: 100 x 100 5 of 12 6.1 ms, 2 of 4
     // 4.1.  Ordinary binnings run in one pass.
     const size_t thr_bytes = threshold_bytes(bins);
     int nrp = n_r;
     {
-        mia_bins part = bins;
-        part.accumulate_variance = any_var ? 1 : 0;
-        auto waves_per_cu = [&](int nr_) {
-            part.n_r = nr_;
-            const size_t hs = wave_hist_bytes(part, any_w);
+        auto waves_per_cu = [&](int c, bool apart) {
+            const size_t hs = hist_bytes(c * n_2, any_w, any_var, apart);
             const int w = private_waves(thr_bytes, hs);
             return det ? w : std::max(w, shared_waves(thr_bytes, hs));
         };
-        if (tuning && tuning->r_bins_per_pass > 0) {
-            // as asked, but no more than one wave's histogram can hold
-            nrp = std::min(n_r, tuning->r_bins_per_pass);
-            while (nrp > 1 && waves_per_cu(nrp) == 0) --nrp;
-        } else {
-            double best = 1e300;
-            int best_p = 0;
+        // rows of the cheapest pass and its price
+        auto best_pass = [&](bool apart, double &best) {
+            int best_c = 1, best_p = 0;
+            best = 1e300;
             for (int pass_min_waves : {4, 1}) {
                 for (int c = n_r; c >= 1; --c) {
-                    const int w = waves_per_cu(c);
+                    const int w = waves_per_cu(c, apart);
                     if (w < pass_min_waves) continue;
                     const int passes = (n_r + c - 1) / c;
                     const double cost = (double)passes / std::min(1.0, w / (det ? 7.0 : 10.0));
                     if (cost < best * (1 - 1e-9) || (cost <= best * (1 + 1e-9) && passes < best_p)) {
                         best = cost;
                         best_p = passes;
-                        nrp = c;
+                        best_c = c;
                     }
                 }
                 if (best_p) break;
             }
+            return best_c;
+        };
+        // Two or four sums have their counts apart only in the deterministic mode,
+        // where narrower bins save passes or leave more private waves; elsewhere
+        // the lanes' bins collide more on the banks (200 bins, 1,000,000 positions
+        // 7.7 -> 8.3 ms of pair kernel).  Deterministic, 1,000,000 positions and
+        // 200,000 shapes, inside / apart: 60 x 60 bins 56.5 / 44.0 ms, 100 x 100
+        // 127 / 92; 300,000 and 60,000: 100 x 20 4.4 / 3.2, with weights and variances
+        // 33 x 101 10.0 / 8.0, 80 x 80 16.3 / 15.2, but 120 x 120, 0.93 of the price,
+        // 32.0 / 32.4.
+        double cost = 1e300, cost_apart;
+        const int c_apart = best_pass(true, cost_apart);
+        if (any_w == any_var) nrp = best_pass(false, cost);
+        A.apart = any_w != any_var || (det && cost_apart < 0.92 * cost);
+        if (A.apart) nrp = c_apart;
+        if (tuning && tuning->r_bins_per_pass > 0) {
+            // as asked, but no more than one wave's histogram can hold
+            nrp = std::min(n_r, tuning->r_bins_per_pass);
+            while (nrp > 1 && waves_per_cu(nrp, A.apart) == 0) --nrp;
         }
     }
     C.nrp = nrp;
@@ -1876,7 +1891,7 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
     const int Bp = nrp * n_2;     // bins of the largest pass
     A.nbins_out = B;
     A.bin_off = 0;
-    A.hist_stride = (int)hist_bytes(Bp, A.weighted, A.var);
+    A.hist_stride = (int)hist_bytes(Bp, any_w, any_var, A.apart);
     // A private histogram per wave (one copy: the pending-slot registers already
     // absorb most same-address collisions), or one per workgroup, shared by its
     // four waves, in as many copies (at most 4) as leave room for
@@ -1920,7 +1935,7 @@ PairConfig pair_config(const mia_bins &bins, bool any_w, bool any_var, const mia
         throw Error{MIA_E_UNSUPPORTED, "histogram too large for LDS (n_r*n_2 too big for MIA_FAST)"};
     C.wpb = wpb;
     // as many workgroups as are resident at once
-    const int blocks_per_cu = resident_workgroups(bins.mode, any_w, any_var, wpb, C.lds);
+    const int blocks_per_cu = resident_workgroups(A, wpb, C.lds);
     int waves = tuning && tuning->waves > 0 ? std::min(tuning->waves, kMaxWaves) : cu_count * blocks_per_cu * wpb;
     C.waves = std::max(1, waves);
     A.n_waves = C.waves;
@@ -1935,9 +1950,8 @@ bool fast_path_fits(const mia_bins &bins, bool weighted, int jk) {
     const int64_t K1 = jk > 0 ? (int64_t)jk * jk * jk : 1;
     if (K1 * K1 > kMaxKeysPerSample) return false;
     // larger binnings run in passes over r-bin ranges: one r row must fit
-    mia_bins row = bins;
-    row.n_r = 1;
-    return threshold_bytes(bins) + wave_hist_bytes(row, weighted) + kPairStaticLds <= kLdsBytes;
+    return threshold_bytes(bins) + hist_bytes(bins.n_2, weighted, bins.accumulate_variance, true) + kPairStaticLds <=
+           kLdsBytes;
 }
 
 // Sets the dynamic-LDS limit of every pair-kernel variant (once per process).
@@ -1948,8 +1962,8 @@ void pair_kernels_init() {
     MIA_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(mu);
     if (dev < 64 && (done >> dev & 1)) return;
-    for (int i = 0; i < 8; ++i)
-        MIA_HIP(hipFuncSetAttribute(pair_kernel(i & 4 ? MIA_RMU : MIA_RPPI, i & 2, i & 1),
+    for (int i = 0; i < 16; ++i)
+        MIA_HIP(hipFuncSetAttribute(pair_kernel(i & 4 ? MIA_RMU : MIA_RPPI, i & 2, i & 1, i & 8),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kLdsBytes - kPairStaticLds)));
     if (dev < 64) done |= 1ull << dev;
 }
